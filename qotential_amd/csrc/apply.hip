@@ -1,8 +1,7 @@
-// Near-correction apply, deterministic scatter, far field and COO triplets.
+// Near-correction apply, deterministic scatter and COO triplets.
 //
 // Reference: naive block + apply   stellarator_grf_core_mod.f90:847-870
 //            fixed-order scatter   stellarator_grf_core_mod.f90:895-899
-//            far field (direct)    stellarator_grf_core_mod.f90:560-611
 //            COO triplets          lap3d_close_mod.f90:935-956
 #include "qol_kernels.h"
 
@@ -184,46 +183,6 @@ __global__ void target_sum_kernel(int nt, const int* __restrict__ toffs, int* __
   double acc = u[t];
   for (int i = a; i < b; ++i) acc = acc + val[tpairs[i]];
   u[t] = acc;
-}
-
-// far field by direct summation (zero at coincident points), sources staged in LDS
-constexpr int kFT = 256, kFS = 256;
-__global__ void __launch_bounds__(256) far_direct_kernel(int nt, const double* __restrict__ tx, int ns,
-                                                         const double* __restrict__ sx, const double* __restrict__ snx,
-                                                         const double* __restrict__ sw, const double* __restrict__ ub,
-                                                         const double* __restrict__ ubn, double* __restrict__ u) {
-  __shared__ double s[8][kFS];
-  const double pi4inv = 1.0 / (16.0 * atan(1.0));
-  const int t = blockIdx.x * kFT + threadIdx.x;
-  double x0 = 0, x1 = 0, x2 = 0;
-  if (t < nt) { x0 = tx[3 * (size_t)t]; x1 = tx[3 * (size_t)t + 1]; x2 = tx[3 * (size_t)t + 2]; }
-  double acc = 0.0;
-  for (int j0 = 0; j0 < ns; j0 += kFS) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < kFS; i += blockDim.x) {
-      const int j = j0 + i;
-      if (j < ns) {
-        s[0][i] = sx[3 * (size_t)j]; s[1][i] = sx[3 * (size_t)j + 1]; s[2][i] = sx[3 * (size_t)j + 2];
-        s[3][i] = snx[3 * (size_t)j]; s[4][i] = snx[3 * (size_t)j + 1]; s[5][i] = snx[3 * (size_t)j + 2];
-        s[6][i] = pi4inv * sw[j] * ubn[j];
-        s[7][i] = pi4inv * sw[j] * ub[j];
-      } else {
-        for (int c = 0; c < 8; ++c) s[c][i] = 0.0;
-        s[0][i] = 1e300;
-      }
-    }
-    __syncthreads();
-    const int jn = min(kFS, ns - j0);
-    for (int i = 0; i < jn; ++i) {
-      const double dx = x0 - s[0][i], dy = x1 - s[1][i], dz = x2 - s[2][i];
-      const double rr = dx * dx + dy * dy + dz * dz;
-      if (rr > 1.0e-28) {
-        const double ri = 1.0 / sqrt(rr);
-        acc += s[6][i] * ri - s[7][i] * (dx * s[3][i] + dy * s[4][i] + dz * s[5][i]) * ri * ri * ri;
-      }
-    }
-  }
-  if (t < nt) u[t] = acc;
 }
 
 // ---------------------------------------------------------------------------

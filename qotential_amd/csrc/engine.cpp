@@ -887,10 +887,14 @@ void Engine::far(const double* ub, const double* ubn, double* u) {
   HIPCHK(hipMemcpyAsync(d_ubn.ptr, ubn, sizeof(double) * nsrc, hipMemcpyHostToDevice, stream));
   density_set = true;
   val_current = false;
-  if (nt > 0)
-    hipLaunchKernelGGL(far_direct_kernel, dim3(blocks(nt, 256)), dim3(256), 0, stream, nt, (const double*)d_tx.ptr,
-                       (int)nsrc, (const double*)d_sx.ptr, (const double*)d_snx.ptr, (const double*)d_sw.ptr,
-                       (const double*)d_ub.ptr, (const double*)d_ubn.ptr, (double*)d_u.ptr);
+  if (nt > 0) {
+    const FarPlan F = far_plan(nt, (int)nsrc);
+    d_fsrc.alloc(sizeof(double) * 8 * nsrc);
+    d_fpart.alloc(sizeof(double) * (size_t)F.nchunk * nt);
+    launch_far(F, nt, (const double*)d_tx.ptr, (int)nsrc, (const double*)d_sx.ptr, (const double*)d_snx.ptr,
+               (const double*)d_sw.ptr, (const double*)d_ub.ptr, (const double*)d_ubn.ptr, (double*)d_fsrc.ptr,
+               (double*)d_fpart.ptr, (double*)d_u.ptr, stream);
+  }
   HIPCHK(hipGetLastError());
   if (nt > 0) HIPCHK(hipMemcpyAsync(u, d_u.ptr, sizeof(double) * nt, hipMemcpyDeviceToHost, stream));
   HIPCHK(hipStreamSynchronize(stream));

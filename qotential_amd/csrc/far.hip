@@ -1,0 +1,141 @@
+// Far field by direct summation over every surface node (zero at coincident
+// points): u(t) = sum_j w_j (ubn_j / r - ub_j (x - y_j).n_j / r^3) / (4 pi).
+//
+// Reference: stellarator_grf_core_mod.f90:560-611
+//
+// Bound by the FP64 vector rate: 17 FP64 operations, one v_rsq_f64 and a select
+// per (target, node), about 96 issue cycles per wave of 64 pairs; measured 102
+// (200,000 targets x 513,000 nodes: 68 ms; one thread a target with the sources
+// in LDS and IEEE divide and square root took 246 ms, and 102 ms at 50,000
+// targets, now 17, because 196 workgroups left the chip idle).  Sources are packed once per call into one 64-byte record
+// each (position, and the strengths with the quadrature weight, 1/(4 pi) and the
+// normal multiplied in), which every wave reads with uniform addresses, so they
+// come through the scalar cache and feed the arithmetic from scalar registers:
+// no LDS traffic, and kFT targets per thread share each record.  The sources are
+// split into chunks so that few targets still fill the chip; each chunk's sums
+// go to part(chunk, target) and are added in chunk order, so the result does not
+// depend on timing.
+#include <algorithm>
+
+#include "qol_kernels.h"
+
+namespace qol {
+
+namespace {
+
+// coordinates beyond this square past the FP64 range: such sources and targets
+// are taken out of the sum below and get what the plain formula gives
+constexpr double kFarHuge = 1e150;
+
+}  // namespace
+
+// A source whose position is NaN contributes nothing (its r^2 fails the test
+// against the coincidence threshold), nor does one so far that r^2 overflows.
+__global__ void __launch_bounds__(256) far_pack_kernel(int ns, const double* __restrict__ sx,
+                                                       const double* __restrict__ snx, const double* __restrict__ sw,
+                                                       const double* __restrict__ ub, const double* __restrict__ ubn,
+                                                       double2* __restrict__ src) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= ns) return;
+  const double pi4inv = 1.0 / (16.0 * atan(1.0));
+  double x = sx[3 * (size_t)j], y = sx[3 * (size_t)j + 1], z = sx[3 * (size_t)j + 2];
+  const double w = pi4inv * sw[j], d = w * ub[j];
+  double s = w * ubn[j], a = d * snx[3 * (size_t)j], b = d * snx[3 * (size_t)j + 1], c = d * snx[3 * (size_t)j + 2];
+  const double big = fmax(fmax(fabs(x), fabs(y)), fabs(z));
+  if (x != x || y != y || z != z || (big >= kFarHuge && !isinf(big))) {
+    x = y = z = 0.0;
+    s = a = b = c = 0.0;
+  }
+  double2* o = src + 4 * (size_t)j;
+  o[0] = double2{x, y};
+  o[1] = double2{z, s};
+  o[2] = double2{a, b};
+  o[3] = double2{c, 0.0};
+}
+
+// one wave per tile of 64 kFT targets and chunk of sources
+template <int kFT>
+__global__ void __launch_bounds__(64) far_direct_kernel(int nt, const double* __restrict__ tx, int ns, int len,
+                                                        const double* __restrict__ src, double* __restrict__ part) {
+  const int t0 = blockIdx.x * 64 * kFT + threadIdx.x;
+  double x[kFT][3], acc[kFT];
+#pragma unroll
+  for (int i = 0; i < kFT; ++i) {
+    const size_t t = min(t0 + 64 * i, nt - 1);
+    x[i][0] = tx[3 * t];
+    x[i][1] = tx[3 * t + 1];
+    x[i][2] = tx[3 * t + 2];
+    acc[i] = 0.0;
+  }
+  const int j0 = blockIdx.y * len, j1 = min(ns, j0 + len);
+#pragma unroll 2
+  for (int j = j0; j < j1; ++j) {
+    const double* s = src + 8 * (size_t)j;
+    const double s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3], s4 = s[4], s5 = s[5], s6 = s[6];
+#pragma unroll
+    for (int i = 0; i < kFT; ++i) {
+      const double dx = x[i][0] - s0, dy = x[i][1] - s1, dz = x[i][2] - s2;
+      const double rr = fma(dz, dz, fma(dy, dy, dx * dx));
+      const double ri = rr > 1.0e-28 ? rsqrt_h3(rr) : 0.0;
+      const double dn = fma(dz, s6, fma(dy, s5, dx * s4));
+      acc[i] = fma(ri, fma(-dn, ri * ri, s3), acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kFT; ++i)
+    if (t0 + 64 * i < nt) part[(size_t)blockIdx.y * nt + t0 + 64 * i] = acc[i];
+}
+
+// u(t) = sum of part(c, t): 64 targets per workgroup, each of the 4 waves adds
+// every fourth chunk in order, then the four sums are added in order
+__global__ void __launch_bounds__(256) far_sum_kernel(int nt, int nchunk, const double* __restrict__ tx,
+                                                      const double* __restrict__ part, double* __restrict__ u) {
+  __shared__ double s[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int t = blockIdx.x * 64 + lane;
+  double acc = 0.0;
+  if (t < nt)
+#pragma unroll 8
+    for (int c = wv; c < nchunk; c += 4) acc += part[(size_t)c * nt + t];
+  s[wv][lane] = acc;
+  __syncthreads();
+  if (wv != 0 || t >= nt) return;
+  double v = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+  const double x = tx[3 * (size_t)t], y = tx[3 * (size_t)t + 1], z = tx[3 * (size_t)t + 2];
+  const double big = fmax(fmax(fabs(x), fabs(y)), fabs(z));
+  if (x != x || y != y || z != z) v = 0.0;                // every r^2 is NaN: no source contributes
+  else if (big >= kFarHuge) v = isinf(big) ? big - big : 0.0;  // 0 * inf, or every 1/r underflows to 0
+  u[t] = v;
+}
+
+// Measured (targets x sources, billions of pairs a second): four targets a thread
+// and 32,768 waves run 200,000 x 513,000 at 1,510 and 20,011 x 79,464 at 1,520;
+// one target a thread at 1,420 and 1,380 (each record feeds a quarter of the
+// arithmetic), 4,096 waves at 1,280 on the second (a few long waves end last).
+// Below four tiles' worth of targets the shorter waves of one or two targets a
+// thread win: 100 x 15,800 takes 8.7, 9.5 and 13.1 us at one, two and four.
+FarPlan far_plan(int nt, int ns) {
+  FarPlan P;
+  P.per = nt > 256 ? 4 : (nt > 64 ? 2 : 1);
+  const int tiles = (nt + 64 * P.per - 1) / (64 * P.per);
+  // no chunk below 32 sources, and at most 512 sums a target to add up
+  const int n = std::min({(32768 + tiles - 1) / tiles, (ns + 31) / 32, 512});
+  P.len = (ns + n - 1) / n;
+  P.nchunk = (ns + P.len - 1) / P.len;
+  return P;
+}
+
+void launch_far(const FarPlan& P, int nt, const double* tx, int ns, const double* sx, const double* snx,
+                const double* sw, const double* ub, const double* ubn, double* src, double* part, double* u,
+                hipStream_t s) {
+  hipLaunchKernelGGL(far_pack_kernel, dim3((ns + 255) / 256), dim3(256), 0, s, ns, sx, snx, sw, ub, ubn, (double2*)src);
+  const dim3 grid((nt + 64 * P.per - 1) / (64 * P.per), P.nchunk);
+  switch (P.per) {
+    case 1: hipLaunchKernelGGL(far_direct_kernel<1>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
+    case 2: hipLaunchKernelGGL(far_direct_kernel<2>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
+    default: hipLaunchKernelGGL(far_direct_kernel<4>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
+  }
+  hipLaunchKernelGGL(far_sum_kernel, dim3((nt + 63) / 64), dim3(256), 0, s, nt, P.nchunk, tx, part, u);
+}
+
+}  // namespace qol

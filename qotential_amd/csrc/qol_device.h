@@ -142,6 +142,14 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return y;
 }
 
+// the same by one third-order step, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2: the
+// estimate's error of at most 2.7e-8 leaves (5/16) e^3 < 1e-22, below rounding
+__device__ __forceinline__ double rsqrt_h3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 // 1/x for finite nonzero x: the hardware estimate refined by two Newton steps
 __device__ __forceinline__ double rcp_nr(double x) {
   double y = __builtin_amdgcn_rcp(x);

@@ -92,6 +92,7 @@ struct Engine {
   bool projected = false;      // the last eval ran the projection (it had RRQ pairs to run)
   DevBuf d_frame, d_edge, d_bX, d_cx, d_basis, d_Fq, d_Msl, d_Fn, d_G, d_Binv, d_scr;
   DevBuf d_ub, d_ubn, d_u, d_tcount, d_toffs, d_tcur, d_tpairs;
+  DevBuf d_fsrc, d_fpart;     // far field: packed sources, per-chunk sums
   RRQPanels RP{};
 
   Engine(i64 p, i64 npan, const double* sx, const double* snx, const double* sw, const double* rts,

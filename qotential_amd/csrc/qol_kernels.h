@@ -157,8 +157,15 @@ __global__ void target_count_kernel(int nnz, const int* tidx, int* tcount);
 __global__ void target_fill_kernel(int nnz, const int* tidx, const int* toffs, int* tcur, int* tpairs);
 __global__ void target_sum_kernel(int nt, const int* toffs, int* tpairs, const double* val, double* u);
 __global__ void hbm_copy_kernel(size_t n, const double2* src, double2* dst);
-__global__ void far_direct_kernel(int nt, const double* tx, int ns, const double* sx, const double* snx,
-                                  const double* sw, const double* ub, const double* ubn, double* u);
+// far field: targets per thread, sources per chunk and chunk count; launch_far's
+// src holds 8 ns doubles, part nchunk nt doubles
+struct FarPlan {
+  int per, len, nchunk;
+};
+FarPlan far_plan(int nt, int ns);
+void launch_far(const FarPlan& P, int nt, const double* tx, int ns, const double* sx, const double* snx,
+                const double* sw, const double* ub, const double* ubn, double* src, double* part, double* u,
+                hipStream_t s);
 __global__ void triplet_kernel(int nnz, int h, const int* tidx, const int* ppanel, const int* trow,
                                const int* offs, const double* tx, const double* sx, const double* snx,
                                const double* sw, const double* wout, int64_t* si, int64_t* sj, double* vs,
