@@ -293,6 +293,8 @@ Engine::~Engine() {
   if (stream) (void)hipStreamDestroy(stream);
 }
 
+// The boundary tangents' part of d_basis (at most 104 KB) is not counted: the
+// largest call qol_rrq_noalloc_ accepts stays what it was without it.
 size_t Engine::one_panel_bytes(i64 p, i64 m, i64 ichart, bool square) {
   const OrderTables& T = order_tables(p, square);
   LevelArgs LA{};
@@ -579,7 +581,7 @@ void Engine::alloc_rrq() {
   d_edge.alloc(sizeof(double) * 9 * nq * np_);
   d_bX.alloc(sizeof(double) * 6 * nb * np_);
   d_cx.alloc(sizeof(double) * 3 * (size_t)h * np_);
-  d_basis.alloc(sizeof(double) * 2 * nb * (size_t)(p * (p + 1) / 2) * np_);  // boundary harmonics of degree < p
+  d_basis.alloc(sizeof(double) * rrq_basis_doubles(p, nq) * np_);
   d_Fq.alloc(sizeof(double) * 3 * (size_t)h * h * np_);
   d_Msl.alloc(sizeof(double) * (size_t)h * h * np_);
   d_Fn.alloc(sizeof(double) * (size_t)h * h * np_);
@@ -717,13 +719,10 @@ void Engine::eval(int exterior, double side_tol, bool want_omega) {
   HIPCHK(hipStreamWaitEvent(stream, ev_edge, 0));
   HIPCHK(hipStreamWaitEvent(stream, ev_system, 0));
   rec(7, 0, stream);
-  const size_t lds3 = rrq_target_smem(p, h, nq, ncoef);
-  set_lds((const void*)rrq_target_kernel, lds3);
-  hipLaunchKernelGGL(rrq_target_kernel, dim3(npan), dim3(256), lds3, stream, tab->RT, RP, (const int*)d_lpairs.ptr,
-                     (const int*)d_lstart.ptr, (const int*)d_ltot.ptr, npan, (const int*)d_tidx.ptr,
-                     (const double*)d_tx.ptr, (const int*)d_nrrq.ptr, (const double*)d_w1.ptr,
-                     (const double*)d_oe.ptr, (double*)d_vt.ptr, want_omega ? (double*)d_omega.ptr : nullptr,
-                     want_omega ? (double*)d_ias.ptr : nullptr);
+  launch_rrq_target(tab->RT, RP, (const int*)d_lpairs.ptr, (const int*)d_lstart.ptr, (const int*)d_ltot.ptr, npan,
+                    (const int*)d_tidx.ptr, (const double*)d_tx.ptr, (const int*)d_nrrq.ptr, (const double*)d_w1.ptr,
+                    (const double*)d_oe.ptr, (double*)d_vt.ptr, want_omega ? (double*)d_omega.ptr : nullptr,
+                    want_omega ? (double*)d_ias.ptr : nullptr, nnz, stream);
   rec(7, 1, stream);
   HIPCHK(hipStreamWaitEvent(stream, ev_solve, 0));
   rec(9, 0, stream);

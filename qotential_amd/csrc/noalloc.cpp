@@ -2,7 +2,7 @@
 //
 // Every device buffer of the call (per-order tables, the panel, targets, pair
 // lists, level geometry, RRQ set-up and per-pair data) is sliced from `scratch`,
-// a file-scope device array of kScratchBytes per GPU that lives until the
+// a file-scope device array of kScratchBytes (and some slack) per GPU that lives until the
 // process ends; the call itself makes no hipMalloc / hipFree.  Set-up happens
 // once per device, on the first call with that device current: the array's
 // device address (hipGetSymbolAddress) and one stream with its events.
@@ -32,10 +32,11 @@ using namespace qol;
 
 namespace {
 
-constexpr size_t kScratchBytes = (size_t)64 << 20;  // 64 MiB per GPU
+constexpr size_t kScratchBytes = (size_t)64 << 20;  // per GPU: what a call's counted buffers may take
+constexpr size_t kScratchSlack = (size_t)1 << 20;   // and room for the few that one_panel_bytes leaves out
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) char scratch[kScratchBytes];
+__device__ __align__(256) char scratch[kScratchBytes + kScratchSlack];
 
 struct DeviceScratch {
   std::mutex mu;     // serialises calls on this device
@@ -108,7 +109,7 @@ extern "C" void qol_rrq_noalloc_(const int64_t* m, const double* tx, const int64
     if (mm > 0) {
       DeviceScratch& d = device_scratch();
       std::lock_guard<std::mutex> g(d.mu);
-      Arena a{d.ptr, kScratchBytes, 0};
+      Arena a{d.ptr, kScratchBytes + kScratchSlack, 0};
       ArenaScope scope(&a);
       Engine e(p, 1, sx, snx, sw, rts, rps, *ichart, sxbd_chart, rv_chart, false, &d.ss, sq);
       e.set_level_mode(ad, sq);

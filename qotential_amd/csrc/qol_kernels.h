@@ -55,7 +55,8 @@ struct RRQPanels {
   double* edge;    // [npan][3][3][nq] power-basis coefficients of the frame boundary (s in [-1, 1])
   double* bX;      // [npan][3*nq][6] boundary X, dX (frame)
   double* cx;      // [npan][3][h] Koornwinder coefficients of the geometry (original coords)
-  double* basis;   // [npan][3*nq][p(p+1)/2] complex: H'_n^m (n < p) at the boundary nodes
+  double* basis;   // [npan][3*nq][p(p+1)/2 + (p-1)(p+2)/2] complex at the boundary nodes: H'_n^m
+                   // (n < p), then T_n^m (n < p - 1, m <= n + 1), its combination with the tangent
   double* Fq;      // [npan][h][h][3] pure quaternions grad F_k(y_i)
   double* Msl;     // [npan][h][h] Msl^T (column-major)
   double* Fn;      // [npan][h][h] F_k at the nodes, F(i,k)
@@ -190,13 +191,13 @@ size_t rrq_edge_order_ints(int64_t nnz);
 void launch_rrq_edge(RRQTables T, RRQPanels P, const int* lpairs, const int* ltot, const int* ppanel,
                      const int* tidx, const double* tx, const double* pq, double* w1, double* root, double* oe,
                      int* order, int64_t nnz, hipStream_t s, hipEvent_t mid);
-__global__ void rrq_target_kernel(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot,
-                                  int npan, const int* tidx, const double* tx, const int* nrrq, const double* w1g,
-                                  const double* oeg, double* vt, double* omega_out, double* ias_out);
+void launch_rrq_target(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
+                       const int* tidx, const double* tx, const int* nrrq, const double* w1g, const double* oeg,
+                       double* vt, double* omega_out, double* ias_out, int64_t nnz, hipStream_t s);
 void launch_rrq_weights(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
                         const int* nrrq, const double* vt, double* wout, hipStream_t s);
 size_t rrq_frame_smem(int h, int nq);
 size_t rrq_system_smem(int h, int nq, int ncoef);
-size_t rrq_target_smem(int p, int h, int nq, int ncoef);
+size_t rrq_basis_doubles(int p, int nq);  // RRQPanels::basis, per panel
 
 }  // namespace qol

@@ -148,6 +148,11 @@ size_t rrq_frame_smem(int h, int nq) {
   const int nb = 3 * nq;
   return (size_t)(7 * h + 3 * h + 16 + 9 * nq + 6 * nb + h) * sizeof(double);
 }
+// complex values per boundary node in P.basis: H'_n^m (n < p, 0 <= m <= n), then
+// T_n^m (n < p - 1, 0 <= m <= n + 1)
+__host__ __device__ inline int rrq_basis_cols(int p) { return p * (p + 1) / 2 + (p - 1) * (p + 2) / 2; }
+size_t rrq_basis_doubles(int p, int nq) { return (size_t)2 * 3 * nq * rrq_basis_cols(p); }
+
 size_t rrq_system_smem(int h, int nq, int ncoef) {
   const int nb = 3 * nq;
   size_t a = (size_t)(6 * h + 16 + 6 * nb) * sizeof(double);
@@ -334,14 +339,31 @@ __global__ void __launch_bounds__(256) rrq_panel_system_kernel(RRQTables T, RRQP
   for (int i = threadIdx.x; i < 16; i += blockDim.x) fr[i] = P.frame[(size_t)k * 16 + i];
   for (int i = threadIdx.x; i < 6 * nb; i += blockDim.x) bx[i] = P.bX[(size_t)k * nb * 6 + i];
   __syncthreads();
-  // harmonic values H'_n^m of degree n < p at the boundary nodes: the moments
-  // of every pair are contracted against these (their gradients and V are
-  // fixed combinations of them, applied after the contraction)
+  // harmonic values H'_n^m of degree n < p at the boundary nodes, and for n < p - 1
+  // their combinations T_n^m with the edge tangent: the moments of every pair are
+  // contracted against these (their gradients are fixed combinations, applied
+  // after the contraction)
   for (int ib = threadIdx.x; ib < nb; ib += blockDim.x) harm_vals(bx + 6 * ib, p, Hs + (size_t)ib * ncoef);
   __syncthreads();
-  const int nc1 = p * (p + 1) / 2;
-  cd* Ho = (cd*)P.basis + (size_t)k * nb * nc1;
-  for (int it = threadIdx.x; it < nb * nc1; it += blockDim.x) Ho[it] = Hs[(size_t)(it / nc1) * ncoef + it % nc1];
+  const int nc1 = p * (p + 1) / 2, ncb = rrq_basis_cols(p);
+  cd* Ho = (cd*)P.basis + (size_t)k * nb * ncb;
+  for (int it = threadIdx.x; it < nb * ncb; it += blockDim.x) {
+    const int ib = it / ncb, kk = it % ncb;
+    const cd* H = Hs + (size_t)ib * ncoef;
+    if (kk < nc1) {
+      Ho[it] = H[kk];
+    } else {
+      // T_n^m = dX_Z H'_n^m + i/2 (dW H'_n^{m-1} + conj(dW) H'_n^{m+1}), m = 0..n+1
+      const int j = kk - nc1;
+      int n = 0;
+      while ((n + 1) * (n + 4) / 2 <= j) ++n;
+      const int m = j - n * (n + 3) / 2;
+      const double* d = bx + 6 * ib + 3;
+      const cd dw = cmk(d[1], d[2]);
+      Ho[it] = cadd(cscale(hget(H, n, m), d[0]),
+                    cscale(cmuli(cadd(cmul(dw, hget(H, n, m - 1)), cmul(cconj(dw), hget(H, n, m + 1)))), 0.5));
+    }
+  }
   __syncthreads();
   // quaternion system at the nodes.  F_k = Im((-i)^m H'_n^m), n=1..p, m=1..n.
   // Fq(i,k) = grad F_k(y_i) as a pure quaternion; the real 4h x 4h matrix of the
@@ -1803,8 +1825,8 @@ __device__ double project_end(const double* cx, const double* __restrict__ kt, i
 //   rrq_edge_kernel     one thread per (pair, edge): complex root, SSQ weights
 //                       for the 1/r line kernel and the edge's solid-angle
 //                       line integral                              -> w1[r][3nq], oe[r][3]
-//   rrq_target_kernel   one workgroup per panel, pairs in tiles: boundary
-//                       moments, degree recursion, weights operator.
+//   rrq_target_kernel   a panel's pairs in tiles: boundary moments, degree
+//                       recursion, moment vectors                   -> vt
 
 __device__ __forceinline__ int rrq_list_base(const int* ltot) { return ltot[0] + ltot[1] + ltot[2] + ltot[3]; }
 
@@ -2164,297 +2186,266 @@ void launch_rrq_edge(RRQTables T, RRQPanels P, const int* lpairs, const int* lto
 #undef QOL_EDGE
 }
 
-// LDS plan of rrq_target_kernel: fixed panel data plus per-target slots.  Per
-// target: the frame point (6), w1 (nb), the raw moments, later the moment vector
-// (rstr doubles), solid angle and Lambda (4), and the node weights, later the
-// boundary moments (mstr complex).
-__host__ __device__ inline int rrq_raw_doubles(int p) { return 2 * (3 * (p * (p + 1) / 2) + 9 * ((p - 1) * p / 2)); }
-__host__ __device__ inline int rrq_rstr(int p, int h) { const int r = rrq_raw_doubles(p); return r > 5 * h ? r : 5 * h; }
-__host__ __device__ inline int rrq_mstr(int nb, int ncoef) { return 6 * nb > 5 * ncoef ? 6 * nb : 5 * ncoef; }
-__host__ __device__ inline size_t rrq_target_fixed(int h, int nq) {
-  return (size_t)(16 + 6 * 3 * nq) * 8;
-}
-__host__ __device__ inline size_t rrq_target_per(int p, int h, int nq, int ncoef) {
-  const int nb = 3 * nq;
-  return (size_t)(6 + nb + rrq_rstr(p, h) + 4) * 8 + (size_t)rrq_mstr(nb, ncoef) * 16;
-}
-__host__ __device__ int rrq_tile(int p, int h, int nq, int ncoef) {
-  // about 48 KB per workgroup keeps three workgroups on a CU
-  const size_t budget = 48 * 1024, fixed = rrq_target_fixed(h, nq), per = rrq_target_per(p, h, nq, ncoef);
-  int t = budget > fixed + per ? (int)((budget - fixed) / per) : 1;
-  return t > 16 ? 16 : (t < 1 ? 1 : t);
-}
-size_t rrq_target_smem(int p, int h, int nq, int ncoef) {
-  return rrq_target_fixed(h, nq) + rrq_target_per(p, h, nq, ncoef) * rrq_tile(p, h, nq, ncoef);
-}
+// Boundary moments, degree recursion and moment vectors of a panel's RRQ pairs, in
+// tiles of up to kRT = 16 pairs.
+//
+// With z = X_b - x, w = (SSQ weight)/|z| and dX the edge tangent at boundary node
+// b, a pair needs chi_n^m = sum_b (w z x dX) . grad H'_n^m and the quaternion
+// moments alpha_n^m = sum_b (w z) (x) V_n^m, V_n^m = n (dX_Z G + i/2 (dW G^{m-1} +
+// conj(dW) G^{m+1})), G = grad H'_{n-1}^m.  Gradients are fixed combinations of
+// harmonics one degree lower, and that step commutes with the combination over
+// dX, so everything follows from six real node weights: R_c = sum_b (w z x dX)_c H'
+// and S_c = sum_b (w z_c) T (T: rrq_panel_system_kernel),
+//   chi  = n (R_0^m + i/2 (R_1^{m-1} + R_1^{m+1}) + 1/2 (R_2^{m+1} - R_2^{m-1}))
+//   U_cd = n (n-1) (S_c^m, i/2 (S_c^{m-1} + S_c^{m+1}), 1/2 (S_c^{m+1} - S_c^{m-1}))_d
+//   alpha = (-(U_00 + U_11 + U_22), U_12 - U_21, U_20 - U_02, U_01 - U_10)
+// (twelve weights against H' alone, a general combination of 39 sums per
+// coefficient and a barrier per degree took 2.6 ms on the 48 x 120 order-8
+// workload, 320,000 pairs, of which the sums 0.9, the combination 0.5 and the
+// degrees 0.75; now 0.96, of which the weights 0.15 and the sums about 0.4).
+//
+// The sums are a matrix product on the FP64 matrix cores: rows (pair, weight),
+// columns the real and imaginary parts of the panel's H' or T, inner dimension
+// the boundary nodes.  The rows of one tile share every harmonic loaded, the
+// weights go through LDS once, and the results land in LDS for the recursion, one
+// lane per (pair, component), which keeps its previous degree in registers and
+// needs no barrier.
+constexpr int kRT = 16;   // pairs a tile at most (12 and 10: 1.07 and 1.10 ms)
+constexpr int kRW = 4;    // waves a workgroup: with 5, two workgroups a CU fit instead of three (1.6 ms)
 
-// entry (n, m) of a raw-moment array of real weights, any m: conjugation and the
-// sign (-1)^m for m < 0, zero outside |m| <= n (selects, no branches)
-__device__ __forceinline__ cd rget(const cd* __restrict__ A, int n, int m) {
-  const int am = m < 0 ? -m : m;
-  const bool ok = n >= 0 && am <= n;
-  const cd v = A[ok ? hidx(n, am) : 0];
-  const double sr = (m < 0 && (am & 1)) ? -1.0 : 1.0, si = m < 0 ? -sr : sr;
-  return ok ? cmk(sr * v.re, si * v.im) : cmk(0.0, 0.0);
-}
-
-// The boundary moments of one target, chi_n^m = sum_b a . grad H'_n^m and
-// alpha_n^m = sum_b z (x) V_n^m with V_n^m = n [dX_Z grad H'_{n-1}^m + i/2 (dW
-// grad H'_{n-1}^{m-1} + conj(dW) grad H'_{n-1}^{m+1})] (a = (w1/R)(z x dX), z
-// scaled by w1/R, (x) the quaternion product (-z.V, z x V)), from raw moments
-// of real node weights: R_c = sum_b a_c H'_{n'}^{m'} (n' < p) and Z_cj = sum_b
-// z_c dX_j H'_{n'}^{m'} (n' < p - 1).  The gradient is linear with constant
-// coefficients in the harmonics of one degree lower (harm_grad), and the
-// weights are real, so the conjugation rule for negative orders carries over to
-// the raw moments.
-__device__ __forceinline__ void moments_from_raw(const cd* __restrict__ R, int p, int n, int m, cd* M) {
-  const int nc1 = p * (p + 1) / 2, nc2 = (p - 1) * p / 2;
-  for (int c = 0; c < 5; ++c) M[c] = cmk(0.0, 0.0);
-  if (n < 1) return;
-  // chi = sum_c (grad of R_c at degree n)_c
-  {
-    const cd a = rget(R, n - 1, m), lo = rget(R + nc1, n - 1, m - 1), hi = rget(R + nc1, n - 1, m + 1);
-    const cd lo2 = rget(R + 2 * nc1, n - 1, m - 1), hi2 = rget(R + 2 * nc1, n - 1, m + 1);
-    M[0] = cscale(cadd(cadd(a, cscale(cmuli(cadd(lo, hi)), 0.5)), cscale(csub(hi2, lo2), 0.5)), (double)n);
+template <int P>
+struct MomentPlan {
+  static constexpr int NB = 3 * (P + 2), KS = (NB + 3) / 4;            // nodes, in steps of 4
+  static constexpr int CH = P * (P + 1), CT = (P - 1) * (P + 2);       // real columns of H' and T
+  static constexpr int NH = (CH + 15) / 16, NN = NH + (CT + 15) / 16;  // 16-column tiles of H', of both
+  static constexpr int RS = 3 * (CH + CT);                             // sums per pair
+  static constexpr int rows(int t) { return 16 * ((3 * t + 15) / 16); }
+  // the region holds the node weights (both sets, and w), then the sums
+  static constexpr int region(int t) {
+    const int w = 2 * 4 * KS * rows(t) + t * NB;
+    return w > t * RS ? w : t * RS;
   }
-  if (n < 2) return;
-  // U_cd = sum_b z_c V_d; alpha = (-(U_00 + U_11 + U_22), U_12 - U_21, U_20 - U_02, U_01 - U_10)
-  // added into M (LDS) term by term
-  const int n2 = n - 2;
-  const double g = 0.5 * (double)(n - 1);
-#pragma unroll 1
-  for (int c = 0; c < 3; ++c) {
-    const cd* Z = R + 3 * nc1 + 3 * c * nc2;
-    cd z0[3], z1[5], z2[5];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) z0[j] = rget(Z, n2, m - 1 + j);
-#pragma unroll
-    for (int j = 0; j < 5; ++j) { z1[j] = rget(Z + nc2, n2, m - 2 + j); z2[j] = rget(Z + 2 * nc2, n2, m - 2 + j); }
-    // with G the gradient at degree n-1 (harm_grad) and g = (n-1)/2:
-    // U_cd = n (G(Z_c0)^m + i/2 [G(Z_c1)^{m-1} + G(Z_c1)^{m+1} + i (G(Z_c2)^{m-1} -
-    // G(Z_c2)^{m+1})])_d = n g (t0 + i/2 a - b/2)_d, the components collected:
-    //   t0 = (2 z0_m, i (z0_{m-1} + z0_{m+1}), z0_{m+1} - z0_{m-1})
-    //   a  = (2 (z1_{m-1} + z1_{m+1}), i (z1_{m-2} + 2 z1_m + z1_{m+2}), z1_{m+2} - z1_{m-2})
-    //   b  = (2 (z2_{m-1} - z2_{m+1}), i (z2_{m-2} - z2_{m+2}), 2 z2_m - z2_{m-2} - z2_{m+2})
-    const double f = (double)n * g;
-    cd u[3];
-    {
-      const cd t0 = cscale(z0[1], 2.0), a = cscale(cadd(z1[1], z1[3]), 2.0), b = cscale(csub(z2[1], z2[3]), 2.0);
-      u[0] = cscale(cadd(t0, csub(cscale(cmuli(a), 0.5), cscale(b, 0.5))), f);
-    }
-    {
-      const cd t0 = cmuli(cadd(z0[0], z0[2])), a = cmuli(cadd(cadd(z1[0], z1[4]), cscale(z1[2], 2.0)));
-      const cd b = cmuli(csub(z2[0], z2[4]));
-      u[1] = cscale(cadd(t0, csub(cscale(cmuli(a), 0.5), cscale(b, 0.5))), f);
-    }
-    {
-      const cd t0 = csub(z0[2], z0[0]), a = csub(z1[4], z1[0]), b = csub(cscale(z2[2], 2.0), cadd(z2[0], z2[4]));
-      u[2] = cscale(cadd(t0, csub(cscale(cmuli(a), 0.5), cscale(b, 0.5))), f);
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      if (d == c) M[1] = csub(M[1], u[d]);
-      else if ((d - c + 3) % 3 == 1) M[1 + (c + 2) % 3 + 1] = cadd(M[1 + (c + 2) % 3 + 1], u[d]);  // U_01, U_12, U_20
-      else M[1 + (c + 1) % 3 + 1] = csub(M[1 + (c + 1) % 3 + 1], u[d]);                            // U_02, U_10, U_21
-    }
+  static constexpr size_t bytes(int t) { return 8 * (size_t)(region(t) + 6 * NB + 4 * kRT); }
+  // three workgroups a CU up to order 8, two above (160 KB of LDS)
+  static constexpr int tile() {
+    int t = kRT;
+    while (t > 1 && bytes(t) > (P <= 8 ? 54400 : 81600)) --t;
+    return t;
   }
-}
+  static constexpr int T = tile(), MT = rows(T) / 16, TW = (NN + kRW - 1) / kRW;
+};
 
-__global__ void __launch_bounds__(256) rrq_target_kernel(RRQTables T, RRQPanels P, const int* __restrict__ lpairs,
-                                                         const int* __restrict__ lstart, const int* __restrict__ ltot,
-                                                         int npan, const int* __restrict__ tidx,
-                                                         const double* __restrict__ tx, const int* __restrict__ nrrq,
-                                                         const double* __restrict__ w1g, const double* __restrict__ oeg,
-                                                         double* __restrict__ vt, double* __restrict__ omega_out,
-                                                         double* __restrict__ ias_out) {
+template <int P>
+__global__ void __launch_bounds__(64 * kRW, P <= 8 ? 3 : 2)
+    rrq_target_kernel(RRQTables tab, RRQPanels pan, const int* __restrict__ lpairs, const int* __restrict__ lstart,
+                      const int* __restrict__ ltot, int npan, const int* __restrict__ tidx,
+                      const double* __restrict__ tx, const int* __restrict__ nrrq, const double* __restrict__ w1g,
+                      const double* __restrict__ oeg, double* __restrict__ vt, double* __restrict__ omega_out,
+                      double* __restrict__ ias_out) {
+  using M = MomentPlan<P>;
+  constexpr int NB = M::NB, KS = M::KS, T = M::T, H = P * (P + 1) / 2;
   const int k = blockIdx.x;
   const int nmine = nrrq[k];
-  if (nmine == 0) return;
-  const int h = T.h, nq = T.nq, p = T.p, nb = 3 * nq, ncoef = T.ncoef, H4 = 4 * h, H5 = 5 * h;
-  const int nc1 = p * (p + 1) / 2, nc2 = (p - 1) * p / 2;
-  const int TT = rrq_tile(p, h, nq, ncoef), rstr = rrq_rstr(p, h), mstr = rrq_mstr(nb, ncoef);
+  if ((int)blockIdx.y * T >= nmine) return;
   extern __shared__ double sm[];
-  double* fr = sm;                        // 16
-  double* bx = fr + 16;                   // [nb][6]
-  double* tX = bx + 6 * nb;               // [TT][6]   frame X, original x
-  double* w1 = tX + 6 * TT;               // [TT][nb]
-  double* rv = w1 + (size_t)nb * TT;      // [TT][rstr]: raw moments, later the moment vector v
-  double* tq = rv + (size_t)rstr * TT;    // [TT][4]: solid angle, Lambda
-  cd* mom = (cd*)(tq + 4 * TT);           // [TT][mstr]: node weights [nb][12], later moments [ncoef][5]
-  __shared__ int plist[16];
-  for (int i = threadIdx.x; i < 16; i += blockDim.x) fr[i] = P.frame[(size_t)k * 16 + i];
-  for (int i = threadIdx.x; i < 6 * nb; i += blockDim.x) bx[i] = P.bX[(size_t)k * nb * 6 + i];
-  const double sigma = P.frame[(size_t)k * 16 + 13], alpha = P.frame[(size_t)k * 16 + 12];
-  const cd* Hb = (const cd*)P.basis + (size_t)k * nb * nc1;
+  double* rg = sm;                 // the region
+  double* bx = rg + M::region(T);  // [NB][6]
+  double* lam = bx + 6 * NB;       // [kRT][4]: sum_b w dX
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const double* fr = pan.frame + (size_t)k * 16;
+  for (int i = threadIdx.x; i < 6 * NB; i += blockDim.x) bx[i] = pan.bX[(size_t)k * NB * 6 + i];
+  const double* basis = pan.basis + (size_t)k * NB * (M::CH + M::CT);
   const int r0 = lstart[4 * (size_t)npan + k];
   const int* mine = lpairs + rrq_list_base(ltot) + r0;
-  for (int tile0 = 0; tile0 < nmine; tile0 += TT) {
-    const int nt = min(TT, nmine - tile0);
-    __syncthreads();
-    for (int t = threadIdx.x; t < nt; t += blockDim.x) plist[t] = mine[tile0 + t];
-    for (int i = threadIdx.x; i < nt * nb; i += blockDim.x)
-      w1[i] = w1g[(size_t)(r0 + tile0) * nb + i];
-    for (int t = threadIdx.x; t < nt; t += blockDim.x) {
-      const double* o = oeg + 3 * (size_t)(r0 + tile0 + t);
-      tq[4 * t] = o[0] + o[1] + o[2];
+  for (int tile0 = blockIdx.y * T; tile0 < nmine; tile0 += gridDim.y * T) {
+    const int nt = min(T, nmine - tile0), mt = (3 * nt + 15) / 16, rows = 16 * mt;
+    double *Wa = rg, *Wz = Wa + 4 * KS * rows, *wl = Wz + 4 * KS * rows;
+    __syncthreads();  // bx; the previous tile's sums are read
+    // node weights, rows (pair, component); the rows of nodes past NB are zero
+    for (int it = threadIdx.x; it < nt * 4 * KS; it += blockDim.x) {
+      const int ib = it / nt, t = it % nt;  // neighbouring lanes: neighbouring rows
+      double a[3] = {0.0, 0.0, 0.0}, zw[3] = {0.0, 0.0, 0.0};
+      if (ib < NB) {
+        const size_t g = (size_t)tidx[mine[tile0 + t]];
+        const double x[3] = {tx[3 * g], tx[3 * g + 1], tx[3 * g + 2]};
+        double X[3], zx[3];
+        to_frame(fr, x, X);
+        const double* Y = bx + 6 * ib;
+        const double z[3] = {Y[0] - X[0], Y[1] - X[1], Y[2] - X[2]};
+        const double wr =
+            w1g[(size_t)(r0 + tile0 + t) * NB + ib] * rsqrt_h3(z[0] * z[0] + z[1] * z[1] + z[2] * z[2]);
+        wl[t * NB + ib] = wr;
+        cross3(z, Y + 3, zx);
+        for (int c = 0; c < 3; ++c) {
+          a[c] = wr * zx[c];
+          zw[c] = wr * z[c];
+        }
+      }
+      for (int c = 0; c < 3; ++c) {
+        Wa[ib * rows + 3 * t + c] = a[c];
+        Wz[ib * rows + 3 * t + c] = zw[c];
+      }
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < nt; t += blockDim.x) {
-      const size_t g = (size_t)tidx[plist[t]];
-      const double x[3] = {tx[3 * g], tx[3 * g + 1], tx[3 * g + 2]};
-      to_frame(fr, x, tX + 6 * t);
-      tX[6 * t + 3] = x[0]; tX[6 * t + 4] = x[1]; tX[6 * t + 5] = x[2];
-    }
-    __syncthreads();
-    // node weights: a = (w1/R)(z x dX) and (w1/R) z_c dX_j
-    for (int it = threadIdx.x; it < nt * nb; it += blockDim.x) {
-      const int t = it / nb, ib = it % nb;
-      const double* Y = bx + 6 * ib;
-      const double z[3] = {Y[0] - tX[6 * t], Y[1] - tX[6 * t + 1], Y[2] - tX[6 * t + 2]};
-      const double wr = w1[(size_t)t * nb + ib] / sqrt(z[0] * z[0] + z[1] * z[1] + z[2] * z[2]);
-      w1[(size_t)t * nb + ib] = wr;  // w1/R from here on
-      double zx[3];
-      cross3(z, Y + 3, zx);
-      double* o = (double*)(mom + (size_t)t * mstr) + 12 * ib;
-      for (int c = 0; c < 3; ++c) o[c] = wr * zx[c];
-      for (int c = 0; c < 3; ++c)
-        for (int j = 0; j < 3; ++j) o[3 + 3 * c + j] = (wr * z[c]) * Y[3 + j];
-    }
-    __syncthreads();
-    // Lambda = sum (w1/R) dX per (target, component), into the spare slots of tq
-    for (int it = threadIdx.x; it < nt * 3; it += blockDim.x) {
-      const int t = it / 3, c = it % 3;
+    // Lambda = sum w dX, by the last wave
+    if (wv == kRW - 1 && lane < 3 * nt) {
+      const int t = lane / 3, c = lane % 3;
       double l = 0.0;
-      for (int ib = 0; ib < nb; ++ib) l += w1[(size_t)t * nb + ib] * bx[6 * ib + 3 + c];
-      tq[4 * t + 1 + c] = l;
+      for (int ib = 0; ib < NB; ++ib) l = fma(wl[t * NB + ib], bx[6 * ib + 3 + c], l);
+      lam[4 * t + c] = l;
     }
-    // raw moments, one thread per (target, harmonic of degree < p): the three
-    // a-weights always, the nine z dX weights for degrees < p - 1; consecutive
-    // threads read consecutive harmonics of a node
-    for (int it = threadIdx.x; it < nt * nc1; it += blockDim.x) {
-      const int t = it / nc1, kk = it % nc1;
-      const bool zp = kk < nc2;
-      const double* wt = (const double*)(mom + (size_t)t * mstr);
-      double acc[24];
+    // the sums: this wave's column tiles, all row tiles (lane numbers the compiler
+    // cannot tell are the same for every tile: it would keep the addresses they
+    // give in registers throughout, and spill)
+    int li = lane & 15, lk = lane >> 4;
+    asm volatile("" : "+v"(li), "+v"(lk));
+    qd4 acc[M::TW][M::MT];
 #pragma unroll
-      for (int c = 0; c < 24; ++c) acc[c] = 0.0;
-      // the harmonics of kHB nodes are loaded together (loads in flight)
-      constexpr int kHB = 6;
-      for (int ib0 = 0; ib0 < nb; ib0 += kHB) {
-        cd hb[kHB];
+    for (int q = 0; q < M::TW; ++q) {
 #pragma unroll
-        for (int u = 0; u < kHB; ++u) hb[u] = Hb[(size_t)min(ib0 + u, nb - 1) * nc1 + kk];
+      for (int m = 0; m < M::MT; ++m) acc[q][m] = qd4{0.0, 0.0, 0.0, 0.0};
+      const int tl = wv + kRW * q;
+      if (tl < M::NN) {
+        const bool tt = tl >= M::NH;
+        const int col = tt ? M::CH + min(16 * (tl - M::NH) + li, M::CT - 1) : min(16 * tl + li, M::CH - 1);
+        const double* W = tt ? Wz : Wa;
+        double b[KS];
 #pragma unroll
-        for (int u = 0; u < kHB; ++u) {
-          if (ib0 + u >= nb) break;
-          const cd hv = hb[u];
-          const double* w = wt + 12 * (ib0 + u);
+        for (int s = 0; s < KS; ++s) b[s] = basis[(size_t)min(4 * s + lk, NB - 1) * (M::CH + M::CT) + col];
 #pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            acc[2 * q] = fma(w[q], hv.re, acc[2 * q]);
-            acc[2 * q + 1] = fma(w[q], hv.im, acc[2 * q + 1]);
+        for (int m = 0; m < M::MT; ++m)
+          if (m < mt)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+              acc[q][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(W[(4 * s + lk) * rows + 16 * m + li], b[s], acc[q][m],
+                                                               0, 0, 0);
+      }
+    }
+    __syncthreads();  // the weights are read: the sums take their place
+#pragma unroll
+    for (int q = 0; q < M::TW; ++q) {
+      const int tl = wv + kRW * q;
+      const bool tt = tl >= M::NH;
+      const int col = 16 * (tt ? tl - M::NH : tl) + li;
+      if (tl < M::NN && col < (tt ? M::CT : M::CH)) {
+#pragma unroll
+        for (int m = 0; m < M::MT; ++m)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int row = 16 * m + 4 * j + lk, t = row / 3, c = row % 3;
+            if (t < nt) rg[t * M::RS + (tt ? 3 * M::CH + c * M::CT : c * M::CH) + col] = acc[q][m][j];
           }
-          if (zp) {
+      }
+    }
+    __syncthreads();
+    // the recursion in degree, component c = 0 (chi) or 1..4 (alpha) of pair t:
+    //   E_n^m = f1 base_n^m + f2 (x_Z E_{n-1}^m + i/2 (w E_{n-1}^{m-1} + conj(w) E_{n-1}^{m+1}))
+    //   base  = s0 A^m + i h1 (B^{m-1} + B^{m+1}) + h2 (C^{m+1} - C^{m-1})
+    // with (f1, f2) = (1, 1) for chi, (n, n / (n - 1)) for alpha, and A, B, C three
+    // of the sums R (degree n - 1) or S (degree n - 2, one entry earlier)
+    const int t = threadIdx.x % kRT, c = threadIdx.x / kRT;
+    if (c < 5 && t < nt) {
+      const int pair = mine[tile0 + t];
+      const size_t g = (size_t)tidx[pair];
+      const double x[3] = {tx[3 * g], tx[3 * g + 1], tx[3 * g + 2]};
+      double X[3];
+      to_frame(fr, x, X);
+      const double* o = oeg + 3 * (size_t)(r0 + tile0 + t);
+      const double om = o[0] + o[1] + o[2];
+      const double l0 = lam[4 * t], l1 = lam[4 * t + 1], l2 = lam[4 * t + 2];
+      const double sigma = fr[13], wr = 0.5 * X[1], wi = 0.5 * X[2], xz = X[0];
+      // (A, B, C) by component: chi R0 R1 R2; alpha S0 S1 S2 negated; -, -S2, S1; S2, -, -S0; -S1, S0, -
+      const double s0 = c == 0 ? 1.0 : (c == 2 ? 0.0 : (c == 3 ? 1.0 : -1.0));
+      const double h1 = c == 0 || c == 4 ? 0.5 : (c == 3 ? 0.0 : -0.5);
+      const double h2 = c == 0 || c == 2 ? 0.5 : (c == 4 ? 0.0 : -0.5);
+      const cd* base = (const cd*)(rg + t * M::RS) + (c == 0 ? 0 : 3 * (M::CH / 2) - 1);
+      const int ca = (c == 0 ? M::CH : M::CT) / 2;
+      const cd *A = base + (c == 3 ? 2 : (c == 4 ? 1 : 0)) * ca;
+      const cd *B = base + (c <= 1 ? 1 : (c == 2 ? 2 : 0)) * ca;
+      const cd *C = base + (c <= 1 ? 2 : (c == 2 ? 1 : 0)) * ca;
+      // slots of the moment vector: (x)-components -> h blocks 0..3, chi -> block 4
+      const double sgn = c == 0 || c == 1 ? sigma : -sigma;
+      double* v = vt + (size_t)r0 * 5 * H + tile0 + t + (size_t)(c == 0 ? 4 * H : (c - 1) * H) * nmine;
+      double* om_row = omega_out && c > 0 ? omega_out + (size_t)pair * 4 * H + (c - 1) * H : nullptr;
+      const double omf = 1.0 / (16.0 * atan(1.0)) / fr[12];
+      cd E[P + 2];
 #pragma unroll
-            for (int q = 3; q < 12; ++q) {
-              acc[2 * q] = fma(w[q], hv.re, acc[2 * q]);
-              acc[2 * q + 1] = fma(w[q], hv.im, acc[2 * q + 1]);
+      for (int m = 0; m < P + 2; ++m) E[m] = cmk(0.0, 0.0);
+      if (c == 0) {
+        E[0] = cmk(om, 0.0);
+        if (ias_out) ias_out[pair] = sigma * om;
+      }
+      int i = 0;
+#pragma unroll 1  // unrolled, its LDS reads are hoisted until the registers spill
+      for (int n = 1; n <= P; ++n) {
+        if (n == 1 && c > 0) {
+          // seeds: Lambda (x) grad H'_1^m with Lambda = -omega + sum w dX
+          E[0] = c == 1 ? cmk(-l0, 0.0) : (c == 2 ? cmk(-om, 0.0) : (c == 3 ? cmk(l2, 0.0) : cmk(-l1, 0.0)));
+          E[1] = c == 1 ? cmk(0.5 * l2, -0.5 * l1)
+                        : (c == 2 ? cmk(-0.5 * l1, -0.5 * l2) : (c == 3 ? cmk(0.5 * l0, -0.5 * om) : cmk(0.5 * om, 0.5 * l0)));
+        } else {
+          const double f1 = c == 0 ? 1.0 : (double)n, f2 = c == 0 ? 1.0 : (double)n / (double)(n - 1);
+          const int b0 = hidx(n - 1, 0);
+          cd bm = cmk(0.0, 0.0), cm = bm, bc = B[b0], cc = C[b0];  // entries m - 1 and m
+          cd lo = cmk(-E[1].re, E[1].im);                         // E_{n-1}^{-1}
+#pragma unroll
+          for (int m = 0; m <= P; ++m) {
+            if (m <= n) {
+              const cd a = m < n ? A[b0 + m] : cmk(0.0, 0.0);
+              const cd bp = m + 1 < n ? B[b0 + m + 1] : cmk(0.0, 0.0), cp = m + 1 < n ? C[b0 + m + 1] : cmk(0.0, 0.0);
+              if (m == 0) {
+                bm = cmk(-bp.re, bp.im);
+                cm = cmk(-cp.re, cp.im);
+              }
+              const double br = fma(h2, cp.re - cm.re, fma(-h1, bm.im + bp.im, s0 * a.re));
+              const double bi = fma(h2, cp.im - cm.im, fma(h1, bm.re + bp.re, s0 * a.im));
+              const cd mid = E[m], hi = E[m + 1];
+              const double sr = lo.re + hi.re, si = lo.im + hi.im, dr = lo.re - hi.re, di = lo.im - hi.im;
+              const double gr = fma(-wi, dr, fma(-wr, si, xz * mid.re));
+              const double gi = fma(-wi, di, fma(wr, sr, xz * mid.im));
+              E[m] = cmk(fma(f1, br, f2 * gr), fma(f1, bi, f2 * gi));
+              lo = mid;
+              bm = bc; bc = bp;
+              cm = cc; cc = cp;
             }
           }
         }
-      }
-      cd* R = (cd*)(rv + (size_t)t * rstr);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) R[q * nc1 + kk] = cmk(acc[2 * q], acc[2 * q + 1]);
-      if (zp) {
-#pragma unroll
-        for (int q = 3; q < 12; ++q) R[3 * nc1 + (q - 3) * nc2 + kk] = cmk(acc[2 * q], acc[2 * q + 1]);
+        for (int m = 1; m <= P; ++m)
+          if (m <= n) {
+            const double e = sgn * imrot(m, E[m]);
+            v[(size_t)i * nmine] = e;
+            if (om_row) om_row[i] = e * omf;
+            ++i;
+          }
       }
     }
-    __syncthreads();
-    // boundary moments chi (component 0) and alpha (1..4) per coefficient
-    for (int it = threadIdx.x; it < nt * ncoef; it += blockDim.x) {
-      const int t = it / ncoef, kk = it % ncoef;
-      int n = 0;
-      while (hidx(n + 1, 0) <= kk) ++n;
-      moments_from_raw((const cd*)(rv + (size_t)t * rstr), p, n, kk - hidx(n, 0), mom + (size_t)t * mstr + 5 * kk);
-    }
-    __syncthreads();
-    // seeds: W~_00 = solid angle, degree-1 Q = Lambda (x) grad H'_1^m with
-    // Lambda = -omega + sum (w1/R) dX
-    for (int t = threadIdx.x; t < nt; t += blockDim.x) {
-      cd* M = mom + (size_t)t * mstr;
-      const double om = tq[4 * t];
-      const double lam[3] = {tq[4 * t + 1], tq[4 * t + 2], tq[4 * t + 3]};
-      M[0] = cmk(om, 0.0);
-      for (int c = 1; c < 5; ++c) M[c] = cmk(0.0, 0.0);
-      for (int m = 0; m <= 1; ++m) {
-        cd g[3];
-        if (m == 0) { g[0] = cmk(1, 0); g[1] = cmk(0, 0); g[2] = cmk(0, 0); }
-        else { g[0] = cmk(0, 0); g[1] = cmk(0, 0.5); g[2] = cmk(-0.5, 0); }
-        cd* Q = M + (size_t)hidx(1, m) * 5 + 1;
-        Q[0] = cscale(cadd(cadd(cscale(g[0], lam[0]), cscale(g[1], lam[1])), cscale(g[2], lam[2])), -1.0);
-        Q[1] = cadd(cscale(g[0], -om), csub(cscale(g[2], lam[1]), cscale(g[1], lam[2])));
-        Q[2] = cadd(cscale(g[1], -om), csub(cscale(g[0], lam[2]), cscale(g[2], lam[0])));
-        Q[3] = cadd(cscale(g[2], -om), csub(cscale(g[1], lam[0]), cscale(g[0], lam[1])));
-      }
-    }
-    // recursion in degree, all (target, m, component) of one degree in parallel
-    for (int n = 1; n <= p; ++n) {
-      __syncthreads();
-      const double dn = (double)n;
-      const int ncomp = n >= 2 ? 5 : 1;  // degree 1 of components 1..4 is the seed
-      for (int it = threadIdx.x; it < nt * (n + 1) * ncomp; it += blockDim.x) {
-        const int c = it % ncomp, tm = it / ncomp;
-        const int t = tm / (n + 1), m = tm % (n + 1);
-        cd* M = mom + (size_t)t * mstr;
-        const double* X = tX + 6 * t;
-        const double xZ = X[0];
-        const cd w = cmk(X[1], X[2]), wc = cmk(X[1], -X[2]);
-        // entries of degree n-1 at m-1, m, m+1 (negative m by conjugation)
-        auto get = [&](int mm, int c) -> cd {
-          const int n1 = n - 1;
-          if (mm > n1 || mm < -n1) return cmk(0, 0);
-          if (mm >= 0) return M[(size_t)hidx(n1, mm) * 5 + c];
-          cd v = cconj(M[(size_t)hidx(n1, -mm) * 5 + c]);
-          return ((-mm) & 1) ? cmk(-v.re, -v.im) : v;
-        };
-        cd* E = M + (size_t)hidx(n, m) * 5;
-        const cd lo = get(m - 1, c), mid = get(m, c), hi = get(m + 1, c);
-        const cd t2 = cscale(cmuli(cadd(cmul(w, lo), cmul(wc, hi))), 0.5);
-        if (c == 0) E[0] = cadd(cadd(cscale(E[0], 1.0 / dn), cscale(mid, xZ)), t2);
-        else E[c] = cscale(cadd(E[c], cscale(cadd(cscale(mid, xZ), t2), dn)), 1.0 / (dn - 1.0));
-      }
-    }
-    __syncthreads();
-    // moment vector v = [rhs (4h); W (h)] into the (now free) raw-moment slots
-    for (int it = threadIdx.x; it < nt * h; it += blockDim.x) {
-      const int t = it / h, kk = it % h;
-      int n = 1;
-      while ((n + 1) * n / 2 <= kk) ++n;
-      const int m = kk - (n - 1) * n / 2 + 1;
-      const cd* E = mom + (size_t)t * mstr + (size_t)hidx(n, m) * 5;
-      double* v = rv + (size_t)t * rstr;
-      v[kk] = sigma * imrot(m, E[1]);
-      v[h + kk] = -sigma * imrot(m, E[2]);
-      v[2 * h + kk] = -sigma * imrot(m, E[3]);
-      v[3 * h + kk] = -sigma * imrot(m, E[4]);
-      v[4 * h + kk] = sigma * imrot(m, E[0]);
-    }
-    __syncthreads();
-    if (omega_out) {
-      const double f = 1.0 / (16.0 * atan(1.0)) / alpha;
-      for (int it = threadIdx.x; it < nt * H4; it += blockDim.x) {
-        const int t = it / H4, i = it % H4;
-        omega_out[(size_t)plist[t] * H4 + i] = rv[(size_t)t * rstr + i] * f;
-      }
-      for (int t = threadIdx.x; t < nt; t += blockDim.x) ias_out[plist[t]] = sigma * tq[4 * t];
-    }
-    // moment vectors to HBM, per panel transposed: vt[r0*5h + i*nrrq + t]
-    for (int it = threadIdx.x; it < nt * H5; it += blockDim.x) {
-      const int t = it % nt, i = it / nt;
-      vt[(size_t)r0 * H5 + (size_t)i * nmine + tile0 + t] = rv[(size_t)t * rstr + i];
-    }
+  }
+}
+
+// Workgroups per panel: one when the panels alone fill the chip, else enough for
+// 2,048 in all (a panel of 1,501 targets ran its 250 RRQ pairs on one workgroup
+// in 470 us), at most one per tile.
+void launch_rrq_target(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
+                       const int* tidx, const double* tx, const int* nrrq, const double* w1g, const double* oeg,
+                       double* vt, double* omega_out, double* ias_out, int64_t nnz, hipStream_t s) {
+  switch (T.p) {
+#define QOL_MOMENTS(P_)                                                                                             \
+  case P_: {                                                                                                        \
+    constexpr size_t lds = MomentPlan<P_>::bytes(MomentPlan<P_>::T);                                                \
+    if (lds > 64 * 1024)                                                                                            \
+      (void)hipFuncSetAttribute((const void*)rrq_target_kernel<P_>, hipFuncAttributeMaxDynamicSharedMemorySize,     \
+                                (int)lds);                                                                          \
+    const int64_t tiles = (nnz + MomentPlan<P_>::T - 1) / MomentPlan<P_>::T;                                        \
+    const int split = (int)std::max<int64_t>(1, std::min<int64_t>((2048 + npan - 1) / npan, tiles));                \
+    hipLaunchKernelGGL(rrq_target_kernel<P_>, dim3(npan, split), dim3(64 * kRW), lds, s, T, P, lpairs, lstart, ltot, \
+                       npan, tidx, tx, nrrq, w1g, oeg, vt, omega_out, ias_out);                                      \
+    break;                                                                                                          \
+  }
+    QOL_MOMENTS(2) QOL_MOMENTS(3) QOL_MOMENTS(4) QOL_MOMENTS(5) QOL_MOMENTS(6) QOL_MOMENTS(7) QOL_MOMENTS(8)
+    QOL_MOMENTS(9) QOL_MOMENTS(10) QOL_MOMENTS(11) QOL_MOMENTS(12)
+#undef QOL_MOMENTS
+    default: throw std::runtime_error("RRQ moments: patch orders 2..12 only");
   }
 }
 
