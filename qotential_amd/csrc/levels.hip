@@ -398,51 +398,184 @@ __global__ void __launch_bounds__(256) compact_kernel(const int* __restrict__ of
 // tile of 16 pairs of one level (tiles of the heaviest level first); for each
 // step of 4 level nodes every lane forms one kernel entry,
 //   S(pair m, node i) = w_i / (4 pi |x - y_i|),  D = w_i (x - y_i).n_i / (4 pi |x - y_i|^3)
-// (zero at coincident points), which is the A operand of
-// v_mfma_f64_16x16x4 against 4 rows of the level's interpolation matrix
-// (row-major, padded to 16*NT columns).  Accumulators: 16 pairs x 16*NT
-// outputs for S and for D.
+// (zero at coincident points), which is the A operand of the matrix cores against
+// 4 rows of the level's interpolation matrix (row-major, padded to whole 16-column
+// tiles).  Accumulators: 16 pairs x h outputs for S and for D, in NT tiles of 16
+// columns (v_mfma_f64_16x16x4) and, for the columns past them, NU units of 4
+// (v_mfma_f64_4x4x4_4b, whose four blocks take the same A operand, four pairs
+// each): 288 matrix-core cycles a step at h = 36 where a padded third tile takes
+// 384.
+//
+// Matrix and vector FP64 share one rate, so a step costs the sum of both (288 and
+// about 100 cycles at h = 36).  What kept the kernel from that was the vector
+// memory path: the lanes of a step load the same few 64-byte node records, 4 loads
+// a step beside the table's.  A tile's pairs come panel by panel, so its nodes are
+// loaded once per run of equal panels, contiguously, and handed out through LDS;
+// the next chunk is in flight meanwhile.  A chunk holds 16 nodes of up to 4 panels,
+// 8 of up to 8 or 4 of up to 16: the same 4 loads and 8.7 KB at most.
+// 48 x 120 order 8, 1.62 million pairs (75 GFLOP): 2.15 -> 1.59 ms (47 TFLOP/s, of
+// which the matrix cores issue 57 with their padding); 30,000 targets at order 12
+// 1.05 -> 0.94; order 6, 20,011 targets (tiles of 5 to 9 panels at levels 3 and 4)
+// 0.41 -> 0.30; one 4-node chunk size for all tiles or 17 KB of LDS a wave: 1.97 ms.
 
-// One step of the direct contraction: this lane's pair (A row m of the tile)
-// against node ic (the step's row kq), S and D entries on the vector ALUs, then
-// accS/D[q] += entry x row ic of the padded interpolation table B (columns
-// 16q + m) on the matrix cores.  use = false gives exactly zero entries (the
-// operands stay finite: clamped index, r^2 = 1), so no branch is needed.
-template <int NT>
-__device__ __forceinline__ void direct_step(const double* __restrict__ G, const double* __restrict__ B, int pad,
-                                            int m, int ic, bool use, double x0, double x1, double x2, double c4,
-                                            qd4* accS, qd4* accD) {
-  const double2* g2 = (const double2*)(G + 8 * ic);
-  const double2 ga = g2[0], gb = g2[1], gc = g2[2], gd = g2[3];
-  const double gx = ga.x, gy = ga.y, gz = gb.x, nx = gb.y, ny = gc.x, nz = gc.y, gw = gd.x;
-  double bq[NT];
+// orders a wave's LDS writes before its lanes' reads
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the matrix-core part of a step
+template <int NT, int NU>
+struct DirectAcc {
+  qd4 S[NT > 0 ? NT : 1], D[NT > 0 ? NT : 1];
+  double Su[NU > 0 ? NU : 1], Du[NU > 0 ? NU : 1];
+  __device__ __forceinline__ void zero() {
 #pragma unroll
-  for (int q = 0; q < NT; ++q) bq[q] = B[(size_t)ic * pad + 16 * q + m];
-  const double dx = x0 - gx, dy = x1 - gy, dz = x2 - gz;
-  const double rr = dx * dx + dy * dy + dz * dz;
-  const bool ok = use && rr > 1.0e-28;
-  const double rs = ok ? rr : 1.0;
-  // 1/r from the hardware estimate and two Newton steps
-  double y = __builtin_amdgcn_rsq(rs);
-  double t = rs * y;
-  y = fma(0.5 * y, fma(-t, y, 1.0), y);
-  t = rs * y;
-  y = fma(0.5 * y, fma(-t, y, 1.0), y);
-  const double msk = ok ? 1.0 : 0.0;
-  const double cw = msk * (c4 * gw);
-  const double dn = dx * nx + dy * ny + dz * nz;
-  const double s = cw * y;
-  const double d = cw * dn * (y * y * y);
-  // past a segment's last node the A entries are exactly zero and the B row
-  // (the clamped node's) is finite, so B needs no mask
+    for (int q = 0; q < NT; ++q) S[q] = D[q] = qd4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < NT; ++q) {
-    accS[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(s, bq[q], accS[q], 0, 0, 0);
-    accD[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, bq[q], accD[q], 0, 0, 0);
+    for (int u = 0; u < NU; ++u) Su[u] = Du[u] = 0.0;
+  }
+  // bq: this lane's entries of the step's table rows
+  __device__ __forceinline__ void add(double s, double d, const double* bq) {
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      S[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(s, bq[q], S[q], 0, 0, 0);
+      D[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, bq[q], D[q], 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      Su[u] = __builtin_amdgcn_mfma_f64_4x4x4f64(s, bq[NT + u], Su[u], 0, 0, 0);
+      Du[u] = __builtin_amdgcn_mfma_f64_4x4x4f64(d, bq[NT + u], Du[u], 0, 0, 0);
+    }
+  }
+  // rows of pairs 0..cnt-1 of the tile into wout, scaled by c4; pair: this lane's
+  // (pair lane % 16).  v_mfma_f64_16x16x4: lane l supplies A[l%16][l/16] and
+  // B[l/16][l%16] and holds D[4r + l/16][l%16] in slot r; v_mfma_f64_4x4x4_4b:
+  // A[4b + i][k] from lane i + 4b + 16k, B_b[k][j] from lane j + 4b + 16k,
+  // D[4b + i][j] in lane j + 4b + 16i
+  __device__ __forceinline__ void store(double c4, int h, int pair, int cnt, double* __restrict__ wout) const {
+    const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * r + kq;
+      const int pr = __shfl(pair, row, 64);
+      if (row < cnt) {
+        double* o = wout + (size_t)pr * 2 * h;
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const int col = 16 * q + m;
+          if (col < h) {
+            o[col] = c4 * S[q][r];
+            o[h + col] = c4 * D[q][r];
+          }
+        }
+      }
+    }
+    if (NU > 0) {
+      const int row = 4 * (m >> 2) + kq;
+      const int pr = __shfl(pair, row, 64);
+      if (row < cnt) {
+        double* o = wout + (size_t)pr * 2 * h;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          const int col = 16 * NT + 4 * u + (m & 3);
+          if (col < h) {
+            o[col] = c4 * Su[u];
+            o[h + col] = c4 * Du[u];
+          }
+        }
+      }
+    }
+  }
+};
+
+// base[offset / 8] with a uniform base and a 32-bit byte offset: one load
+// instruction, no 64-bit address arithmetic
+template <class V>
+__device__ __forceinline__ V load_at(const void* base, unsigned offset) {
+  return *(const V*)((const char*)base + offset);
+}
+
+// this lane's table entries of row i of B (below 2^32 bytes in all): tile columns
+// 16q + m, unit columns 16 NT + 4u + m % 4
+template <int NT, int NU>
+__device__ __forceinline__ void direct_row(const double* __restrict__ B, unsigned i, unsigned m, double* bq) {
+  const unsigned o = i * (8 * 16 * (NT + (NU > 0 ? 1 : 0)));
+#pragma unroll
+  for (int q = 0; q < NT; ++q) bq[q] = load_at<double>(B, o + 8 * (m + 16 * q));
+#pragma unroll
+  for (int u = 0; u < NU; ++u) bq[NT + u] = load_at<double>(B, o + 8 * ((m & 3) + 16 * NT + 4 * u));
+}
+
+// this lane's entries (without 1/(4 pi)) from its node record g2 = (x, y, z, nx,
+// ny, nz, w, -); use = false gives exactly zero ones
+__device__ __forceinline__ void direct_entry(const double2 ga, const double2 gb, const double2 gc, double gw, bool use,
+                                             double x0, double x1, double x2, double& s, double& d) {
+  const double dx = x0 - ga.x, dy = x1 - ga.y, dz = x2 - gb.x;
+  const double rr = fma(dz, dz, fma(dy, dy, dx * dx));
+  const double dn = fma(dz, gc.y, fma(dy, gc.x, dx * gb.y));
+  const double y = use && rr > 1.0e-28 ? rsqrt_h3(rr) : 0.0;
+  s = gw * y;
+  d = s * (dn * (y * y));
+}
+
+// One tile whose nodes are staged through LDS in chunks of C nodes of each of its
+// nrun <= 64 / C panels: one load of the wave takes the chunk of 16 / C panels, C
+// nodes of four 16-byte parts each.  The runs' chunks lie 64 C + 16 bytes apart, so
+// the 16 pairs' records of one node fall in different banks.
+constexpr int kDBuf = 16 * (8 * 4 + 2);  // doubles a buffer takes at most (C = 4: 16 runs)
+template <int C, int NT, int NU>
+__device__ __forceinline__ void direct_staged(double (*buf)[kDBuf], const int* run_panel, int nrun, int run,
+                                              const double* G0, size_t gstride, const double* __restrict__ B, int n,
+                                              bool live, double x0, double x1, double x2, DirectAcc<NT, NU>& acc) {
+  constexpr int RL = 16 / C, STR = 8 * C + 2;
+  const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
+  const int sub = lane / (4 * C), part = lane % (4 * C);  // run RL r + sub of load r, 16-byte part of its chunk
+  typedef double pair_t __attribute__((ext_vector_type(2)));
+  const char* src[4];
+  pair_t pre[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int j = RL * r + sub;
+    src[r] = (const char*)(G0 + (size_t)run_panel[j < nrun ? j : 0] * gstride) + 16 * (part & 3);
+  }
+  auto fetch = [&](int k0) {
+    const unsigned e = 64 * min(k0 + (part >> 2), n - 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (RL * r < nrun) pre[r] = *(const pair_t*)(src[r] + e);
+  };
+  auto put = [&](int w) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (RL * r < nrun) *(pair_t*)(buf[w] + (RL * r + sub) * STR + 2 * part) = pre[r];
+    wave_fence();
+  };
+  auto step = [&](int w, int j, int i, bool use) {
+    double bq[NT + NU], s, d;
+    direct_row<NT, NU>(B, i, m, bq);
+    const double2* g2 = (const double2*)(buf[w] + run * STR + 8 * (4 * j + kq));
+    direct_entry(g2[0], g2[1], g2[2], g2[3].x, use, x0, x1, x2, s, d);
+    acc.add(s, d, bq);
+  };
+  fetch(0);
+  put(0);
+  int k0 = 0, w = 0;
+  for (; k0 + C <= n; k0 += C, w ^= 1) {  // whole chunks: no node past the end
+    fetch(k0 + C);
+#pragma unroll
+    for (int j = 0; j < C / 4; ++j) step(w, j, k0 + 4 * j + kq, live);
+    put(w ^ 1);
+  }
+#pragma unroll 1
+  for (int j = 0; k0 + 4 * j < n; ++j) {
+    const int i = k0 + 4 * j + kq;
+    step(w, j, min(i, n - 1), live && i < n);
   }
 }
 
-template <int NT>
+template <int NT, int NU>
 __global__ void __launch_bounds__(64) direct_mfma_kernel(LevelArgs A, const int* __restrict__ lpairs,
                                                          const int* __restrict__ ltot,
                                                          const int* __restrict__ ppanel,
@@ -450,84 +583,78 @@ __global__ void __launch_bounds__(64) direct_mfma_kernel(LevelArgs A, const int*
                                                          const double* __restrict__ tx,
                                                          const double* __restrict__ lgeo,
                                                          double* __restrict__ wout, int lo, int hi) {
+  __shared__ __align__(16) double buf[2][kDBuf];
+  __shared__ int run_panel[16];
   int b = blockIdx.x, l = -1;
-  int start[4];
-  {
-    int s = 0;
-    for (int q = 0; q < 4; ++q) { start[q] = s; s += ltot[q]; }
-  }
   for (int q = hi; q >= lo; --q) {
     const int ntile = (ltot[q] + 15) >> 4;
     if (b < ntile) { l = q; break; }
     b -= ntile;
   }
   if (l < 0) return;
-  const int h = A.h, ntot = A.ntot, pad = A.pad;
-  const int first = start[l] + 16 * b;
+  int first = 16 * b;
+  for (int q = 0; q < l; ++q) first += ltot[q];
   const int cnt = min(16, ltot[l] - 16 * b);
   const int lane = threadIdx.x, m = lane & 15, kq = lane >> 4;
   const bool live = m < cnt;
-  const int pair = live ? lpairs[first + m] : 0;
-  double x0 = 0.0, x1 = 0.0, x2 = 0.0;
-  const double* G = lgeo;
-  if (live) {
-    const size_t t = (size_t)tidx[pair];
-    x0 = tx[3 * t]; x1 = tx[3 * t + 1]; x2 = tx[3 * t + 2];
-    G = lgeo + 8 * ((size_t)ppanel[pair] * ntot + A.lev_off[l]);
-  }
+  const int pair = lpairs[first + min(m, cnt - 1)];
+  const size_t t = (size_t)tidx[pair];
+  const double x0 = tx[3 * t], x1 = tx[3 * t + 1], x2 = tx[3 * t + 2];
+  const int panel = ppanel[pair];
   const int n = A.lev_n[l];
-  const double* B = A.imp + (size_t)pad * A.lev_off[l];
-  const double c4 = 1.0 / (16.0 * atan(1.0));
-  qd4 accS[NT], accD[NT];
-#pragma unroll
-  for (int q = 0; q < NT; ++q) {
-    accS[q] = qd4{0.0, 0.0, 0.0, 0.0};
-    accD[q] = qd4{0.0, 0.0, 0.0, 0.0};
-  }
-  // branch-free body (clamped indices, selects) so the accumulators stay put
-  for (int k0 = 0; k0 < n; k0 += 4) {
-    const int i = k0 + kq;
-    const bool in = i < n;
-    direct_step<NT>(G, B, pad, m, in ? i : n - 1, live && in, x0, x1, x2, c4, accS, accD);
-  }
-  // v_mfma_f64_16x16x4 operands and result: lane l supplies A[l%16][l/16] and
-  // B[l/16][l%16] and holds D[4r + l/16][l%16] in slot r, so this lane has
-  // pairs 4r + kq of output column 16q + m
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = 4 * r + kq;
-    const int pr = __shfl(pair, row, 64);
-    if (row < cnt) {
-      double* o = wout + (size_t)pr * 2 * h;
-#pragma unroll
-      for (int q = 0; q < NT; ++q) {
-        const int col = 16 * q + m;
-        if (col < h) {
-          o[col] = accS[q][r];
-          o[h + col] = accD[q][r];
-        }
-      }
-    }
-  }
+  const double* B = A.imp + (size_t)A.pad * A.lev_off[l];
+  const double* G0 = lgeo + 8 * (size_t)A.lev_off[l];  // panel 0's first node of the level
+  const size_t gstride = 8 * (size_t)A.ntot;
+  DirectAcc<NT, NU> acc;
+  acc.zero();
+  // runs of equal panels: lane m starts one where its panel differs from lane m-1's
+  const int before = __shfl(panel, m > 0 ? m - 1 : 0, 64);
+  const unsigned starts = (unsigned)__ballot(panel != before) & 0xffffu;
+  const int nrun = 1 + __popc(starts), run = __popc(starts & ((2u << m) - 1u));
+  if (lane < 16 && (m == 0 || (starts >> m & 1u))) run_panel[run] = panel;
+  wave_fence();
+  if (nrun <= 4) direct_staged<16>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
+  else if (nrun <= 8) direct_staged<8>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
+  else direct_staged<4>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
+  acc.store(1.0 / (16.0 * atan(1.0)), A.h, pair, cnt, wout);
 }
+
+// the template of h columns: whole tiles of 16, then the rest in units of 4, or as
+// one more tile when it takes four units (the same matrix-core time, one load)
+#define QOL_DIRECT_COLUMNS(H, CALL)                                                         \
+  switch (((H) % 16 > 12 || (H) % 16 == 0) ? 4 * (((H) + 15) / 16) : 4 * ((H) / 16) + ((H) % 16 + 3) / 4) { \
+    case 1: CALL(0, 1); break;                                                              \
+    case 2: CALL(0, 2); break;                                                              \
+    case 3: CALL(0, 3); break;                                                              \
+    case 4: CALL(1, 0); break;                                                              \
+    case 5: CALL(1, 1); break;                                                              \
+    case 6: CALL(1, 2); break;                                                              \
+    case 7: CALL(1, 3); break;                                                              \
+    case 8: CALL(2, 0); break;                                                              \
+    case 9: CALL(2, 1); break;                                                              \
+    case 10: CALL(2, 2); break;                                                             \
+    case 11: CALL(2, 3); break;                                                             \
+    case 12: CALL(3, 0); break;                                                             \
+    case 14: CALL(3, 2); break;                                                             \
+    case 17: CALL(4, 1); break;                                                             \
+    case 20: CALL(5, 0); break;                                                             \
+    case 23: CALL(5, 3); break;                                                             \
+    case 27: CALL(6, 3); break;                                                             \
+    case 30: CALL(7, 2); break;                                                             \
+    case 34: CALL(8, 2); break;                                                             \
+    default: throw std::runtime_error("direct level kernel: unsupported patch order");      \
+  }
 
 void launch_direct_mfma(LevelArgs A, const int* lpairs, const int* ltot, const int* ppanel, const int* tidx,
                         const double* tx, const double* lgeo, double* wout, int64_t nnz, hipStream_t s, int lo,
                         int hi) {
   if (lo > hi) return;
   const int grid = (int)((nnz + 15) / 16) + 4;
-  switch ((A.h + 15) / 16) {
-    case 1: hipLaunchKernelGGL(direct_mfma_kernel<1>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 2: hipLaunchKernelGGL(direct_mfma_kernel<2>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 3: hipLaunchKernelGGL(direct_mfma_kernel<3>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 4: hipLaunchKernelGGL(direct_mfma_kernel<4>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 5: hipLaunchKernelGGL(direct_mfma_kernel<5>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 6: hipLaunchKernelGGL(direct_mfma_kernel<6>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 7: hipLaunchKernelGGL(direct_mfma_kernel<7>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 8: hipLaunchKernelGGL(direct_mfma_kernel<8>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    case 9: hipLaunchKernelGGL(direct_mfma_kernel<9>, dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, lgeo, wout, lo, hi); break;
-    default: throw std::runtime_error("direct level kernel: unsupported patch order");
-  }
+#define QOL_DIRECT(NT_, NU_)                                                                                   \
+  hipLaunchKernelGGL((direct_mfma_kernel<NT_, NU_>), dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, \
+                     lgeo, wout, lo, hi)
+  QOL_DIRECT_COLUMNS(A.h, QOL_DIRECT)
+#undef QOL_DIRECT
 }
 
 // ---------------------------------------------------------------------------
@@ -612,7 +739,7 @@ __global__ void __launch_bounds__(256) abucket_scatter_kernel(const int* __restr
 
 // one wave per 16 pairs of one cut: direct_mfma_kernel's step over the cut's
 // leaf cells (n1 nodes each) instead of one level's nodes
-template <int NT>
+template <int NT, int NU>
 __global__ void __launch_bounds__(64) direct_adaptive_kernel(LevelArgs A, const int* __restrict__ acnt,
                                                              const int* __restrict__ apairs,
                                                              const int* __restrict__ ppanel,
@@ -627,7 +754,7 @@ __global__ void __launch_bounds__(64) direct_adaptive_kernel(LevelArgs A, const 
     b -= ntile;
   }
   if (bk < 0) return;
-  const int h = A.h, n1 = A.n1, pad = A.pad;
+  const int h = A.h, n1 = A.n1;
   const int first = acnt[kAdaptBuckets + bk] + 16 * b;
   const int cnt = min(16, acnt[bk] - 16 * b);
   const int lane = threadIdx.x, m = lane & 15, kq = lane >> 4;
@@ -642,37 +769,20 @@ __global__ void __launch_bounds__(64) direct_adaptive_kernel(LevelArgs A, const 
   }
   const int* sg = A.aseg + bk * (kAdaptSegs + 1);
   const int nseg = sg[0];
-  const double c4 = 1.0 / (16.0 * atan(1.0));
-  qd4 accS[NT], accD[NT];
-#pragma unroll
-  for (int q = 0; q < NT; ++q) {
-    accS[q] = qd4{0.0, 0.0, 0.0, 0.0};
-    accD[q] = qd4{0.0, 0.0, 0.0, 0.0};
-  }
+  DirectAcc<NT, NU> acc;
+  acc.zero();
   for (int c = 0; c < nseg; ++c) {
     const int o = sg[1 + c];
     for (int k0 = 0; k0 < n1; k0 += 4) {
-      const int i = k0 + kq;
-      const bool in = i < n1;
-      direct_step<NT>(G, A.imp, pad, m, o + (in ? i : n1 - 1), live && in, x0, x1, x2, c4, accS, accD);
+      const int i = k0 + kq, ic = o + min(i, n1 - 1);
+      double bq[NT + NU], s, d;
+      direct_row<NT, NU>(A.imp, ic, m, bq);
+      const double2* g2 = (const double2*)(G + 8 * ic);
+      direct_entry(g2[0], g2[1], g2[2], g2[3].x, live && i < n1, x0, x1, x2, s, d);
+      acc.add(s, d, bq);
     }
   }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = 4 * r + kq;
-    const int pr = __shfl(pair, row, 64);
-    if (row < cnt) {
-      double* o = wout + (size_t)pr * 2 * h;
-#pragma unroll
-      for (int q = 0; q < NT; ++q) {
-        const int col = 16 * q + m;
-        if (col < h) {
-          o[col] = accS[q][r];
-          o[h + col] = accD[q][r];
-        }
-      }
-    }
-  }
+  acc.store(1.0 / (16.0 * atan(1.0)), h, pair, cnt, wout);
 }
 
 void launch_direct_adaptive(LevelArgs A, const int* ltot, const int* lpairs, const int8_t* abucket, int* acnt,
@@ -686,16 +796,10 @@ void launch_direct_adaptive(LevelArgs A, const int* ltot, const int* lpairs, con
   hipLaunchKernelGGL(abucket_offsets_kernel, dim3(1), dim3(64), 0, s, acnt);
   hipLaunchKernelGGL(abucket_scatter_kernel, gs, blk, 0, s, ltot, lpairs, abucket, acnt, apairs);
   const int grid = (int)((nnz + 15) / 16) + kAdaptBuckets;
-#define QOL_ADAPT(NT_)                                                                                       \
-  case NT_:                                                                                                  \
-    hipLaunchKernelGGL(direct_adaptive_kernel<NT_>, dim3(grid), dim3(64), 0, s, A, (const int*)acnt,         \
-                       (const int*)apairs, ppanel, tidx, tx, lgeo, wout);                                    \
-    break;
-  switch ((A.h + 15) / 16) {
-    QOL_ADAPT(1) QOL_ADAPT(2) QOL_ADAPT(3) QOL_ADAPT(4) QOL_ADAPT(5) QOL_ADAPT(6) QOL_ADAPT(7) QOL_ADAPT(8)
-    QOL_ADAPT(9)
-    default: throw std::runtime_error("adaptive direct kernel: unsupported patch order");
-  }
+#define QOL_ADAPT(NT_, NU_)                                                                                      \
+  hipLaunchKernelGGL((direct_adaptive_kernel<NT_, NU_>), dim3(grid), dim3(64), 0, s, A, (const int*)acnt,        \
+                     (const int*)apairs, ppanel, tidx, tx, lgeo, wout)
+  QOL_DIRECT_COLUMNS(A.h, QOL_ADAPT)
 #undef QOL_ADAPT
 }
 
