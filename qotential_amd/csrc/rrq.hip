@@ -8,6 +8,8 @@
 //            (SSQ weights, solid angle, omega moments: absent LQ/QA modules,
 //             re-derived -- see the oracle header for the identities used)
 // FP64 throughout.
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <stdexcept>
 
@@ -1705,26 +1707,35 @@ __device__ void ssq_w1(const double* cf, const double* tgl, const double* wgl, c
   }
 }
 
-// Dirac-string line integral of one edge, adaptive march toward the near point
-template <int NQ>
+// Dirac-string line integral of one edge, adaptive march toward the near point.
+// The march takes the largest interval [lo, hi], halving from twice the last one,
+// whose Bernstein ellipse of parameter thr leaves the root s0 outside: with foci lo
+// and hi that is |s0 - lo| + |s0 - hi| >= (thr + 1/thr) (hi - lo)/2, two square
+// roots (hardware estimates do: which of two equally good intervals is taken when
+// they tie changes the sum by the rule's own 1e-15) where the parameter itself
+// takes a complex division, two complex square roots and three hypots.
+// LW lanes share an item: lane i of them takes node i of every interval (LW = 1:
+// all nodes); the caller adds the lanes' sums.
+template <int NQ, int LW>
 __device__ double solid_angle_edge(const double* cf, const double* tgl, const double* wgl, const double* x,
-                                   const double* q, cd s0, bool ok, double rho_thr) {
+                                   const double* q, cd s0, bool ok, double ell, int i0) {
   double total = 0.0, lo = -1.0, len = 2.0;
   int guard = 0;
+  const double im2 = s0.im * s0.im;
   while (lo < 1.0 && guard < 512) {
     ++guard;
     double hi = fmin(1.0, lo + len);
     if (ok) {
+      const double dl = __builtin_amdgcn_sqrt(fma(s0.re - lo, s0.re - lo, im2));
       while (hi - lo > 1e-14) {
-        const double c = 0.5 * (lo + hi), hh = 0.5 * (hi - lo);
-        const cd t0 = cdiv(csub(s0, cmk(c, 0.0)), cmk(hh, 0.0));
-        if (bernstein_rho(t0) >= rho_thr) break;
+        const double dh = __builtin_amdgcn_sqrt(fma(s0.re - hi, s0.re - hi, im2));
+        if (dl + dh >= ell * (hi - lo)) break;
         hi = lo + 0.5 * (hi - lo);
       }
     }
     const double c = 0.5 * (lo + hi), hh = 0.5 * (hi - lo);
 #pragma unroll 2
-    for (int i = 0; i < NQ; ++i) {
+    for (int i = i0; i < NQ; i += LW) {
       const double s = c + hh * tgl[i];
       double X[3], dX[3];
       pow3_r<NQ>(cf, s, X, dX);
@@ -2057,16 +2068,34 @@ __global__ void __launch_bounds__(256) rrq_root_kernel(RRQTables T, RRQPanels P,
   o[0] = s0.re; o[1] = s0.im; o[2] = ok ? 1.0 : 0.0;
 }
 
-// per (pair, edge): the edge's Dirac-string line integral of the solid angle -> oe[r][3]
+// per (pair, edge): the edge's Dirac-string line integral of the solid angle -> oe[r][3].
+// One thread an item when the items fill the chip (their march is up to 50 intervals,
+// and the sort makes a wave's lengths alike); below that 8 or 16 lanes an item, one
+// per node, since then one march's latency is all that counts.  The line: 98,000
+// and 291,000 items at order 6 take 141 and 194 us with one thread and 50 and 147
+// with 8 lanes; 145,000 at order 12 take 146 and 148 with 16 lanes (of which 14
+// work), 240,000 at order 8 (10 work) 152 and 296.  With the parameter test in
+// solid_angle_edge and one thread an item these took 239, 319, 189 and 229 us, the
+// 60 items of one panel 148 (now 31), the 960,000 of the 48 x 120 order-8 workload
+// 480 (now 325, bound by the vector rate).
+template <int NQ>
+constexpr int solid_lanes() { return NQ <= 8 ? 8 : 16; }
+template <int NQ>
+constexpr int solid_wide() { return NQ <= 8 ? 393216 : 131072; }
+
 template <int NQ>
 __global__ void __launch_bounds__(256) rrq_solid_kernel(RRQTables T, RRQPanels P, const int* __restrict__ lpairs,
                                                         const int* __restrict__ ltot, const int* __restrict__ ppanel,
                                                         const int* __restrict__ tidx, const double* __restrict__ tx,
                                                         const double* __restrict__ pq, const double* __restrict__ root,
-                                                        const int* __restrict__ perm, double* __restrict__ oe) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= 3 * ltot[4]) return;
-  const int it = perm[gid];  // items in order of their cost bucket
+                                                        const int* __restrict__ perm, double ell,
+                                                        double* __restrict__ oe) {
+  constexpr int LW = solid_lanes<NQ>();
+  const int gid = blockIdx.x * blockDim.x + threadIdx.x, n = 3 * ltot[4];
+  const bool wide = n <= solid_wide<NQ>();
+  const int item = wide ? gid / LW : gid;
+  if (item >= n) return;
+  const int it = perm[item];  // items in order of their cost bucket
   const int r = it / 3, e = it % 3;
   const int pair = lpairs[rrq_list_base(ltot) + r];
   const int k = ppanel[pair];
@@ -2076,10 +2105,18 @@ __global__ void __launch_bounds__(256) rrq_solid_kernel(RRQTables T, RRQPanels P
   double X[3];
   to_frame(fr, x, X);
   const double* cf = P.edge + (size_t)k * 9 * NQ + e * 3 * NQ;
-  const double rho_thr = pow(8.0, 8.0 / (double)NQ);
   const double* rt = root + 3 * (size_t)it;
   const double q[3] = {pq[4 * (size_t)r], pq[4 * (size_t)r + 1], pq[4 * (size_t)r + 2]};
-  oe[it] = solid_angle_edge<NQ>(cf, T.tgl, T.wgl, X, q, cmk(rt[0], rt[1]), rt[2] != 0.0, rho_thr);
+  const cd s0 = cmk(rt[0], rt[1]);
+  const bool ok = rt[2] != 0.0;
+  if (wide) {
+    double v = solid_angle_edge<NQ, LW>(cf, T.tgl, T.wgl, X, q, s0, ok, ell, gid % LW);
+#pragma unroll
+    for (int o = LW / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (gid % LW == 0) oe[it] = v;
+  } else {
+    oe[it] = solid_angle_edge<NQ, 1>(cf, T.tgl, T.wgl, X, q, s0, ok, ell, 0);
+  }
 }
 
 // The solid-angle march of a (pair, edge) item takes about 2 log2(1/d) intervals,
@@ -2167,6 +2204,7 @@ void launch_rrq_edge(RRQTables T, RRQPanels P, const int* lpairs, const int* lto
   int* cnt = order;                  // [2 kSB]: counts, then bucket starts
   int* key = order + 2 * kSB;        // [3 nnz]
   int* perm = key + 3 * nnz;         // [3 nnz]
+  const double thr = std::pow(8.0, 8.0 / (double)T.nq), ell = 0.5 * (thr + 1.0 / thr);
 #define QOL_EDGE(NQ_)                                                                                      \
   case NQ_:                                                                                                \
     hipLaunchKernelGGL(rrq_root_kernel<NQ_>, grid, blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, w1, root); \
@@ -2175,8 +2213,9 @@ void launch_rrq_edge(RRQTables T, RRQPanels P, const int* lpairs, const int* lto
     hipLaunchKernelGGL(solid_count_kernel, gsort, blk, 0, s, ltot, (const double*)root, cnt, key);        \
     hipLaunchKernelGGL(solid_offsets_kernel, dim3(1), dim3(64), 0, s, cnt);                               \
     hipLaunchKernelGGL(solid_scatter_kernel, gsort, blk, 0, s, ltot, (const int*)key, cnt, perm);         \
-    hipLaunchKernelGGL(rrq_solid_kernel<NQ_>, grid, blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, pq, root,  \
-                       (const int*)perm, oe);                                                             \
+    hipLaunchKernelGGL(rrq_solid_kernel<NQ_>,                                                              \
+                       dim3((unsigned)((std::max(3 * nnz, std::min<int64_t>(3 * nnz, solid_wide<NQ_>()) * solid_lanes<NQ_>()) + 255) / 256)), \
+                       blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, pq, root, (const int*)perm, ell, oe); \
     break;
   switch (T.nq) {
     QOL_EDGE(4) QOL_EDGE(5) QOL_EDGE(6) QOL_EDGE(7) QOL_EDGE(8) QOL_EDGE(9) QOL_EDGE(10) QOL_EDGE(11)
