@@ -5,6 +5,7 @@
 // Reference: build_patch_levels_r64   patch_refine_mod.f90:423-502
 //            lap3dsdlpmat_levels_r64  patch_refine_mod.f90:516-615
 //            lap3dsdlpmat_r64 (direct kernel; zero at coincident points)
+#include <algorithm>
 #include <stdexcept>
 #include <vector>
 
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(256) level_geom_kernel(LevelArgs A, int npan, 
   const int np_ = min(kLP, npan - k0);
   const size_t nt_ = A.ntot;
   double* cn = smem;  // [kLP][kCP]: x, y, z, w of the chunk's nodes (4 x kChunk) and padding
-  for (int ch = 0; ch < A.nchunk; ++ch) {
+  for (int ch = blockIdx.y; ch < A.nchunk; ch += gridDim.y) {
     const int* C = A.chunks + 5 * ch;
     const int l = C[0], c0 = C[1], c1 = C[2], sb0 = C[3], sb1 = C[4];
     const int n = A.lev_n[l], off = A.lev_off[l];
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(256) level_geom_mfma_kernel(LevelArgs A, int n
       }
       bf[s][t] = v;
     }
-  for (int ch = 0; ch < A.nchunk; ++ch) {
+  for (int ch = blockIdx.y; ch < A.nchunk; ch += gridDim.y) {
     const int* C = A.chunks + 5 * ch;
     const int l = C[0], c0 = C[1], c1 = C[2], sb0 = C[3], sb1 = C[4];
     const int off = A.lev_off[l];
@@ -306,7 +307,10 @@ __global__ void __launch_bounds__(256) level_geom_mfma_kernel(LevelArgs A, int n
 void launch_level_geom(const LevelArgs& A, int npan, const double* sx, const double* rts, const double* rps,
                        double* lgeo, double* balls, hipStream_t s) {
   const int ks = (A.h + 3) / 4;
-  const dim3 grid(level_geom_blocks(npan)), blk(256);
+  // few panels: a panel group's chunks are dealt to several workgroups, about 1,024
+  // in all (one panel took 44 and 97 us at orders 4 and 6 on one workgroup, now 9 and 13)
+  const int groups = level_geom_blocks(npan);
+  const dim3 grid(groups, std::max(1, std::min((1024 + groups - 1) / groups, A.nchunk))), blk(256);
   if (ks <= 20 && 4 * ks <= A.pad) {
     const size_t lds = level_geom_mfma_smem();
 #define QOL_LEVEL_MFMA(KS_)                                                                                    \
