@@ -670,10 +670,7 @@ void Engine::eval(int exterior, double side_tol, bool want_omega) {
                      (const double*)d_sx.ptr, (const double*)d_snx.ptr, (const double*)d_sw.ptr, ichart,
                      (const double*)d_sxbd.ptr, (const double*)d_rv.ptr);
   HIPCHK(hipEventRecord(ev_setup, s2));
-  const size_t lds2 = rrq_system_smem(h, nq, ncoef);
-  set_lds((const void*)rrq_panel_system_kernel, lds2);
-  hipLaunchKernelGGL(rrq_panel_system_kernel, dim3(npan), dim3(256), lds2, s2, tab->RT, RP, npan, (const int*)nullptr,
-                     (const double*)d_sx.ptr, (const double*)d_snx.ptr);
+  launch_rrq_system(p, RP, npan, (const double*)d_sx.ptr, (const double*)d_snx.ptr, s2);
   rec(3, 1, s2);
   HIPCHK(hipEventRecord(ev_system, s2));
   rec(4, 0, s2);

@@ -176,8 +176,7 @@ __global__ void triplet_kernel(int nnz, int h, const int* tidx, const int* ppane
 __global__ void rrq_panel_frame_kernel(RRQTables T, RRQPanels P, int npan, const int* nrrq, const double* sx,
                                        const double* snx, const double* sw, int ichart, const double* sxbd_chart,
                                        const double* rv_chart);
-__global__ void rrq_panel_system_kernel(RRQTables T, RRQPanels P, int npan, const int* nrrq, const double* sx,
-                                        const double* snx);
+void launch_rrq_system(int p, RRQPanels P, int npan, const double* sx, const double* snx, hipStream_t s);
 // variant 0: register-resident inverses up to order 8 (QOL_SOLVE_FUSED=1 / QOL_SOLVE_MFMA=1
 // select the others), 1: the fused vector-unit elimination, 2: the matrix-core
 // quaternion elimination (orders up to 8; the default above)
@@ -197,7 +196,6 @@ void launch_rrq_target(RRQTables T, RRQPanels P, const int* lpairs, const int* l
 void launch_rrq_weights(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
                         const int* nrrq, const double* vt, double* wout, hipStream_t s);
 size_t rrq_frame_smem(int h, int nq);
-size_t rrq_system_smem(int h, int nq, int ncoef);
 size_t rrq_basis_doubles(int p, int nq);  // RRQPanels::basis, per panel
 
 }  // namespace qol

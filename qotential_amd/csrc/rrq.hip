@@ -113,28 +113,6 @@ __device__ __forceinline__ void rotate(const double* fr, const double* v, double
   for (int r = 0; r < 3; ++r) V[r] = fr[3 * r] * v[0] + fr[3 * r + 1] * v[1] + fr[3 * r + 2] * v[2];
 }
 
-// harmonic values H'_n^m (m=0..n, n=0..p) at frame point X into H (ncoef complex)
-__device__ void harm_vals(const double* X, int p, cd* H) {
-  const cd W = cmk(X[1], X[2]);
-  const double Z = X[0];
-  H[0] = cmk(1.0, 0.0);
-  for (int n = 1; n <= p; ++n)
-    for (int m = 0; m <= n; ++m) {
-      const cd a = cscale(hget(H, n - 1, m), Z);
-      const cd b = cadd(cmul(W, hget(H, n - 1, m - 1)), cmul(cconj(W), hget(H, n - 1, m + 1)));
-      H[hidx(n, m)] = cadd(a, cscale(cmuli(b), 0.5));
-    }
-}
-
-// gradient of H'_n^m (frame x,y,z) from degree n-1 values
-__device__ __forceinline__ void harm_grad(const cd* H, int n, int m, cd* g) {
-  const double dn = (double)n;
-  const cd lo = hget(H, n - 1, m - 1), hi = hget(H, n - 1, m + 1);
-  g[0] = cscale(hget(H, n - 1, m), dn);
-  g[1] = cscale(cmuli(cadd(lo, hi)), 0.5 * dn);
-  g[2] = cscale(csub(hi, lo), 0.5 * dn);
-}
-
 // Im((-i)^m z)
 __device__ __forceinline__ double imrot(int m, cd z) {
   switch (m & 3) {
@@ -152,15 +130,8 @@ size_t rrq_frame_smem(int h, int nq) {
 }
 // complex values per boundary node in P.basis: H'_n^m (n < p, 0 <= m <= n), then
 // T_n^m (n < p - 1, 0 <= m <= n + 1)
-__host__ __device__ inline int rrq_basis_cols(int p) { return p * (p + 1) / 2 + (p - 1) * (p + 2) / 2; }
-size_t rrq_basis_doubles(int p, int nq) { return (size_t)2 * 3 * nq * rrq_basis_cols(p); }
-
-size_t rrq_system_smem(int h, int nq, int ncoef) {
-  const int nb = 3 * nq;
-  size_t a = (size_t)(6 * h + 16 + 6 * nb) * sizeof(double);
-  size_t b = (size_t)nb * ncoef * sizeof(cd);
-  size_t c = (size_t)64 * ncoef * sizeof(cd);
-  return a + (b > c ? b : c);
+size_t rrq_basis_doubles(int p, int nq) {
+  return (size_t)2 * 3 * nq * (p * (p + 1) / 2 + (p - 1) * (p + 2) / 2);
 }
 
 // One workgroup per panel (with RRQ pairs, or every panel when nrrq is null):
@@ -316,98 +287,121 @@ __global__ void __launch_bounds__(256) rrq_panel_frame_kernel(RRQTables T, RRQPa
   __syncthreads();
 }
 
-// One workgroup per panel: harmonic values at the boundary nodes, and the quaternion
-// matrix, Msl^T and Fn at the panel nodes, from the frame and boundary nodes
-// written by rrq_panel_frame_kernel.
-__global__ void __launch_bounds__(256) rrq_panel_system_kernel(RRQTables T, RRQPanels P, int npan,
-                                                               const int* __restrict__ nrrq,
-                                                               const double* __restrict__ sx,
-                                                               const double* __restrict__ snx) {
-  const int k = blockIdx.x;
-  if (nrrq && nrrq[k] == 0) return;  // null: every panel
-  extern __shared__ double sm[];
-  const int h = T.h, nq = T.nq, p = T.p, nb = 3 * nq, ncoef = T.ncoef;
-  double* ssx = sm;             // [3][h]
-  double* ssn = ssx + 3 * h;    // [3][h]
-  double* fr = ssn + 3 * h;     // 16
-  double* bx = fr + 16;         // [nb][6]
-  cd* Hs = (cd*)(bx + 6 * nb);  // [nb or 64][ncoef]
-  const size_t gk = (size_t)k * h;
-  for (int i = threadIdx.x; i < h; i += blockDim.x)
-    for (int c = 0; c < 3; ++c) {
-      ssx[c * h + i] = sx[3 * (gk + i) + c];
-      ssn[c * h + i] = snx[3 * (gk + i) + c];
-    }
-  for (int i = threadIdx.x; i < 16; i += blockDim.x) fr[i] = P.frame[(size_t)k * 16 + i];
-  for (int i = threadIdx.x; i < 6 * nb; i += blockDim.x) bx[i] = P.bX[(size_t)k * nb * 6 + i];
-  __syncthreads();
-  // harmonic values H'_n^m of degree n < p at the boundary nodes, and for n < p - 1
-  // their combinations T_n^m with the edge tangent: the moments of every pair are
-  // contracted against these (their gradients are fixed combinations, applied
-  // after the contraction)
-  for (int ib = threadIdx.x; ib < nb; ib += blockDim.x) harm_vals(bx + 6 * ib, p, Hs + (size_t)ib * ncoef);
-  __syncthreads();
-  const int nc1 = p * (p + 1) / 2, ncb = rrq_basis_cols(p);
-  cd* Ho = (cd*)P.basis + (size_t)k * nb * ncb;
-  for (int it = threadIdx.x; it < nb * ncb; it += blockDim.x) {
-    const int ib = it / ncb, kk = it % ncb;
-    const cd* H = Hs + (size_t)ib * ncoef;
-    if (kk < nc1) {
-      Ho[it] = H[kk];
-    } else {
-      // T_n^m = dX_Z H'_n^m + i/2 (dW H'_n^{m-1} + conj(dW) H'_n^{m+1}), m = 0..n+1
-      const int j = kk - nc1;
-      int n = 0;
-      while ((n + 1) * (n + 4) / 2 <= j) ++n;
-      const int m = j - n * (n + 3) / 2;
-      const double* d = bx + 6 * ib + 3;
-      const cd dw = cmk(d[1], d[2]);
-      Ho[it] = cadd(cscale(hget(H, n, m), d[0]),
-                    cscale(cmuli(cadd(cmul(dw, hget(H, n, m - 1)), cmul(cconj(dw), hget(H, n, m + 1)))), 0.5));
-    }
-  }
-  __syncthreads();
-  // quaternion system at the nodes.  F_k = Im((-i)^m H'_n^m), n=1..p, m=1..n.
-  // Fq(i,k) = grad F_k(y_i) as a pure quaternion; the real 4h x 4h matrix of the
-  // reference (Mmatrix with its first two diagonal blocks zeroed, rrq_r64:851-858)
-  // is left multiplication by this h x h quaternion matrix.
-  double* FQ = P.Fq + (size_t)k * 3 * h * h;
-  double* MS = P.Msl + (size_t)k * h * h;
-  double* FN = P.Fn + (size_t)k * h * h;
-  // node positions and normals in the frame (in place), then per chunk of nodes:
-  // harmonics at the nodes, and one thread per (node, basis function)
-  for (int i = threadIdx.x; i < h; i += blockDim.x) {
-    const double x[3] = {ssx[i], ssx[h + i], ssx[2 * h + i]}, nn0[3] = {ssn[i], ssn[h + i], ssn[2 * h + i]};
-    double X[3], N[3];
+// Harmonics at a panel's boundary nodes (and their combinations with the edge
+// tangent), and the quaternion matrix, Msl^T and Fn at its nodes, from the frame and
+// boundary nodes written by rrq_panel_frame_kernel.
+//
+// One thread per node, panel nodes first, then (from the next wave on where that
+// separates them) the boundary nodes: each keeps the previous degree's harmonics in
+// registers.  Bound by its stores (1.24 GB for the 14,250 order-8 panels of the 48 x
+// 120 workload): 0.31 ms; with the harmonics' degrees handed on through LDS, one
+// thread a node and then one a matrix entry, it took 0.60 (0.48 before it also
+// wrote the tangent combinations), without the gathering below 0.54.  1,580 panels
+// of order 12: 0.60 -> 0.25.
+template <int P>
+struct SystemPlan {
+  static constexpr int H = P * (P + 1) / 2, NB = 3 * (P + 2);
+  static constexpr int B0 = H + NB <= 64 ? H : (H > 64 ? H : 64);  // first thread of the boundary nodes
+  static constexpr int N = (B0 + NB + 63) / 64 * 64;
+  // up to order 8 a panel's Fq and Msl^T (41 KB) are gathered in LDS and written in
+  // order; rows of an odd number of doubles, so the nodes' lanes fall in different banks
+  static constexpr bool GATHER = P <= 8;
+  static constexpr int RF = 3 * H + 1 - (3 * H) % 2, RM = H + 1 - H % 2;
+};
+
+template <int P>
+__global__ void __launch_bounds__(SystemPlan<P>::N) rrq_panel_system_kernel(RRQPanels pan, const double* __restrict__ sx,
+                                                                            const double* __restrict__ snx) {
+  using S = SystemPlan<P>;
+  constexpr int H = S::H, NB = S::NB, NC1 = P * (P + 1) / 2, NCB = NC1 + (P - 1) * (P + 2) / 2;
+  __shared__ double gq[S::GATHER ? H * S::RF : 1], gm[S::GATHER ? H * S::RM : 1];
+  const int k = blockIdx.x, i = threadIdx.x;
+  const bool node = i < H, bnd = i >= S::B0 && i < S::B0 + NB;
+  const double* fr = pan.frame + (size_t)k * 16;
+  double X[3] = {0.0, 0.0, 0.0}, N[3] = {0.0, 0.0, 0.0};  // position; normal at a panel node, tangent at a boundary node
+  if (node) {
+    const size_t g = (size_t)k * H + i;
+    const double x[3] = {sx[3 * g], sx[3 * g + 1], sx[3 * g + 2]};
+    const double n0[3] = {snx[3 * g], snx[3 * g + 1], snx[3 * g + 2]};
     to_frame(fr, x, X);
-    rotate(fr, nn0, N);
-    for (int c = 0; c < 3; ++c) { ssx[c * h + i] = X[c]; ssn[c * h + i] = N[c]; }
+    rotate(fr, n0, N);
+  } else if (bnd) {
+    const double* bx = pan.bX + ((size_t)k * NB + i - S::B0) * 6;
+    for (int c = 0; c < 3; ++c) {
+      X[c] = bx[c];
+      N[c] = bx[3 + c];
+    }
   }
-  __syncthreads();
-  const int chunk = nb > 64 ? nb : 64;
-  for (int i0 = 0; i0 < h; i0 += chunk) {
-    const int ni = min(chunk, h - i0);
-    for (int t = threadIdx.x; t < ni; t += blockDim.x) {
-      const double X[3] = {ssx[i0 + t], ssx[h + i0 + t], ssx[2 * h + i0 + t]};
-      harm_vals(X, p, Hs + (size_t)t * ncoef);
+  // Fq(i,k) = grad F_k(y_i) as a pure quaternion, F_k = Im((-i)^m H'_n^m), n = 1..p,
+  // m = 1..n; the real 4h x 4h matrix of the reference (Mmatrix with its first two
+  // diagonal blocks zeroed, rrq_r64:851-858) is left multiplication by this h x h
+  // quaternion matrix
+  double *FQ0 = pan.Fq + (size_t)k * 3 * H * H, *MS0 = pan.Msl + (size_t)k * H * H;
+  double* FQ = S::GATHER ? gq + i * S::RF : FQ0 + (size_t)i * 3 * H;
+  double* MS = S::GATHER ? gm + i * S::RM : MS0 + (size_t)i * H;
+  double* FN = pan.Fn + (size_t)k * H * H + i;
+  cd* Ho = (cd*)pan.basis + ((size_t)k * NB + (i - S::B0)) * NCB;
+  cd* To = Ho + NC1;
+  const cd W = cmk(X[1], X[2]), dw = cmk(N[1], N[2]);
+  cd E[P + 2];  // H'_{n-1}^m, zero past m = n - 1
+#pragma unroll
+  for (int m = 0; m < P + 2; ++m) E[m] = cmk(0.0, 0.0);
+  E[0] = cmk(1.0, 0.0);
+  int kk = 0, ih = 0, jt = 0;
+#pragma unroll 1
+  for (int n = 1; n <= P; ++n) {
+    if (bnd) {
+      // degree n - 1: H' and, below degree p - 1, T_n^m = dX_Z H'_n^m + i/2 (dW
+      // H'_n^{m-1} + conj(dW) H'_n^{m+1})
+      cd lo = cmk(-E[1].re, E[1].im);
+#pragma unroll
+      for (int m = 0; m <= P; ++m) {
+        if (m < n) Ho[ih++] = E[m];
+        if (m <= n && n < P)
+          To[jt++] = cadd(cscale(E[m], N[0]), cscale(cmuli(cadd(cmul(dw, lo), cmul(cconj(dw), E[m + 1]))), 0.5));
+        lo = E[m];
+      }
     }
-    __syncthreads();
-    for (int it = threadIdx.x; it < ni * h; it += blockDim.x) {
-      const int t = it / h, kk = it % h, i = i0 + t;
-      int n = 1;
-      while ((n + 1) * n / 2 <= kk) ++n;
-      const int m = kk - (n - 1) * n / 2 + 1;
-      const cd* H = Hs + (size_t)t * ncoef;
-      cd g[3];
-      harm_grad(H, n, m, g);
-      const double F = imrot(m, H[hidx(n, m)]);
-      const double F1 = imrot(m, g[0]), F2 = imrot(m, g[1]), F3 = imrot(m, g[2]);
-      FN[i + (size_t)h * kk] = F;
-      MS[kk + (size_t)h * i] = ssn[i] * F1 + ssn[h + i] * F2 + ssn[2 * h + i] * F3;
-      double* q = FQ + 3 * ((size_t)i * h + kk);
-      q[0] = F1; q[1] = F2; q[2] = F3;
+    const double dn = (double)n;
+    cd lo = cmk(-E[1].re, E[1].im);
+#pragma unroll
+    for (int m = 0; m <= P; ++m) {
+      if (m <= n) {
+        const cd mid = E[m], hi = E[m + 1];
+        const cd b = cadd(cmul(W, lo), cmul(cconj(W), hi));
+        E[m] = cadd(cscale(mid, X[0]), cscale(cmuli(b), 0.5));
+        if (node && m > 0) {
+          // the gradient from degree n - 1 (harm_grad)
+          const double F1 = imrot(m, cscale(mid, dn)), F2 = imrot(m, cscale(cmuli(cadd(lo, hi)), 0.5 * dn)),
+                       F3 = imrot(m, cscale(csub(hi, lo), 0.5 * dn));
+          FN[(size_t)H * kk] = imrot(m, E[m]);
+          MS[kk] = N[0] * F1 + N[1] * F2 + N[2] * F3;
+          FQ[3 * kk] = F1;
+          FQ[3 * kk + 1] = F2;
+          FQ[3 * kk + 2] = F3;
+          ++kk;
+        }
+        lo = mid;
+      }
     }
+  }
+  if (S::GATHER) {
     __syncthreads();
+    for (int e = i; e < 3 * H * H; e += S::N) FQ0[e] = gq[e / (3 * H) * S::RF + e % (3 * H)];
+    for (int e = i; e < H * H; e += S::N) MS0[e] = gm[e / H * S::RM + e % H];
+  }
+}
+
+void launch_rrq_system(int p, RRQPanels P, int npan, const double* sx, const double* snx, hipStream_t s) {
+  switch (p) {
+#define QOL_SYSTEM(P_)                                                                                                 \
+  case P_:                                                                                                             \
+    hipLaunchKernelGGL(rrq_panel_system_kernel<P_>, dim3(npan), dim3(SystemPlan<P_>::N), 0, s, P, sx, snx);            \
+    break;
+    QOL_SYSTEM(2) QOL_SYSTEM(3) QOL_SYSTEM(4) QOL_SYSTEM(5) QOL_SYSTEM(6) QOL_SYSTEM(7) QOL_SYSTEM(8) QOL_SYSTEM(9)
+    QOL_SYSTEM(10) QOL_SYSTEM(11) QOL_SYSTEM(12)
+#undef QOL_SYSTEM
+    default: throw std::runtime_error("RRQ set-up: patch orders 2..12 only");
   }
 }
 
