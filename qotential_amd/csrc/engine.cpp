@@ -702,8 +702,9 @@ void Engine::eval(int exterior, double side_tol, bool want_omega) {
   HIPCHK(hipEventRecord(ev_edge, s3));
   // s1: direct levels, after the edge chain (projection, roots, solid angle): that
   // chain heads the path the moments wait for, the direct kernel's 121k waves
-  // would crowd it out, and the direct kernel then runs beside the moments
-  HIPCHK(hipStreamWaitEvent(s1, ev_edge, 0));
+  // would crowd it out, and the direct kernel then runs beside the moments.  A list
+  // too short to fill the GPU crowds nothing out: its direct levels start at once
+  HIPCHK(hipStreamWaitEvent(s1, nnz <= 16384 ? ev_lists : ev_edge, 0));
   rec(2, 0, s1);
   direct(s1);
   rec(2, 1, s1);

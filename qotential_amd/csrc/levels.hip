@@ -337,21 +337,13 @@ void launch_level_geom(const LevelArgs& A, int npan, const double* sx, const dou
 // ltot[l] = length of list l.  One block per label.
 __global__ void __launch_bounds__(1024) level_scan_kernel(const int* __restrict__ lcount, int npan,
                                                           int* __restrict__ lstart, int* __restrict__ ltot) {
-  __shared__ int part[1024];
   const int l = blockIdx.x;
   const int per = (npan + blockDim.x - 1) / blockDim.x;
   const int a = threadIdx.x * per, b = min(npan, a + per);
-  int s = 0;
+  int s = 0, total;
   for (int k = a; k < b; ++k) s += lcount[5 * k + l];
-  part[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int i = 0; i < (int)blockDim.x; ++i) { const int v = part[i]; part[i] = acc; acc += v; }
-    ltot[l] = acc;
-  }
-  __syncthreads();
-  int acc = part[threadIdx.x];
+  int acc = block_scan_1024(s, &total);
+  if (threadIdx.x == 0) ltot[l] = total;
   for (int k = a; k < b; ++k) { lstart[(size_t)l * npan + k] = acc; acc += lcount[5 * k + l]; }
 }
 
@@ -439,6 +431,24 @@ struct DirectAcc {
     for (int q = 0; q < NT; ++q) S[q] = D[q] = qd4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int u = 0; u < NU; ++u) Su[u] = Du[u] = 0.0;
+  }
+  template <class F>
+  __device__ __forceinline__ void each(F&& f) {
+#pragma unroll
+    for (int q = 0; q < NT; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double s = S[q][j], d = D[q][j];
+        f(8 * q + j, s);
+        f(8 * q + 4 + j, d);
+        S[q][j] = s;
+        D[q][j] = d;
+      }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      f(8 * NT + 2 * u, Su[u]);
+      f(8 * NT + 2 * u + 1, Du[u]);
+    }
   }
   // bq: this lane's entries of the step's table rows
   __device__ __forceinline__ void add(double s, double d, const double* bq) {
@@ -529,10 +539,11 @@ __device__ __forceinline__ void direct_entry(const double2 ga, const double2 gb,
 // nodes of four 16-byte parts each.  The runs' chunks lie 64 C + 16 bytes apart, so
 // the 16 pairs' records of one node fall in different banks.
 constexpr int kDBuf = 16 * (8 * 4 + 2);  // doubles a buffer takes at most (C = 4: 16 runs)
+constexpr int kDC = 16;                  // the largest chunk
 template <int C, int NT, int NU>
 __device__ __forceinline__ void direct_staged(double (*buf)[kDBuf], const int* run_panel, int nrun, int run,
-                                              const double* G0, size_t gstride, const double* __restrict__ B, int n,
-                                              bool live, double x0, double x1, double x2, DirectAcc<NT, NU>& acc) {
+                                              const double* G0, size_t gstride, const double* __restrict__ B, int n0,
+                                              int n, bool live, double x0, double x1, double x2, DirectAcc<NT, NU>& acc) {
   constexpr int RL = 16 / C, STR = 8 * C + 2;
   const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
   const int sub = lane / (4 * C), part = lane % (4 * C);  // run RL r + sub of load r, 16-byte part of its chunk
@@ -563,9 +574,9 @@ __device__ __forceinline__ void direct_staged(double (*buf)[kDBuf], const int* r
     direct_entry(g2[0], g2[1], g2[2], g2[3].x, use, x0, x1, x2, s, d);
     acc.add(s, d, bq);
   };
-  fetch(0);
+  fetch(n0);
   put(0);
-  int k0 = 0, w = 0;
+  int k0 = n0, w = 0;
   for (; k0 + C <= n; k0 += C, w ^= 1) {  // whole chunks: no node past the end
     fetch(k0 + C);
 #pragma unroll
@@ -579,16 +590,17 @@ __device__ __forceinline__ void direct_staged(double (*buf)[kDBuf], const int* r
   }
 }
 
-template <int NT, int NU>
-__global__ void __launch_bounds__(64) direct_mfma_kernel(LevelArgs A, const int* __restrict__ lpairs,
+template <int NT, int NU, int KS>
+__global__ void __launch_bounds__(64 * KS) direct_mfma_kernel(LevelArgs A, const int* __restrict__ lpairs,
                                                          const int* __restrict__ ltot,
                                                          const int* __restrict__ ppanel,
                                                          const int* __restrict__ tidx,
                                                          const double* __restrict__ tx,
                                                          const double* __restrict__ lgeo,
                                                          double* __restrict__ wout, int lo, int hi) {
-  __shared__ __align__(16) double buf[2][kDBuf];
-  __shared__ int run_panel[16];
+  __shared__ __align__(16) double buf[KS][2][kDBuf];
+  __shared__ int run_panel[KS][16];
+  const int wv = KS > 1 ? threadIdx.x >> 6 : 0;
   int b = blockIdx.x, l = -1;
   for (int q = hi; q >= lo; --q) {
     const int ntile = (ltot[q] + 15) >> 4;
@@ -599,7 +611,7 @@ __global__ void __launch_bounds__(64) direct_mfma_kernel(LevelArgs A, const int*
   int first = 16 * b;
   for (int q = 0; q < l; ++q) first += ltot[q];
   const int cnt = min(16, ltot[l] - 16 * b);
-  const int lane = threadIdx.x, m = lane & 15, kq = lane >> 4;
+  const int lane = threadIdx.x & 63, m = lane & 15;
   const bool live = m < cnt;
   const int pair = lpairs[first + min(m, cnt - 1)];
   const size_t t = (size_t)tidx[pair];
@@ -615,11 +627,27 @@ __global__ void __launch_bounds__(64) direct_mfma_kernel(LevelArgs A, const int*
   const int before = __shfl(panel, m > 0 ? m - 1 : 0, 64);
   const unsigned starts = (unsigned)__ballot(panel != before) & 0xffffu;
   const int nrun = 1 + __popc(starts), run = __popc(starts & ((2u << m) - 1u));
-  if (lane < 16 && (m == 0 || (starts >> m & 1u))) run_panel[run] = panel;
+  int* rp = run_panel[wv];
+  if (lane < 16 && (m == 0 || (starts >> m & 1u))) rp[run] = panel;
   wave_fence();
-  if (nrun <= 4) direct_staged<16>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
-  else if (nrun <= 8) direct_staged<8>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
-  else direct_staged<4>(buf, run_panel, nrun, run, G0, gstride, B, n, live, x0, x1, x2, acc);
+  // this wave's nodes: all, or its share in whole chunks
+  const int per = kDC * ((n + kDC * KS - 1) / (kDC * KS)), n0 = wv * per, n1 = min(n, n0 + per);
+  if (n0 < n1) {
+    if (nrun <= 4) direct_staged<16>(buf[wv], rp, nrun, run, G0, gstride, B, n0, n1, live, x0, x1, x2, acc);
+    else if (nrun <= 8) direct_staged<8>(buf[wv], rp, nrun, run, G0, gstride, B, n0, n1, live, x0, x1, x2, acc);
+    else direct_staged<4>(buf[wv], rp, nrun, run, G0, gstride, B, n0, n1, live, x0, x1, x2, acc);
+  }
+  if constexpr (KS > 1) {  // the waves' sums, in order, into the first's
+    double* sum = &buf[0][0][0];
+    static_assert(64 * (8 * NT + 2 * NU) <= KS * 2 * kDBuf, "one wave's accumulators fit the buffers");
+    for (int w = 1; w < KS; ++w) {
+      __syncthreads();
+      if (wv == w) acc.each([&](int i, double& v) { sum[64 * i + lane] = v; });
+      __syncthreads();
+      if (wv == 0) acc.each([&](int i, double& v) { v += sum[64 * i + lane]; });
+    }
+    if (wv != 0) return;
+  }
   acc.store(1.0 / (16.0 * atan(1.0)), A.h, pair, cnt, wout);
 }
 
@@ -653,10 +681,19 @@ void launch_direct_mfma(LevelArgs A, const int* lpairs, const int* ltot, const i
                         const double* tx, const double* lgeo, double* wout, int64_t nnz, hipStream_t s, int lo,
                         int hi) {
   if (lo > hi) return;
+  // few tiles: four waves share one, each a quarter of the nodes, since a level-4
+  // tile's steps follow one another and its last tiles leave the chip idle: one
+  // panel's 124 targets 33 -> 13 us, 2,500 tiles at order 4 88 -> 31, 12,500 at order
+  // 6 305 -> 196, 7,400 at order 12 620 -> 390; 18,400 at order 12 932 -> 986
   const int grid = (int)((nnz + 15) / 16) + 4;
-#define QOL_DIRECT(NT_, NU_)                                                                                   \
-  hipLaunchKernelGGL((direct_mfma_kernel<NT_, NU_>), dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel, tidx, tx, \
-                     lgeo, wout, lo, hi)
+  const bool split = grid <= 16384;
+#define QOL_DIRECT(NT_, NU_)                                                                                    \
+  if (split)                                                                                                    \
+    hipLaunchKernelGGL((direct_mfma_kernel<NT_, NU_, 4>), dim3(grid), dim3(256), 0, s, A, lpairs, ltot, ppanel, \
+                       tidx, tx, lgeo, wout, lo, hi);                                                           \
+  else                                                                                                          \
+    hipLaunchKernelGGL((direct_mfma_kernel<NT_, NU_, 1>), dim3(grid), dim3(64), 0, s, A, lpairs, ltot, ppanel,  \
+                       tidx, tx, lgeo, wout, lo, hi)
   QOL_DIRECT_COLUMNS(A.h, QOL_DIRECT)
 #undef QOL_DIRECT
 }

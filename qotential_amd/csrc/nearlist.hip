@@ -123,20 +123,12 @@ __global__ void __launch_bounds__(256) nearlist_fill_kernel(int npan, int nt, co
 
 // exclusive scan of n ints into out[0..n] with a single workgroup of 1024 threads
 __global__ void __launch_bounds__(1024) scan_kernel(const int* __restrict__ in, int n, int* __restrict__ out) {
-  __shared__ int part[1024];
   const int per = (n + blockDim.x - 1) / blockDim.x;
   const int a = threadIdx.x * per, b = min(n, a + per);
-  int s = 0;
+  int s = 0, total;
   for (int i = a; i < b; ++i) s += in[i];
-  part[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int i = 0; i < (int)blockDim.x; ++i) { const int v = part[i]; part[i] = acc; acc += v; }
-    out[n] = acc;
-  }
-  __syncthreads();
-  int acc = part[threadIdx.x];
+  int acc = block_scan_1024(s, &total);
+  if (threadIdx.x == 0) out[n] = total;
   for (int i = a; i < b; ++i) { out[i] = acc; acc += in[i]; }
 }
 

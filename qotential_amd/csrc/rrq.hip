@@ -2089,7 +2089,7 @@ __global__ void __launch_bounds__(256) rrq_solid_kernel(RRQTables T, RRQPanels P
   const bool wide = n <= solid_wide<NQ>();
   const int item = wide ? gid / LW : gid;
   if (item >= n) return;
-  const int it = perm[item];  // items in order of their cost bucket
+  const int it = perm ? perm[item] : item;  // items in order of their cost bucket
   const int r = it / 3, e = it % 3;
   const int pair = lpairs[rrq_list_base(ltot) + r];
   const int k = ppanel[pair];
@@ -2198,18 +2198,23 @@ void launch_rrq_edge(RRQTables T, RRQPanels P, const int* lpairs, const int* lto
   int* cnt = order;                  // [2 kSB]: counts, then bucket starts
   int* key = order + 2 * kSB;        // [3 nnz]
   int* perm = key + 3 * nnz;         // [3 nnz]
+  // so few items that all their waves run at once: their order does not matter, and
+  // the sort's four launches (16 us) cost more than it saves
+  const bool sort = 3 * nnz > 16384;
   const double thr = std::pow(8.0, 8.0 / (double)T.nq), ell = 0.5 * (thr + 1.0 / thr);
 #define QOL_EDGE(NQ_)                                                                                      \
   case NQ_:                                                                                                \
     hipLaunchKernelGGL(rrq_root_kernel<NQ_>, grid, blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, w1, root); \
     if (mid) (void)hipEventRecord(mid, s);                                                                 \
-    hipLaunchKernelGGL(zero_ints_kernel, dim3(1), dim3(2 * kSB), 0, s, cnt, 2 * kSB);                      \
-    hipLaunchKernelGGL(solid_count_kernel, gsort, blk, 0, s, ltot, (const double*)root, cnt, key);        \
-    hipLaunchKernelGGL(solid_offsets_kernel, dim3(1), dim3(64), 0, s, cnt);                               \
-    hipLaunchKernelGGL(solid_scatter_kernel, gsort, blk, 0, s, ltot, (const int*)key, cnt, perm);         \
+    if (sort) {                                                                                           \
+      hipLaunchKernelGGL(zero_ints_kernel, dim3(1), dim3(2 * kSB), 0, s, cnt, 2 * kSB);                    \
+      hipLaunchKernelGGL(solid_count_kernel, gsort, blk, 0, s, ltot, (const double*)root, cnt, key);      \
+      hipLaunchKernelGGL(solid_offsets_kernel, dim3(1), dim3(64), 0, s, cnt);                             \
+      hipLaunchKernelGGL(solid_scatter_kernel, gsort, blk, 0, s, ltot, (const int*)key, cnt, perm);       \
+    }                                                                                                     \
     hipLaunchKernelGGL(rrq_solid_kernel<NQ_>,                                                              \
                        dim3((unsigned)((std::max(3 * nnz, std::min<int64_t>(3 * nnz, solid_wide<NQ_>()) * solid_lanes<NQ_>()) + 255) / 256)), \
-                       blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, pq, root, (const int*)perm, ell, oe); \
+                       blk, 0, s, T, P, lpairs, ltot, ppanel, tidx, tx, pq, root, sort ? (const int*)perm : nullptr, ell, oe); \
     break;
   switch (T.nq) {
     QOL_EDGE(4) QOL_EDGE(5) QOL_EDGE(6) QOL_EDGE(7) QOL_EDGE(8) QOL_EDGE(9) QOL_EDGE(10) QOL_EDGE(11)
