@@ -293,8 +293,10 @@ Engine::~Engine() {
   if (stream) (void)hipStreamDestroy(stream);
 }
 
-// The boundary tangents' part of d_basis (at most 104 KB) is not counted: the
-// largest call qol_rrq_noalloc_ accepts stays what it was without it.
+// The count sets the largest call qol_rrq_noalloc_ accepts, and stays what callers
+// know: the boundary tangents' part of d_basis (at most 104 KB) is not in it, and the
+// 10 h^2 (and above 120 KB another 4 h^2) doubles of a former weights operator are,
+// where d_X takes 4 h^2.
 size_t Engine::one_panel_bytes(i64 p, i64 m, i64 ichart, bool square) {
   const OrderTables& T = order_tables(p, square);
   LevelArgs LA{};
@@ -326,7 +328,7 @@ size_t Engine::one_panel_bytes(i64 p, i64 m, i64 ichart, bool square) {
   for (size_t b : {16 * D, 9 * nq * D, 6 * nb * D, 3 * h * D, 2 * nb * (size_t)(p * (p + 1) / 2) * D, 3 * h * h * D, h * h * D,
                    h * h * D, 10 * h * h * D, h * h * D})
     add(b);
-  if (!rrq_solve_g1_in_lds((int)h)) add(4 * h * h * D);
+  if (6 * h * h * D > 120 * 1024) add(4 * h * h * D);
   // eval: Omega, Ias, the per-pair RRQ data, the level geometry
   for (size_t b : {4 * h * mm * D, mm * D, 4 * mm * D, 3 * nq * mm * D, 3 * mm * D, 9 * mm * D,
                    rrq_edge_order_ints((int64_t)mm) * I, (size_t)16, 5 * h * mm * D, 8 * ntot * D, 4 * nsubtot * D})
@@ -585,13 +587,16 @@ void Engine::alloc_rrq() {
   d_Fq.alloc(sizeof(double) * 3 * (size_t)h * h * np_);
   d_Msl.alloc(sizeof(double) * (size_t)h * h * np_);
   d_Fn.alloc(sizeof(double) * (size_t)h * h * np_);
-  d_G.alloc(sizeof(double) * 10 * (size_t)h * h * np_);
+  d_X.alloc(sizeof(double) * 4 * (size_t)h * h * np_);
   d_Binv.alloc(sizeof(double) * (size_t)h * h * np_);
-  if (!rrq_solve_g1_in_lds(h)) d_scr.alloc(sizeof(double) * 4 * (size_t)h * h * np_);
   RP.frame = (double*)d_frame.ptr; RP.edge = (double*)d_edge.ptr; RP.bX = (double*)d_bX.ptr;
   RP.cx = (double*)d_cx.ptr; RP.basis = (double*)d_basis.ptr; RP.Fq = (double*)d_Fq.ptr;
   RP.Msl = (double*)d_Msl.ptr; RP.Fn = (double*)d_Fn.ptr;
-  RP.G = (double*)d_G.ptr; RP.Binv = (double*)d_Binv.ptr; RP.scr = rrq_solve_g1_in_lds(h) ? nullptr : (double*)d_scr.ptr;
+  if (rrq_forms_operator(p)) {
+    d_G.alloc(sizeof(double) * 4 * (size_t)h * h * np_);
+    RP.G = (double*)d_G.ptr;
+  }
+  RP.X = (double*)d_X.ptr; RP.Binv = (double*)d_Binv.ptr;
   rrq_alloc = true;
 }
 
@@ -725,7 +730,7 @@ void Engine::eval(int exterior, double side_tol, bool want_omega) {
   HIPCHK(hipStreamWaitEvent(stream, ev_solve, 0));
   rec(9, 0, stream);
   launch_rrq_weights(tab->RT, RP, (const int*)d_lpairs.ptr, (const int*)d_lstart.ptr, (const int*)d_ltot.ptr, npan,
-                     (const int*)d_nrrq.ptr, (const double*)d_vt.ptr, (double*)d_wout.ptr, stream);
+                     (const int*)d_nrrq.ptr, (const double*)d_vt.ptr, (double*)d_wout.ptr, nnz, stream);
   rec(9, 1, stream);
   if (fuse) launch_correction(4, 4, stream);
   // join: everything after eval on the main stream sees every weight

@@ -90,7 +90,7 @@ struct Engine {
   DevBuf d_lgeo, d_balls, d_pq, d_w1, d_oe, d_root, d_eorder, d_vt;
   DevBuf d_pfail;              // projections ended at the step cap: count, largest last step
   bool projected = false;      // the last eval ran the projection (it had RRQ pairs to run)
-  DevBuf d_frame, d_edge, d_bX, d_cx, d_basis, d_Fq, d_Msl, d_Fn, d_G, d_Binv, d_scr;
+  DevBuf d_frame, d_edge, d_bX, d_cx, d_basis, d_Fq, d_Msl, d_Fn, d_X, d_G, d_Binv;
   DevBuf d_ub, d_ubn, d_u, d_tcount, d_toffs, d_tcur, d_tpairs;
   DevBuf d_fsrc, d_fpart;     // far field: packed sources, per-chunk sums
   RRQPanels RP{};

@@ -60,9 +60,9 @@ struct RRQPanels {
   double* Fq;      // [npan][h][h][3] pure quaternions grad F_k(y_i)
   double* Msl;     // [npan][h][h] Msl^T (column-major)
   double* Fn;      // [npan][h][h] F_k at the nodes, F(i,k)
-  double* G;       // [npan][5h][2h] weights operator (transposed)
-  double* Binv;    // [npan][h][h] (Msl^T)^{-1}, row-major
-  double* scr;     // [npan][4h^2] G1 when it does not fit in LDS, else null
+  double* X;       // [npan][4h][h] inverse X of Fq by component: (X_kj)_q at (q*h + k)*h + j
+  double* G;       // [npan][4h][h] B Fn^T X_q / (4pi alpha), transposed; where rrq_forms_operator, else null
+  double* Binv;    // [npan][h][h] B = (Msl^T)^{-1}, transposed: B(j, r) at r*h + j
 };
 
 __global__ void level_geom_kernel(LevelArgs A, int npan, const double* sx, const double* rts, const double* rps,
@@ -177,11 +177,11 @@ __global__ void rrq_panel_frame_kernel(RRQTables T, RRQPanels P, int npan, const
                                        const double* snx, const double* sw, int ichart, const double* sxbd_chart,
                                        const double* rv_chart);
 void launch_rrq_system(int p, RRQPanels P, int npan, const double* sx, const double* snx, hipStream_t s);
-// variant 0: register-resident inverses up to order 8 (QOL_SOLVE_FUSED=1 / QOL_SOLVE_MFMA=1
-// select the others), 1: the fused vector-unit elimination, 2: the matrix-core
-// quaternion elimination (orders up to 8; the default above)
+// variant 0: register-resident inverses (QOL_SOLVE_FUSED=1 / QOL_SOLVE_MFMA=1 select
+// the others), 1: the fused vector-unit elimination, 2: the matrix-core quaternion
+// elimination (orders up to 8; the default above)
 void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq, hipStream_t s, int variant = 0);
-bool rrq_solve_g1_in_lds(int h);
+bool rrq_forms_operator(int p);
 void launch_rrq_project(RRQTables T, RRQPanels P, const int* lpairs, const int* ltot, const int* ppanel,
                         const int* tidx, const double* tx, const double* sx, int exterior, double side_tol,
                         double* pq, int* order, int* nfail, int64_t nnz, hipStream_t s);
@@ -194,7 +194,7 @@ void launch_rrq_target(RRQTables T, RRQPanels P, const int* lpairs, const int* l
                        const int* tidx, const double* tx, const int* nrrq, const double* w1g, const double* oeg,
                        double* vt, double* omega_out, double* ias_out, int64_t nnz, hipStream_t s);
 void launch_rrq_weights(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
-                        const int* nrrq, const double* vt, double* wout, hipStream_t s);
+                        const int* nrrq, const double* vt, double* wout, int64_t nnz, hipStream_t s);
 size_t rrq_frame_smem(int h, int nq);
 size_t rrq_basis_doubles(int p, int nq);  // RRQPanels::basis, per panel
 

@@ -417,9 +417,10 @@ void launch_rrq_system(int p, RRQPanels P, int npan, const double* sx, const dou
 // pivot row, so row piv[k] ends as row k of the inverse.  Two barriers per step;
 // LDS buffers alternate between steps.
 //
-// With G1(i, (b,k)) = (X_ki)_b, Ad = G1 rhs / 4pi solves M^T w = rhs (first h
-// components), and As = B (W/4pi + Fn^T Ad) / alpha = (C rhs + B W) / (4pi alpha),
-// C = B Fn^T G1.  Rows j < h of G: As, rows h..2h-1: Ad.
+// A pair's weights then are Ad = v / 4pi with v_j = sum_{k,q} (X_kj)_q rhs_qk, the
+// solution of M^T w = rhs (first h components), and As = B (W + Fn^T v) / (4pi alpha)
+// (rrq_weights_kernel).  Every solve kernel leaves the four components of X in P.X,
+// (X_kj)_q at (q h + k) h + j, and B in P.Binv, transposed: B(j, r) at r h + j.
 __device__ __forceinline__ void qmul_fma(const double* a, const double* b, double* c) {
   c[0] = fma(a[0], b[0], fma(-a[1], b[1], fma(-a[2], b[2], -a[3] * b[3])));
   c[1] = fma(a[0], b[1], fma(a[1], b[0], fma(a[2], b[3], -a[3] * b[2])));
@@ -440,63 +441,21 @@ __device__ __forceinline__ int first_unused(const unsigned long long* u) {
   return u[0] != ~0ull ? __builtin_ctzll(~u[0]) : 64 + __builtin_ctzll(~u[1]);
 }
 
-bool rrq_solve_g1_in_lds(int h) { return (size_t)6 * h * h * sizeof(double) <= 120 * 1024; }
-size_t rrq_solve_smem(int h) {
-  return sizeof(double) * (size_t)((rrq_solve_g1_in_lds(h) ? 4 * h * h : 0) + 2 * h * h);
-}
-
-// Shared tail of the solve kernels: C = B Fn^T, then G (stored transposed,
-// G(row, c) at c*2h + row): rows j<h  As = (C rhs + B W) * fa, rows h..2h-1
-// Ad = G1 rhs * fac.  Bt = B^T (Bt[r*h + j] = B(j, r)) and Ct = C^T in LDS, G1 in
-// LDS or scratch.  Threads run over consecutive j, so the G stores coalesce and
-// the LDS reads of Bt / Ct are conflict-free (G1 and Fn values are broadcasts).
-__device__ void solve_tail(int h, const double* Bt, double* Ct, const double* G1, const double* __restrict__ FN,
-                           double* __restrict__ G, double fa, double fac) {
-  const int H4 = 4 * h, H5 = 5 * h, m = 2 * h;
-  // Ct[i*h + j] = C(j, i) = sum_r B(j, r) Fn(i, r)
-  for (int e = threadIdx.x; e < h * h; e += blockDim.x) {
-    const int j = e % h, i = e / h;
-    double s = 0.0;
-    for (int r = 0; r < h; ++r) s = fma(Bt[(size_t)r * h + j], FN[i + (size_t)h * r], s);
-    Ct[(size_t)i * h + j] = s;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < h * H5; e += blockDim.x) {
-    const int j = e % h, c = e / h;
-    double* Gc = G + (size_t)c * m;
-    Gc[h + j] = c < H4 ? G1[(size_t)j * H4 + c] * fac : 0.0;
-    double s = 0.0;
-    if (c < H4) {
-      for (int i = 0; i < h; ++i) s = fma(Ct[(size_t)i * h + j], G1[(size_t)i * H4 + c], s);
-    } else {
-      s = Bt[(size_t)(c - H4) * h + j];
-    }
-    Gc[j] = s * fa;
-  }
-}
-
 template <int RPT, int CPT>
 __global__ void __launch_bounds__(256) rrq_panel_solve_kernel(RRQTables T, RRQPanels P, int npan,
                                                               const int* __restrict__ nrrq) {
   const int k = blockIdx.x;
   if (nrrq && nrrq[k] == 0) return;  // null: every panel
-  const int h = T.h, H4 = 4 * h, H5 = 5 * h, m = 2 * h;
+  const int h = T.h, m = 2 * h;
   constexpr int NR = 16 * RPT, NC = 16 * CPT;
   __shared__ double colq[2][4 * NR], colr[2][NR], prq[2][4 * NC], prr[2][NC];
   __shared__ double cvq[2][4], cvr[2][4];
   __shared__ int ciq[2][4], cir[2][4];
   __shared__ int pivq[NR], pivr[NR];
-  extern __shared__ double dyn[];
-  double* Bm = dyn;                      // [h][h] B(r,c) at r*h+c
-  double* Cm = Bm + (size_t)h * h;       // [h][h] (B Fn^T)(j,i) at j*h+i
-  double* G1 = P.scr ? P.scr + (size_t)k * 4 * h * h : Cm + (size_t)h * h;  // [h][4h]
+  double *X = P.X + (size_t)k * 4 * h * h, *Bk = P.Binv + (size_t)k * h * h;
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
   const double* FQ = P.Fq + (size_t)k * 3 * h * h;
   const double* MS = P.Msl + (size_t)k * h * h;
-  const double* FN = P.Fn + (size_t)k * h * h;
-  double* G = P.G + (size_t)k * 2 * h * H5;
-  const double alpha = P.frame[(size_t)k * 16 + 12];
-  const double fac = 1.0 / (16.0 * atan(1.0));
   double Aq[RPT][CPT][4], Ar[RPT][CPT];
 #pragma unroll
   for (int a = 0; a < RPT; ++a)
@@ -666,12 +625,10 @@ __global__ void __launch_bounds__(256) rrq_panel_solve_kernel(RRQTables T, RRQPa
         // row piv[k] holds row k of the inverse, column h+j' holds its column piv[j']
         const int jq = pivq[c - h], jr = pivr[c - h];
         const int kq = posq[r], kr = posr[r];
-        for (int q = 0; q < 4; ++q) G1[(size_t)jq * H4 + q * h + kq] = Aq[a][b][q];
-        Bm[(size_t)jr * h + kr] = Ar[a][b];  // transposed: Bt[r*h + j] = B(j, r)
+        for (int q = 0; q < 4; ++q) X[(size_t)(q * h + kq) * h + jq] = Aq[a][b][q];
+        Bk[(size_t)jr * h + kr] = Ar[a][b];
       }
     }
-  __syncthreads();
-  solve_tail(h, Bm, Cm, G1, FN, G, fac / alpha, fac);
 }
 
 // Entry (a, b) of the left-multiplication matrix of quaternion q (q*x = L(q) x):
@@ -699,22 +656,15 @@ __global__ void __launch_bounds__(256) rrq_panel_solve_mfma_kernel(RRQTables T, 
                                                                    const int* __restrict__ nrrq) {
   const int k = blockIdx.x;
   if (nrrq && nrrq[k] == 0) return;  // null: every panel
-  const int h = T.h, H4 = 4 * h, m = 2 * h;
+  const int h = T.h, m = 2 * h;
   constexpr int RTW = (RT + 3) / 4, NQR = 4 * RT, NC = 16 * CT;
   __shared__ double colq[2][4 * NQR], prq[2][4 * NC];
   __shared__ double cvq[2][4];
   __shared__ int ciq[2][4];
   __shared__ int pivq[NQR], posq[NQR];
-  extern __shared__ double dyn[];
-  double* Bm = dyn;
-  double* Cm = Bm + (size_t)h * h;
-  double* G1 = P.scr ? P.scr + (size_t)k * 4 * h * h : Cm + (size_t)h * h;
+  double* X = P.X + (size_t)k * 4 * h * h;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
   const double* FQ = P.Fq + (size_t)k * 3 * h * h;
-  const double* FN = P.Fn + (size_t)k * h * h;
-  double* G = P.G + (size_t)k * 2 * h * 5 * h;
-  const double alpha = P.frame[(size_t)k * 16 + 12];
-  const double fac = 1.0 / (16.0 * atan(1.0));
   qd4 D[RTW][CT];
 #pragma unroll
   for (int t = 0; t < RTW; ++t)
@@ -725,8 +675,6 @@ __global__ void __launch_bounds__(256) rrq_panel_solve_mfma_kernel(RRQTables T, 
         const int rt = wv + 4 * t, r = 4 * rt + i, c = 16 * ct + li;
         D[t][ct][i] = (rt < RT && r < h && c < h && lk > 0) ? FQ[3 * ((size_t)r * h + c) + lk - 1] : 0.0;
       }
-  // B = (Msl^T)^{-1} from its own kernel, to LDS transposed (Bt[r*h + j] = B(j, r))
-  for (int e = threadIdx.x; e < h * h; e += blockDim.x) Bm[(size_t)(e % h) * h + e / h] = P.Binv[(size_t)k * h * h + e];
   unsigned long long uq[2] = {0ull, 0ull};
   for (int kk = 0; kk < h; ++kk) {
     const int buf = kk & 1, kt = kk & 15, kb = kk >> 4;
@@ -852,14 +800,12 @@ __global__ void __launch_bounds__(256) rrq_panel_solve_mfma_kernel(RRQTables T, 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * rt + i, c = 16 * ct + li;
-        if (r < h && c >= h && c < m) G1[(size_t)pivq[c - h] * H4 + lk * h + posq[r]] = D[t][ct][i];
+        if (r < h && c >= h && c < m) X[(size_t)(lk * h + posq[r]) * h + pivq[c - h]] = D[t][ct][i];
       }
   }
-  __syncthreads();
-  solve_tail(h, Bm, Cm, G1, FN, G, fac / alpha, fac);
 }
 
-// B = (Msl^T)^{-1} (row-major, B(r,c) at r*h + c) by the same windowed
+// B = (Msl^T)^{-1} (transposed, B(r,c) at c*h + r) by the same windowed
 // Gauss-Jordan on the 16 x 16 thread grid; small enough to run many panels per CU.
 template <int RPT, int CPT>
 __global__ void __launch_bounds__(256) rrq_msl_inverse_kernel(RRQTables T, RRQPanels P, int npan,
@@ -966,7 +912,7 @@ __global__ void __launch_bounds__(256) rrq_msl_inverse_kernel(RRQTables T, RRQPa
 #pragma unroll
     for (int b = 0; b < CPT; ++b) {
       const int r = ty + 16 * a, c = tx + 16 * b;
-      if (r < h && c >= h && c < m) Bk[(size_t)posr[r] * h + pivr[c - h]] = Ar[a][b];
+      if (r < h && c >= h && c < m) Bk[(size_t)pivr[c - h] * h + posr[r]] = Ar[a][b];
     }
 }
 
@@ -981,90 +927,6 @@ struct RowMask {
   // lowest row not yet pivoted
   __device__ __forceinline__ int first_free() const { return ~lo ? __builtin_ctzll(~lo) : 64 + __builtin_ctzll(~hi); }
 };
-
-// The epilogue of the quaternion solve, shared by rrq_quat_inverse_kernel with
-// EPI (X in registers) and rrq_quat_epilogue_kernel (X from the Ad rows of G):
-// with
-// B = (Msl^T)^{-1} from rrq_real_inverse_kernel and X = Fq^{-1},
-//   Ad rows  G(h+j, q*h+k) = (X_kj)_q fac
-//   As rows  G(j, q*h+k)   = (fac/alpha) sum_i C(j,i) (X_ki)_q,  C = B Fn^T
-//   W block  G(j, 4h+r)    = (fac/alpha) B(j,r),  G(h+j, 4h+r) = 0
-// G is stored transposed, G(row, c) at c*2h + row.  LDS (3h^2 doubles): C, then
-// Bt and Fn (for C) or one component of X at a time (Xq aliases Bt).
-struct SolveLds {
-  double* Ct;  // Ct[i*h + j] = C(j, i)
-  double* Bt;  // Bt[r*h + j] = B(j, r)
-  double* Fs;  // Fs[i + h*r] = Fn(i, r)
-  double* Xq;  // Xq[i*h + k] = (X_ki)_q
-  __device__ SolveLds(double* dyn, int h)
-      : Ct(dyn), Bt(dyn + (size_t)h * h), Fs(dyn + (size_t)2 * h * h), Xq(dyn + (size_t)h * h) {}
-};
-
-// C = B Fn^T into LDS and the W block of G; ends with C visible to every thread
-// once the caller's next barrier has passed
-__device__ __forceinline__ void solve_epilogue_c(const RRQPanels& P, int k, int h, const SolveLds& L, double fa,
-                                                 double* G, int tid, int nth) {
-  const int m = 2 * h;
-  {
-    const double* Bk = P.Binv + (size_t)k * h * h;
-    const double* FN = P.Fn + (size_t)k * h * h;
-    for (int e = tid; e < h * h; e += nth) {
-      L.Bt[(size_t)(e % h) * h + e / h] = Bk[e];
-      L.Fs[e] = FN[e];
-    }
-  }
-  __syncthreads();
-  const int nig = (h + 3) / 4;
-  for (int it = tid; it < h * nig; it += nth) {
-    const int j = it % h, i0 = 4 * (it / h);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int r = 0; r < h; ++r) {
-      const double bv = L.Bt[(size_t)r * h + j];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc[u] = fma(bv, L.Fs[(i0 + u < h ? i0 + u : h - 1) + (size_t)h * r], acc[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u < h) L.Ct[(size_t)(i0 + u) * h + j] = acc[u];
-  }
-  for (int e = tid; e < h * h; e += nth) {
-    const int j = e % h, r = e / h;
-    double* w = G + (size_t)(4 * h + r) * m;
-    w[j] = L.Bt[(size_t)r * h + j] * fa;
-    w[h + j] = 0.0;
-  }
-}
-
-// As rows of component q from C and Xq in LDS: tiles of 3 rows j x 4 columns k
-__device__ __forceinline__ void solve_epilogue_as(int h, int q, const SolveLds& L, double fa, double* G, int tid,
-                                                  int nth) {
-  const int m = 2 * h;
-  const int njg = (h + 2) / 3, nkg = (h + 3) / 4;
-  for (int it = tid; it < njg * nkg; it += nth) {
-    const int j0 = 3 * (it % njg), k0 = 4 * (it / njg);
-    double acc[3][4];
-#pragma unroll
-    for (int v = 0; v < 3; ++v)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc[v][u] = 0.0;
-    for (int i = 0; i < h; ++i) {
-      double cv[3], xv[4];
-#pragma unroll
-      for (int v = 0; v < 3; ++v) cv[v] = L.Ct[(size_t)i * h + (j0 + v < h ? j0 + v : h - 1)];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) xv[u] = L.Xq[(size_t)i * h + (k0 + u < h ? k0 + u : h - 1)];
-#pragma unroll
-      for (int v = 0; v < 3; ++v)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc[v][u] = fma(cv[v], xv[u], acc[v][u]);
-    }
-#pragma unroll
-    for (int v = 0; v < 3; ++v)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if ((j0 + v < h) & (k0 + u < h)) G[(size_t)(q * h + k0 + u) * m + j0 + v] = acc[v][u] * fa;
-  }
-}
 
 // X = Fq^{-1} for the h x h pure-quaternion matrix Fq by Gauss-Jordan, the
 // matrix in registers of NW waves (one panel per workgroup).  Lane (ly, lx) of
@@ -1081,18 +943,14 @@ __device__ __forceinline__ void solve_epilogue_as(int h, int q, const SolveLds& 
 // pivot afterwards).  Each wave already holds its part of the pivot row, so one
 // workgroup barrier per step suffices (LDS double-buffered by step parity).
 // Afterwards row piv[k] holds row k of X with slot s holding column piv[s].
-// EPI: the kernel also forms G (solve_epilogue_*, 3h^2 doubles of dynamic LDS);
-// otherwise it writes X itself into the Ad rows of G, G(h+j, q*h+k) = (X_kj)_q,
-// and rrq_quat_epilogue_kernel finishes G, so that the elimination needs no
-// dynamic LDS and more panels share a CU.
-template <int RL, int RA, int CL, int CB, int NW, bool EPI>
+template <int RL, int RA, int CL, int CB, int NW>
 __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, RRQPanels P, int npan,
                                                                    const int* __restrict__ nrrq) {
   static_assert(RL * CL <= 64 && RL * RA <= 128 && CB % NW == 0, "lane grid");
   constexpr int CW = CB / NW;  // slot groups per wave
   const int k = blockIdx.x;
   if (nrrq && nrrq[k] == 0) return;  // null: every panel
-  const int h = T.h, m = 2 * h;
+  const int h = T.h;
   constexpr int NRW = RL * RA, NSL = CL * CB;
   __shared__ double colq[2][4 * NRW], rowq[2][4 * NSL], pivel[2][4];
   __shared__ int pivs[2], piv[NRW], pos[NRW];
@@ -1236,85 +1094,26 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
   }
   __syncthreads();
   for (int i = threadIdx.x; i < h; i += 64 * NW) pos[piv[i]] = i;
-  double* G = P.G + (size_t)k * m * 5 * h;
-  if constexpr (!EPI) {
-    __syncthreads();
+  __syncthreads();
+  double* X = P.X + (size_t)k * 4 * h * h;
 #pragma unroll
-    for (int a = 0; a < RA; ++a)
+  for (int a = 0; a < RA; ++a)
 #pragma unroll
-      for (int b = 0; b < CW; ++b) {
-        const int r = ly + RL * a, c = lx + CL * (wv * CW + b);
-        if (act & (r < h) & (c < h)) {
-          const int kx = pos[r], j = piv[c];
+    for (int b = 0; b < CW; ++b) {
+      const int r = ly + RL * a, c = lx + CL * (wv * CW + b);
+      if (act & (r < h) & (c < h)) {
+        const int kx = pos[r], j = piv[c];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) G[(size_t)(q * h + kx) * m + h + j] = A[a][b][q];
-        }
+        for (int q = 0; q < 4; ++q) X[(size_t)(q * h + kx) * h + j] = A[a][b][q];
       }
-  } else {
-    extern __shared__ double dyn[];
-    const SolveLds L(dyn, h);
-    const double fac = 1.0 / (16.0 * atan(1.0));
-    const double fa = fac / P.frame[(size_t)k * 16 + 12];
-    solve_epilogue_c(P, k, h, L, fa, G, threadIdx.x, 64 * NW);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      __syncthreads();  // Bt/Fn (q = 0) or the previous component no longer read
-#pragma unroll
-      for (int a = 0; a < RA; ++a)
-#pragma unroll
-        for (int b = 0; b < CW; ++b) {
-          const int r = ly + RL * a, c = lx + CL * (wv * CW + b);
-          if (act & (r < h) & (c < h)) {
-            const int kx = pos[r], j = piv[c];
-            L.Xq[(size_t)j * h + kx] = A[a][b][q];
-            G[(size_t)(q * h + kx) * m + h + j] = A[a][b][q] * fac;
-          }
-        }
-      __syncthreads();
-      solve_epilogue_as(h, q, L, fa, G, threadIdx.x, 64 * NW);
     }
-  }
 }
-
-// The rest of G after rrq_quat_inverse_kernel<..., false> has left X in its Ad
-// rows: the same epilogue as the fused form (so the same results), one
-// workgroup of 16 waves per panel (its 3h^2 doubles of LDS leave one workgroup
-// per CU at h = 66 and 78, so the waves hide the LDS latency: 256, 512 and 1024
-// threads took 4.3, 2.8 and 2.0 ms at order 12), X read back one component at a
-// time and the Ad rows scaled in place.
-__global__ void __launch_bounds__(1024) rrq_quat_epilogue_kernel(RRQTables T, RRQPanels P, int npan,
-                                                                const int* __restrict__ nrrq) {
-  const int k = blockIdx.x;
-  if (nrrq && nrrq[k] == 0) return;
-  const int h = T.h, m = 2 * h;
-  extern __shared__ double dyn[];
-  const SolveLds L(dyn, h);
-  const double fac = 1.0 / (16.0 * atan(1.0));
-  const double fa = fac / P.frame[(size_t)k * 16 + 12];
-  double* G = P.G + (size_t)k * m * 5 * h;
-  solve_epilogue_c(P, k, h, L, fa, G, threadIdx.x, blockDim.x);
-  for (int q = 0; q < 4; ++q) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < h * h; e += blockDim.x) {
-      const int j = e % h, kx = e / h;
-      double* g = G + (size_t)(q * h + kx) * m + h + j;
-      const double x = *g;
-      L.Xq[(size_t)j * h + kx] = x;
-      *g = x * fac;
-    }
-    __syncthreads();
-    solve_epilogue_as(h, q, L, fa, G, threadIdx.x, blockDim.x);
-  }
-}
-
-// dynamic LDS of rrq_quat_inverse_kernel: C plus Bt and Fn (or one component of X)
-size_t rrq_quat_inverse_smem(int h) { return sizeof(double) * (size_t)3 * h * h; }
 
 // B = (Msl^T)^{-1} by Gauss-Jordan in the registers of one wave per panel, the
 // real counterpart of rrq_quat_inverse_kernel (same lane grid, slot reuse,
 // implicit pivoting with ties to the lower row, zeroed pivot-row column entry).
-// The system matrix is A(r, c) = Msl[r + h*c]; output B row-major, B(kx, j) at
-// Binv[kx*h + j].
+// The system matrix is A(r, c) = Msl[r + h*c]; output B transposed, B(kx, j) at
+// Binv[j*h + kx].
 template <int RL, int RA, int CL, int CB>
 __global__ void __launch_bounds__(64) rrq_real_inverse_kernel(RRQTables T, RRQPanels P, int npan,
                                                               const int* __restrict__ nrrq) {
@@ -1419,28 +1218,85 @@ __global__ void __launch_bounds__(64) rrq_real_inverse_kernel(RRQTables T, RRQPa
   __syncthreads();
   double* Bk = P.Binv + (size_t)k * h * h;
 #pragma unroll
-  for (int a = 0; a < RA; ++a)
+  for (int b = 0; b < CB; ++b)
 #pragma unroll
-    for (int b = 0; b < CB; ++b) {
+    for (int a = 0; a < RA; ++a) {
       const int r = ly + RL * a, c = lx + CL * b;
-      if (act & (r < h) & (c < h)) Bk[(size_t)pos[r] * h + piv[c]] = A[a][b];
+      if (act & (r < h) & (c < h)) Bk[(size_t)piv[c] * h + pos[r]] = A[a][b];
     }
 }
 
-// whether one workgroup on the current device may take this much dynamic LDS
-// (beside a few KB of static LDS)
-static bool lds_fits(size_t bytes) {
-  int dev = 0, mx = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  if (hipDeviceGetAttribute(&mx, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) return false;
-  return bytes + 16 * 1024 <= (size_t)mx;
+// G of orders 11 and 12 (RRQPanels::G): G(j, q h + k) = sum_i C(j,i) (X_ki)_q / (4pi alpha)
+// with C = B Fn^T.  One workgroup per panel, C in LDS; a wave forms 16 columns of G at a
+// time from 16 rows of X, the order-12 panel's five tiles of 16 rows j as five independent
+// chains over i that share every X value.
+// Bound by memory (10h^2 doubles a panel in 165 us at order 12, 1,600 panels) and its latency:
+// 0.31 ms there, where forming As, Ad and W blocks on the vector units took 0.70.
+constexpr int kOpW = 8;  // waves
+constexpr int kOpT = 5;  // tiles of 16 rows: 16 * 5 >= h
+
+template <int P_>
+__global__ void __launch_bounds__(64 * kOpW) rrq_operator_kernel(RRQPanels P, const int* __restrict__ nrrq) {
+  const int k = blockIdx.x;
+  if (nrrq && nrrq[k] == 0) return;
+  constexpr int h = P_ * (P_ + 1) / 2, hp = 16 * kOpT + 4;
+  static_assert(16 * kOpT >= h);
+  __shared__ double Ct[h * hp];  // C(j, i) at i*hp + j, zero for j >= h
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+  const double *X = P.X + (size_t)k * 4 * h * h, *Fn = P.Fn + (size_t)k * h * h, *B = P.Binv + (size_t)k * h * h;
+  double* G = P.G + (size_t)k * 4 * h * h;
+  const double fac = 1.0 / (16.0 * atan(1.0)), fa = fac / P.frame[(size_t)k * 16 + 12];
+  // D[4q + lk][li]: row i = i0 + 4q + lk, column j = j0 + li
+  for (int tile = w; tile < kOpT * kOpT; tile += kOpW) {
+    const int i0 = 16 * (tile / kOpT), j0 = 16 * (tile % kOpT);
+    const int ic = min(i0 + li, h - 1), jc = min(j0 + li, h - 1);
+    qd4 acc{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int r0 = 0; r0 < h; r0 += 4) {
+      const int r = r0 + lk, rc = min(r, h - 1);
+      const double f = r < h ? Fn[ic + (size_t)h * rc] : 0.0;
+      const double b = j0 + li < h ? B[(size_t)rc * h + jc] : 0.0;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(f, b, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (i0 + 4 * q + lk < h) Ct[(i0 + 4 * q + lk) * hp + j0 + li] = acc[q];
+  }
+  __syncthreads();
+  for (int c0 = 16 * w; c0 < 4 * h; c0 += 16 * kOpW) {
+    const int cc = min(c0 + li, 4 * h - 1);
+    qd4 acc[kOpT];
+#pragma unroll
+    for (int t = 0; t < kOpT; ++t) acc[t] = qd4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 5
+    for (int i0 = 0; i0 < h; i0 += 4) {
+      const int i = i0 + lk, ii = min(i, h - 1);
+      const double x = i < h ? X[(size_t)cc * h + ii] : 0.0;
+#pragma unroll
+      for (int t = 0; t < kOpT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, Ct[ii * hp + 16 * t + li], acc[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < kOpT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = c0 + 4 * q + lk, j = 16 * t + li;
+        if ((c < 4 * h) & (j < h)) G[(size_t)c * h + j] = acc[t][q] * fa;
+      }
+  }
 }
+
+// Where the solve forms G for the weights rather than leave them X, Fn and B.  The
+// two differ by how v's rounding passes through B Fn^T, which grows with the condition
+// of X: against the weights by G the potentials of a 12 x 36 surface move by 1e-10
+// (relative 2-norm, largest 7e-9) at order 10, 4e-10 (2e-8) at 11 and 2e-8 (1e-6) at
+// 12, so that the two highest orders keep G.  Up to order 10 the shorter product is the
+// faster one.
+bool rrq_forms_operator(int p) { return p >= 11; }
 
 void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq, hipStream_t s, int variant) {
   const int h = T.h;
   const int rpt = (h + 15) / 16, cpt = (2 * h + 15) / 16;
-  const size_t lds = rrq_solve_smem(h);
-  if (!rrq_solve_g1_in_lds(h) && !P.scr) throw std::runtime_error("RRQ solve: scratch for G1 not allocated");
   // variant 2 (or QOL_SOLVE_MFMA=1) selects, for patch orders up to 8, the
   // matrix-core quaternion elimination (A as 4-wave accumulator tiles, B from a
   // separate real inverse), which is slower on the order-8 workload (5.3 vs 4.9
@@ -1450,7 +1306,7 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
 #define QOL_SOLVE_MFMA(P_, RT_, CT_, RPT_)                                                                  \
   case P_:                                                                                                \
     hipLaunchKernelGGL((rrq_msl_inverse_kernel<RPT_, CT_>), dim3(npan), dim3(256), 0, s, T, P, npan, nrrq);  \
-    hipLaunchKernelGGL((rrq_panel_solve_mfma_kernel<RT_, CT_>), dim3(npan), dim3(256), lds, s, T, P, npan,   \
+    hipLaunchKernelGGL((rrq_panel_solve_mfma_kernel<RT_, CT_>), dim3(npan), dim3(256), 0, s, T, P, npan,     \
                        nrrq);                                                                             \
     return;
     QOL_SOLVE_MFMA(2, 1, 1, 1)
@@ -1464,60 +1320,40 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
   }
 #undef QOL_SOLVE_MFMA
   // by default the real and the quaternion inverse with the matrix in registers;
-  // variant 1 (or QOL_SOLVE_FUSED=1) selects the single fused kernel, which also
-  // serves orders 9-12 where the epilogue's LDS does not fit
+  // variant 1 (or QOL_SOLVE_FUSED=1) selects the single fused kernel
   const char* fu = std::getenv("QOL_SOLVE_FUSED");
   const bool fused = variant == 1 || (variant == 0 && fu && fu[0] == '1');
-  if (h <= 36 && !fused) {
-    // lane grid per order (rows RL x RA, slots CL x CB)
+  if (h <= 78 && !fused) {
+    // lane grid per order (rows RL x RA, slots CL x CB) and waves, about 48 quaternion
+    // entries per lane
 #define QOL_QINV(RL_, RA_, CL_, CB_, NW_)                                                                \
   hipLaunchKernelGGL((rrq_real_inverse_kernel<RL_, RA_, CL_, CB_>), dim3(npan), dim3(64), 0, s, T, P, npan, nrrq); \
-  hipLaunchKernelGGL((rrq_quat_inverse_kernel<RL_, RA_, CL_, CB_, NW_, true>), dim3(npan), dim3(64 * NW_),       \
-                     rrq_quat_inverse_smem(h), s, T, P, npan, nrrq)
+  hipLaunchKernelGGL((rrq_quat_inverse_kernel<RL_, RA_, CL_, CB_, NW_>), dim3(npan), dim3(64 * NW_), 0, s, T, P,   \
+                     npan, nrrq)
     if (h <= 3) { QOL_QINV(3, 1, 3, 1, 1); }
     else if (h <= 6) { QOL_QINV(6, 1, 6, 1, 1); }
     else if (h <= 10) { QOL_QINV(5, 2, 10, 1, 1); }
     else if (h <= 15) { QOL_QINV(3, 5, 15, 1, 1); }
     else if (h <= 21) { QOL_QINV(3, 7, 21, 1, 1); }
     else if (h <= 28) { QOL_QINV(4, 7, 16, 2, 2); }
-    else { QOL_QINV(6, 6, 10, 4, 2); }
+    else if (h <= 36) { QOL_QINV(6, 6, 10, 4, 2); }
+    else if (h <= 45) { QOL_QINV(8, 6, 8, 6, 3); }
+    else if (h <= 55) { QOL_QINV(9, 7, 7, 8, 4); }
+    else if (h <= 66) { QOL_QINV(10, 7, 6, 12, 6); }
+    else { QOL_QINV(12, 7, 5, 16, 8); }
 #undef QOL_QINV
-    return;
-  }
-  // patch orders 9 to 12: the same register-resident inverses over more waves
-  // (about 48 quaternion entries per lane), the elimination without dynamic LDS
-  // and G finished by rrq_quat_epilogue_kernel, whose 3h^2 doubles (146 KB at
-  // h = 78) must fit one workgroup's LDS
-  if (h <= 78 && !fused && lds_fits(rrq_quat_inverse_smem(h))) {
-    const size_t el = rrq_quat_inverse_smem(h);
-    if (el > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)rrq_quat_epilogue_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)el);
-#define QOL_QINV_SPLIT(RL_, RA_, CL_, CB_, NW_)                                                                   \
-  hipLaunchKernelGGL((rrq_real_inverse_kernel<RL_, RA_, CL_, CB_>), dim3(npan), dim3(64), 0, s, T, P, npan, nrrq); \
-  hipLaunchKernelGGL((rrq_quat_inverse_kernel<RL_, RA_, CL_, CB_, NW_, false>), dim3(npan), dim3(64 * NW_), 0, s, T, \
-                     P, npan, nrrq);                                                                              \
-  hipLaunchKernelGGL(rrq_quat_epilogue_kernel, dim3(npan), dim3(1024), el, s, T, P, npan, nrrq)
-    if (h <= 45) { QOL_QINV_SPLIT(8, 6, 8, 6, 3); }
-    else if (h <= 55) { QOL_QINV_SPLIT(9, 7, 7, 8, 4); }
-    else if (h <= 66) { QOL_QINV_SPLIT(10, 7, 6, 12, 6); }
-    else { QOL_QINV_SPLIT(12, 7, 5, 16, 8); }
-#undef QOL_QINV_SPLIT
-    return;
-  }
-  if (rpt <= 3 && cpt <= 5) {
-    if (lds > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)rrq_panel_solve_kernel<3, 5>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((rrq_panel_solve_kernel<3, 5>), dim3(npan), dim3(256), lds, s, T, P, npan, nrrq);
+  } else if (rpt <= 3 && cpt <= 5) {
+    hipLaunchKernelGGL((rrq_panel_solve_kernel<3, 5>), dim3(npan), dim3(256), 0, s, T, P, npan, nrrq);
   } else if (rpt <= 4 && cpt <= 7) {
-    (void)hipFuncSetAttribute((const void*)rrq_panel_solve_kernel<4, 7>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((rrq_panel_solve_kernel<4, 7>), dim3(npan), dim3(256), lds, s, T, P, npan, nrrq);
+    hipLaunchKernelGGL((rrq_panel_solve_kernel<4, 7>), dim3(npan), dim3(256), 0, s, T, P, npan, nrrq);
   } else if (rpt <= 5 && cpt <= 10) {
-    (void)hipFuncSetAttribute((const void*)rrq_panel_solve_kernel<5, 10>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((rrq_panel_solve_kernel<5, 10>), dim3(npan), dim3(256), lds, s, T, P, npan, nrrq);
+    hipLaunchKernelGGL((rrq_panel_solve_kernel<5, 10>), dim3(npan), dim3(256), 0, s, T, P, npan, nrrq);
   } else {
     throw std::runtime_error("RRQ solve supports patch orders up to 12");
   }
+  if (rrq_forms_operator(T.p))
+    hipLaunchKernelGGL(T.p == 11 ? rrq_operator_kernel<11> : rrq_operator_kernel<12>, dim3(npan), dim3(64 * kOpW), 0, s,
+                       P, nrrq);
 }
 
 // ---------------------------------------------------------------------------
@@ -2487,82 +2323,146 @@ void launch_rrq_target(RRQTables T, RRQPanels P, const int* lpairs, const int* l
   }
 }
 
-// RRQ weights of every RRQ pair of a panel: W (2h x nrrq) = G (2h x 5h) V (5h x nrrq)
-// on the FP64 matrix cores.  One workgroup of kWM waves per panel; wave w owns
-// output rows 16w..16w+15 and walks the panel's targets 16 at a time.  A operand:
-// G (stored transposed, coalesced over rows); B operand: the panel's moment
-// vectors (stored transposed, coalesced over targets).
-constexpr int kWM = 5;  // 16*kWM >= 2h for p <= 8; larger orders loop over row tiles
+// RRQ weights of a panel's pairs from their moment vectors (rhs_0 ... rhs_3, W), on
+// the FP64 matrix cores: v = X^T rhs (4h terms), y = W + Fn^T v, Ad = v / 4pi and
+// As = B y / (4pi alpha) (h terms each).  Rows: 32 pairs; columns: one wave per 16;
+// v and y pass from one product to the next through LDS.
+//
+// Applying B and Fn here takes 4h^2 multiply-adds a pair, so that the solve need not
+// multiply them into X (10h^3 a panel) and nothing but X, Fn and B goes through
+// memory (6h^2 doubles a panel where the product took 10h^2, and 162 instead of 225
+// matrix steps per 16 pairs at order 8).
+// Bound by the matrix cores and, with few panels, by the chains of 4h/8 dependent steps;
+// a panel's rounds are split over workgroups until there are 2048 of them.  Order 8,
+// 200,000 targets: weights 0.55 to 0.45 ms and the solve 2.1 to 1.6 ms; order 6, 1,501
+// targets of one panel: 44 to 13 us.
+constexpr int kWT = 32;  // pairs a round
 
-__global__ void __launch_bounds__(64 * kWM) rrq_weights_kernel(RRQTables T, RRQPanels P,
-                                                               const int* __restrict__ lpairs,
-                                                               const int* __restrict__ lstart,
-                                                               const int* __restrict__ ltot, int npan,
-                                                               const int* __restrict__ nrrq,
-                                                               const double* __restrict__ vt,
-                                                               double* __restrict__ wout) {
+// acc0, acc1 = A (kWT rows, from at(row, k)) times the lane's column of M (col(k)), over
+// k < n in steps of four: two row tiles share every column loaded, and even and odd
+// steps are separate chains
+template <class F, class M>
+__device__ __forceinline__ void weights_product(F&& at, M&& col, int n, qd4& acc0, qd4& acc1) {
+  const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+  acc0 = acc1 = qd4{0.0, 0.0, 0.0, 0.0};
+  qd4 acc2 = acc0, acc3 = acc0;
+#pragma unroll 3
+  for (int k0 = 0; k0 < n; k0 += 8) {
+    const int ka = k0 + lk, kb = k0 + 4 + lk, ca = min(ka, n - 1), cb = min(kb, n - 1);
+    const double ma = col(ca), mb = col(cb);
+    const double a0 = ka < n ? at(li, ca) : 0.0, a1 = ka < n ? at(16 + li, ca) : 0.0;
+    const double b0 = kb < n ? at(li, cb) : 0.0, b1 = kb < n ? at(16 + li, cb) : 0.0;
+    acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, ma, acc0, 0, 0, 0);
+    acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, ma, acc1, 0, 0, 0);
+    acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(b0, mb, acc2, 0, 0, 0);
+    acc3 = __builtin_amdgcn_mfma_f64_16x16x4f64(b1, mb, acc3, 0, 0, 0);
+  }
+  acc0 += acc2;
+  acc1 += acc3;
+}
+
+__global__ void __launch_bounds__(320) rrq_weights_kernel(RRQTables T, RRQPanels P, const int* __restrict__ lpairs,
+                                                          const int* __restrict__ lstart, const int* __restrict__ ltot,
+                                                          int npan, const int* __restrict__ nrrq,
+                                                          const double* __restrict__ vt, double* __restrict__ wout) {
   const int k = blockIdx.x;
   const int nm = nrrq[k];
-  if (nm == 0) return;
-  const int h = T.h, H5 = 5 * h, m2 = 2 * h;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
+  if ((int)blockIdx.y * kWT >= nm) return;
+  extern __shared__ double sm[];
+  const int h = T.h, hs = h + 1 - h % 2;  // rows of an odd number of doubles: a column's lanes in different banks
+  double *vs = sm, *ys = vs + kWT * hs;
+  const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+  const int j = 16 * (threadIdx.x >> 6) + li, jc = min(j, h - 1);  // this lane's column
   const int r0 = lstart[4 * (size_t)npan + k];
   const int* mine = lpairs + rrq_list_base(ltot) + r0;
-  const double* G = P.G + (size_t)k * m2 * H5;  // G(j, r) at r*2h + j
-  const double* V = vt + (size_t)r0 * H5;       // V(r, t) at r*nm + t
-  for (int mt = w; 16 * mt < m2; mt += kWM) {
-    const int j = 16 * mt + li;
-    const bool jin = j < m2;
-    const int jc = jin ? j : m2 - 1;
-    // two 16-target tiles per pass: two independent accumulator chains share
-    // every loaded G value
-    for (int t0 = 0; t0 < nm; t0 += 32) {
-      const int ta = t0 + li, tb = t0 + 16 + li;
-      const bool ina = ta < nm, inb = tb < nm;
-      const int tca = ina ? ta : nm - 1, tcb = inb ? tb : nm - 1;
-      // K split into even and odd steps as well: four independent chains
-      qd4 acc0 = qd4{0.0, 0.0, 0.0, 0.0}, acc1 = qd4{0.0, 0.0, 0.0, 0.0};
-      qd4 acc2 = qd4{0.0, 0.0, 0.0, 0.0}, acc3 = qd4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 3
-      for (int k0 = 0; k0 < H5; k0 += 8) {
-        const int r = k0 + lk, s2 = k0 + 4 + lk;
-        const bool rin = r < H5, sin_ = s2 < H5;
-        const int rc = rin ? r : H5 - 1, sc = sin_ ? s2 : H5 - 1;
-        const double a = (jin & rin) ? G[(size_t)rc * m2 + jc] : 0.0;
-        const double b0 = (ina & rin) ? V[(size_t)rc * nm + tca] : 0.0;
-        const double b1 = (inb & rin) ? V[(size_t)rc * nm + tcb] : 0.0;
-        const double a2 = (jin & sin_) ? G[(size_t)sc * m2 + jc] : 0.0;
-        const double b2 = (ina & sin_) ? V[(size_t)sc * nm + tca] : 0.0;
-        const double b3 = (inb & sin_) ? V[(size_t)sc * nm + tcb] : 0.0;
-        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, acc1, 0, 0, 0);
-        acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, b2, acc2, 0, 0, 0);
-        acc3 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, b3, acc3, 0, 0, 0);
-      }
-      acc0 += acc2;
-      acc1 += acc3;
-      // D[4q + lk][li]: output row 16mt + 4q + lk, target t0 + li (and t0 + 16 + li)
+  const double *X = P.X + (size_t)k * 4 * h * h, *Fn = P.Fn + (size_t)k * h * h, *B = P.Binv + (size_t)k * h * h;
+  const double* V = vt + (size_t)r0 * 5 * h;  // V(r, t) at r*nm + t
+  const double fac = 1.0 / (16.0 * atan(1.0)), fa = fac / P.frame[(size_t)k * 16 + 12];
+  for (int t0 = blockIdx.y * kWT; t0 < nm; t0 += kWT * gridDim.y) {
+    const int nt = min(kWT, nm - t0);
+    qd4 acc[2];
+    // D[4q + lk][li]: pair 4q + lk of the row tile, column j
+    auto each = [&](auto&& f) {
+      if (j < h)
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int t = half ? tb : ta;
-        if (!(half ? inb : ina)) continue;
-        const qd4& acc = half ? acc1 : acc0;
-        double* o = wout + (size_t)mine[t] * m2;
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int t = 16 * half + 4 * q + lk;
+            f(t, acc[half][q]);
+          }
+    };
+    weights_product([&](int t, int c) { return V[(size_t)c * nm + t0 + min(t, nt - 1)]; }, 
+                    [&](int c) { return X[(size_t)c * h + jc]; }, 4 * h, acc[0], acc[1]);
+    __syncthreads();  // the previous round has read vs and ys
+    each([&](int t, double v) {
+      vs[t * hs + j] = v;
+      if (t < nt) wout[(size_t)mine[t0 + t] * 2 * h + h + j] = v * fac;
+    });
+    __syncthreads();
+    weights_product([&](int t, int i) { return vs[t * hs + i]; }, [&](int i) { return Fn[(size_t)h * jc + i]; }, h, acc[0],
+                    acc[1]);
+    each([&](int t, double v) { ys[t * hs + j] = v + V[(size_t)(4 * h + j) * nm + t0 + min(t, nt - 1)]; });
+    __syncthreads();
+    weights_product([&](int t, int r) { return ys[t * hs + r]; }, [&](int r) { return B[(size_t)r * h + jc]; }, h, acc[0],
+                    acc[1]);
+    each([&](int t, double v) {
+      if (t < nt) wout[(size_t)mine[t0 + t] * 2 * h + j] = v * fa;
+    });
+  }
+}
+
+// The same with G formed (orders 11 and 12): As = G rhs + B W / (4pi alpha), Ad = X^T rhs
+// / 4pi with the factor in X, one wave per 16 columns of As and then of Ad (order 12,
+// 30,000 targets: 0.42 ms, from 0.51 with five waves a panel and all of G in memory)
+__global__ void __launch_bounds__(640) rrq_weights_formed_kernel(int h, RRQPanels P, const int* __restrict__ lpairs,
+                                                                 const int* __restrict__ lstart,
+                                                                 const int* __restrict__ ltot, int npan,
+                                                                 const int* __restrict__ nrrq,
+                                                                 const double* __restrict__ vt,
+                                                                 double* __restrict__ wout) {
+  const int nt16 = (h + 15) / 16;
+  const int k = blockIdx.x;
+  const int nm = nrrq[k];
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool ad = w >= nt16;
+  const int j = 16 * (ad ? w - nt16 : w) + li, jc = min(j, h - 1);
+  const int r0 = lstart[4 * (size_t)npan + k];
+  const int* mine = lpairs + rrq_list_base(ltot) + r0;
+  const double *X = P.X + (size_t)k * 4 * h * h + jc, *G = P.G + (size_t)k * 4 * h * h + jc;
+  const double *B = P.Binv + (size_t)k * h * h + jc, *V = vt + (size_t)r0 * 5 * h;
+  const double fac = 1.0 / (16.0 * atan(1.0)), fa = fac / P.frame[(size_t)k * 16 + 12];
+  for (int t0 = blockIdx.y * kWT; t0 < nm; t0 += kWT * gridDim.y) {
+    const int nt = min(kWT, nm - t0);
+    qd4 acc[2];
+    auto at = [&](int t, int c) { return V[(size_t)c * nm + t0 + min(t, nt - 1)]; };
+    if (ad)
+      weights_product(at, [&](int c) { return X[(size_t)c * h] * fac; }, 4 * h, acc[0], acc[1]);
+    else
+      weights_product(at, [&](int c) { return c < 4 * h ? G[(size_t)c * h] : B[(size_t)(c - 4 * h) * h] * fa; }, 5 * h, acc[0], acc[1]);
+    if (j < h)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int jj = 16 * mt + 4 * q + lk;
-          if (jj < m2) o[jj] = acc[q];
+          const int t = 16 * half + 4 * q + lk;
+          if (t < nt) wout[(size_t)mine[t0 + t] * 2 * h + (ad ? h : 0) + j] = acc[half][q];
         }
-      }
-    }
   }
 }
 
 void launch_rrq_weights(RRQTables T, RRQPanels P, const int* lpairs, const int* lstart, const int* ltot, int npan,
-                        const int* nrrq, const double* vt, double* wout, hipStream_t s) {
-  hipLaunchKernelGGL(rrq_weights_kernel, dim3(npan), dim3(64 * kWM), 0, s, T, P, lpairs, lstart, ltot, npan, nrrq,
-                     vt, wout);
+                        const int* nrrq, const double* vt, double* wout, int64_t nnz, hipStream_t s) {
+  const int64_t rounds = (nnz + kWT - 1) / kWT;
+  const int split = (int)std::max<int64_t>(1, std::min<int64_t>((2048 + npan - 1) / npan, rounds));
+  if (rrq_forms_operator(T.p)) {
+    hipLaunchKernelGGL(rrq_weights_formed_kernel, dim3(npan, split), dim3(128 * ((T.h + 15) / 16)), 0, s, T.h, P, lpairs, lstart, ltot, npan, nrrq, vt, wout);
+    return;
+  }
+  const int nw = (T.h + 15) / 16, hs = T.h + 1 - T.h % 2;
+  hipLaunchKernelGGL(rrq_weights_kernel, dim3(npan, split), dim3(64 * nw), sizeof(double) * 2 * kWT * hs, s, T, P,
+                     lpairs, lstart, ltot, npan, nrrq, vt, wout);
 }
 
 }  // namespace qol
