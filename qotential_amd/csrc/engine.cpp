@@ -296,7 +296,7 @@ Engine::~Engine() {
 // The count sets the largest call qol_rrq_noalloc_ accepts, and stays what callers
 // know: the boundary tangents' part of d_basis (at most 104 KB) is not in it, and the
 // 10 h^2 (and above 120 KB another 4 h^2) doubles of a former weights operator are,
-// where d_X takes 4 h^2.
+// where d_X (and d_G) take 4 h^2.
 size_t Engine::one_panel_bytes(i64 p, i64 m, i64 ichart, bool square) {
   const OrderTables& T = order_tables(p, square);
   LevelArgs LA{};
@@ -435,14 +435,13 @@ i64 Engine::nearlist() {
   d_cnt.alloc(sizeof(int) * npan);
   d_offs.alloc(sizeof(int) * (npan + 1));
   HIPCHK(hipMemsetAsync(d_cnt.ptr, 0, sizeof(int) * npan, stream));
-  hipLaunchKernelGGL(nearlist_prep_kernel, dim3(blocks(npan, 256)), dim3(256), 0, stream, npan, h,
+  hipLaunchKernelGGL(nearlist_prep_kernel, dim3(blocks(npan, 64)), dim3(64), 0, stream, npan, h,
                      (const double*)d_sx.ptr, (const double*)d_sw.ptr, (const double*)tab->d_corner.ptr, near_diam,
                      (double*)d_nball.ptr);
-  const int pb = 16;
-  const int gy = nt > 0 ? std::min(64, blocks(nt, 256)) : 1;
+  d_npart.alloc(sizeof(int) * (size_t)npan * std::max(1, nearlist_parts(npan, nt)));
   if (nt > 0)
-    hipLaunchKernelGGL(nearlist_count_kernel, dim3(blocks(npan, pb), gy), dim3(256), 0, stream, npan, nt,
-                       (const double*)d_tx.ptr, (const double*)d_nball.ptr, (int*)d_cnt.ptr);
+    launch_nearlist(false, npan, nt, (const double*)d_tx.ptr, (const double*)d_nball.ptr, (int*)d_npart.ptr,
+                    (int*)d_cnt.ptr, nullptr, nullptr, stream);
   hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, (const int*)d_cnt.ptr, npan, (int*)d_offs.ptr);
   int tot = 0;
   HIPCHK(hipMemcpyAsync(&tot, (int*)d_offs.ptr + npan, sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -450,8 +449,8 @@ i64 Engine::nearlist() {
   nnz = tot;
   d_tidx.alloc(sizeof(int) * (size_t)(nnz > 0 ? nnz : 1));
   if (nt > 0 && nnz > 0)
-    hipLaunchKernelGGL(nearlist_fill_kernel, dim3(blocks(npan, pb)), dim3(256), 0, stream, npan, nt,
-                       (const double*)d_tx.ptr, (const double*)d_nball.ptr, (const int*)d_offs.ptr, (int*)d_tidx.ptr);
+    launch_nearlist(true, npan, nt, (const double*)d_tx.ptr, (const double*)d_nball.ptr, (int*)d_npart.ptr, nullptr,
+                    (const int*)d_offs.ptr, (int*)d_tidx.ptr, stream);
   HIPCHK(hipGetLastError());
   alloc_pairs();
   evaluated = false;
@@ -465,7 +464,7 @@ i64 Engine::nearlist_grid() {
   d_nball.alloc(sizeof(double) * 4 * npan);
   d_cnt.alloc(sizeof(int) * npan);
   d_offs.alloc(sizeof(int) * (npan + 1));
-  hipLaunchKernelGGL(nearlist_prep_kernel, dim3(blocks(npan, 256)), dim3(256), 0, stream, npan, h,
+  hipLaunchKernelGGL(nearlist_prep_kernel, dim3(blocks(npan, 64)), dim3(64), 0, stream, npan, h,
                      (const double*)d_sx.ptr, (const double*)d_sw.ptr, (const double*)tab->d_corner.ptr, near_diam,
                      (double*)d_nball.ptr);
   std::vector<double> bl(4 * (size_t)npan);

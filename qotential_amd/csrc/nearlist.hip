@@ -6,14 +6,14 @@
 // factor f > 0 the radius is f h instead, h the largest distance between the
 // corners of the panel's interpolant (the "radius 2h" near list, f = 2; h as the
 // target generator defines the patch diameter).
-// Brute force over (panel, target) like the reference, but kPB panels per
-// workgroup share every target load, and the fill keeps ascending target order
-// with wavefront ballots so the CSR is bit-identical to the serial loop.
+// Brute force over (panel, target) like the reference, behind a test of groups of
+// panels, and the fill keeps ascending target order with wavefront ballots so the
+// CSR is bit-identical to the serial loop.
 #include "qol_kernels.h"
 
 namespace qol {
 
-constexpr int kPB = 16;  // panels per workgroup
+constexpr int kNearG = 4;  // groups of 16 panels a wave tests
 
 // ball[k] = (c0, c1, c2, r^2), summed in the reference's order; corner: the 3 x h
 // rows interpolating a panel at its corners (used when diam > 0)
@@ -57,79 +57,147 @@ __device__ __forceinline__ bool in_ball(const double* b, double x0, double x1, d
   return d0 * d0 + d1 * d1 + d2 * d2 < b[3];
 }
 
-__global__ void __launch_bounds__(256) nearlist_count_kernel(int npan, int nt, const double* __restrict__ tx,
-                                                             const double* __restrict__ ball, int* __restrict__ count) {
-  __shared__ double sb[4 * kPB];
-  __shared__ int sc[kPB];
-  const int k0 = blockIdx.x * kPB;
-  if (threadIdx.x < 4 * kPB) sb[threadIdx.x] = (k0 + threadIdx.x / 4 < npan) ? ball[4 * k0 + threadIdx.x] : 0.0;
-  if (threadIdx.x < kPB) sc[threadIdx.x] = 0;
-  __syncthreads();
-  int my[kPB];
-  for (int q = 0; q < kPB; ++q) my[q] = 0;
-  for (int t = blockIdx.y * blockDim.x + threadIdx.x; t < nt; t += gridDim.y * blockDim.x) {
-    const double x0 = tx[3 * (size_t)t], x1 = tx[3 * (size_t)t + 1], x2 = tx[3 * (size_t)t + 2];
-    for (int q = 0; q < kPB; ++q) my[q] += in_ball(sb + 4 * q, x0, x1, x2) ? 1 : 0;
+// One wave per 64 panels (lane = panel) and segment of `seg` targets: counts of the
+// segment (part[segment][panel], and added to count), or with FILL the targets
+// themselves from offs[panel] plus the counts of the earlier segments.
+//
+// Bound by the vector units (a test is 9 double operations; all pairs took 476 + 587 us
+// for 14,250 panels x 50,000 targets), and most pairs are far apart.  So a target is
+// first tested against a ball around the balls of 16 consecutive panels, widened beyond
+// any rounding of either test, and targets inside wait in LDS until 64 of them fill the
+// wave for the 16 panels' own tests: 1/16 of the tests plus those of the candidates, in
+// the targets' order.  A not-a-number ball or target passes the first test and fails the
+// second.  Segments and 64-thread workgroups because the fill's serial walk over all
+// targets left most of the chip idle.  14,250 panels x
+// 50,000 targets: 88 + 88 us; 2,400 x 20,011: 121 + 242 to 29 + 31.
+template <bool FILL>
+__global__ void __launch_bounds__(64) nearlist_kernel(int npan, int nt, int seg, const double* __restrict__ tx,
+                                                      const double* __restrict__ ball, int* __restrict__ part,
+                                                      int* __restrict__ count, const int* __restrict__ offs,
+                                                      int* __restrict__ idx) {
+  __shared__ int cand[kNearG][128];
+  const int lane = threadIdx.x, k0 = blockIdx.x * 64, k = min(k0 + lane, npan - 1);
+  const int t_lo = blockIdx.y * seg, t_hi = min(nt, t_lo + seg);
+  // the ball around this lane's group of 16 (panels past the last repeat it)
+  double bc[kNearG][4];
+  {
+    double c[3], m[3], r = sqrt(ball[4 * (size_t)k + 3]), d2 = 0.0;
+    for (int d = 0; d < 3; ++d) m[d] = c[d] = ball[4 * (size_t)k + d];
+    for (int o = 1; o < 16; o <<= 1)
+      for (int d = 0; d < 3; ++d) m[d] += __shfl_xor(m[d], o);
+    for (int d = 0; d < 3; ++d) {
+      m[d] *= 1.0 / 16.0;
+      d2 += (c[d] - m[d]) * (c[d] - m[d]);
+    }
+    r += sqrt(d2);
+    for (int o = 1; o < 16; o <<= 1) {
+      const double u = __shfl_xor(r, o);
+      r = u > r || u != u ? u : r;  // not-a-number wins
+    }
+    for (int g = 0; g < kNearG; ++g) {
+      for (int d = 0; d < 3; ++d) bc[g][d] = __shfl(m[d], 16 * g);
+      const double rg = __shfl(r, 16 * g);
+      bc[g][3] = rg * rg * (1.0 + 1e-9) + 1e-290;
+    }
   }
-  for (int q = 0; q < kPB; ++q) {
-    int v = my[q];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(&sc[q], v);
+  int held[kNearG] = {}, acc = 0;
+  if (FILL) {
+    acc = offs[k];
+#pragma unroll 4
+    for (int y = 0; y < (int)blockIdx.y; ++y) acc += part[(size_t)y * npan + k];
+  }
+  // the tests of group g's 16 panels on its first n candidates
+  auto test = [&](int g, int n) {
+    const int t = cand[g][lane];
+    const bool on = lane < n;
+    const double x0 = on ? tx[3 * (size_t)t] : 0.0, x1 = on ? tx[3 * (size_t)t + 1] : 0.0,
+                 x2 = on ? tx[3 * (size_t)t + 2] : 0.0;
+    for (int q = 0; q < 16; ++q) {
+      const int kq = k0 + 16 * g + q;
+      if (kq >= npan) break;
+      const bool in = on && in_ball(ball + 4 * (size_t)kq, x0, x1, x2);
+      const uint64_t b = __ballot(in);
+      if (b == 0) continue;
+      const int base = __builtin_amdgcn_readlane(acc, 16 * g + q);
+      if (FILL && in) idx[base + __popcll(b & ((1ull << lane) - 1ull))] = t;
+      acc += lane == 16 * g + q ? __popcll(b) : 0;
+    }
+  };
+  double x[3];
+  auto load = [&](int t) {
+    const size_t i = 3 * (size_t)min(t, nt - 1);
+    for (int d = 0; d < 3; ++d) x[d] = tx[i + d];
+  };
+  load(t_lo + lane);
+  for (int t0 = t_lo; t0 < t_hi; t0 += 64) {
+    const int t = t0 + lane;
+    const double x0 = x[0], x1 = x[1], x2 = x[2];
+    load(t + 64);
+#pragma unroll
+    for (int g = 0; g < kNearG; ++g) {
+      const double e0 = x0 - bc[g][0], e1 = x1 - bc[g][1], e2 = x2 - bc[g][2];
+      const bool keep = t < t_hi && !(fma(e0, e0, fma(e1, e1, e2 * e2)) > bc[g][3]);
+      const uint64_t b = __ballot(keep);
+      if (b == 0) continue;
+      if (keep) cand[g][held[g] + __popcll(b & ((1ull << lane) - 1ull))] = t;
+      held[g] += __popcll(b);
+      __syncthreads();
+      if (held[g] < 64) continue;
+      test(g, 64);
+      held[g] -= 64;
+      const int rest = cand[g][64 + lane];
+      __syncthreads();
+      cand[g][lane] = rest;
+    }
   }
   __syncthreads();
-  if (threadIdx.x < kPB && k0 + threadIdx.x < npan && sc[threadIdx.x]) atomicAdd(&count[k0 + threadIdx.x], sc[threadIdx.x]);
+  for (int g = 0; g < kNearG; ++g)
+    if (held[g] > 0) test(g, held[g]);
+  if (!FILL && k0 + lane < npan) {
+    part[(size_t)blockIdx.y * npan + k] = acc;
+    if (acc) atomicAdd(&count[k], acc);
+  }
 }
 
-// one workgroup per kPB panels, targets in ascending chunks of blockDim
-__global__ void __launch_bounds__(256) nearlist_fill_kernel(int npan, int nt, const double* __restrict__ tx,
-                                                            const double* __restrict__ ball,
-                                                            const int* __restrict__ offs, int* __restrict__ idx) {
-  __shared__ double sb[4 * kPB];
-  __shared__ int base[kPB];
-  __shared__ int wcnt[kPB][4];
-  const int k0 = blockIdx.x * kPB;
-  if (threadIdx.x < 4 * kPB) sb[threadIdx.x] = (k0 + threadIdx.x / 4 < npan) ? ball[4 * k0 + threadIdx.x] : 0.0;
-  if (threadIdx.x < kPB) base[threadIdx.x] = (k0 + threadIdx.x < npan) ? offs[k0 + threadIdx.x] : 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int t0 = 0; t0 < nt; t0 += blockDim.x) {
-    const int t = t0 + threadIdx.x;
-    double x0 = 0.0, x1 = 0.0, x2 = 0.0;
-    if (t < nt) { x0 = tx[3 * (size_t)t]; x1 = tx[3 * (size_t)t + 1]; x2 = tx[3 * (size_t)t + 2]; }
-    uint64_t bal[kPB];
-    for (int q = 0; q < kPB; ++q) {
-      const bool in = (t < nt) && (k0 + q < npan) && in_ball(sb + 4 * q, x0, x1, x2);
-      bal[q] = __ballot(in);
-      if (lane == 0) wcnt[q][wv] = __popcll(bal[q]);
-    }
-    __syncthreads();
-    for (int q = 0; q < kPB; ++q) {
-      if ((bal[q] >> lane) & 1ull) {
-        int pos = base[q];
-        for (int w = 0; w < wv; ++w) pos += wcnt[q][w];
-        pos += __popcll(bal[q] & ((1ull << lane) - 1ull));
-        idx[pos] = t;
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < kPB) {
-      int s = 0;
-      for (int w = 0; w < 4; ++w) s += wcnt[threadIdx.x][w];
-      base[threadIdx.x] += s;
-    }
-    __syncthreads();
-  }
+// targets of a segment: a multiple of 64, so that about 8,192 waves run
+static int near_segment(int npan, int nt) {
+  const int sets = (npan + 63) / 64, most = std::max(1, std::min(64, 8192 / sets));
+  const int chunks = (nt + 63) / 64;
+  return 64 * std::max(1, (chunks + most - 1) / most);
 }
 
-// exclusive scan of n ints into out[0..n] with a single workgroup of 1024 threads
+int nearlist_parts(int npan, int nt) { return nt > 0 ? (nt - 1) / near_segment(npan, nt) + 1 : 0; }
+
+void launch_nearlist(bool fill, int npan, int nt, const double* tx, const double* ball, int* part, int* count,
+                     const int* offs, int* idx, hipStream_t s) {
+  const dim3 grid((npan + 63) / 64, nearlist_parts(npan, nt));
+  hipLaunchKernelGGL(fill ? nearlist_kernel<true> : nearlist_kernel<false>, grid, dim3(64), 0, s, npan, nt,
+                     near_segment(npan, nt), tx, ball, part, count, offs, idx);
+}
+
+// exclusive scan of n ints into out[0..n] with a single workgroup of 1024 threads,
+// 4,096 at a time, the next ones loaded ahead of the scan (a thread's own run of n/1024
+// took 87 us for 50,000, this 30)
 __global__ void __launch_bounds__(1024) scan_kernel(const int* __restrict__ in, int n, int* __restrict__ out) {
-  const int per = (n + blockDim.x - 1) / blockDim.x;
-  const int a = threadIdx.x * per, b = min(n, a + per);
-  int s = 0, total;
-  for (int i = a; i < b; ++i) s += in[i];
-  int acc = block_scan_1024(s, &total);
-  if (threadIdx.x == 0) out[n] = total;
-  for (int i = a; i < b; ++i) { out[i] = acc; acc += in[i]; }
+  int v[4], carry = 0;
+  auto load = [&](int i0) {
+    for (int u = 0; u < 4; ++u) v[u] = i0 + u < n ? in[i0 + u] : 0;
+  };
+  load(4 * threadIdx.x);
+  for (int base = 0; base < n; base += 4096) {
+    const int i0 = base + 4 * threadIdx.x;
+    int w[4], total;
+    for (int u = 0; u < 4; ++u) w[u] = v[u];
+    load(i0 + 4096);
+    int acc = carry + block_scan_1024(w[0] + w[1] + w[2] + w[3], &total);
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + u < n) out[i0 + u] = acc;
+      acc += w[u];
+    }
+    carry += total;
+    __syncthreads();  // the scan's shared sums are read
+  }
+  if (threadIdx.x == 0) out[n] = carry;
 }
 
 

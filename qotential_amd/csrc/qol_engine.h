@@ -84,7 +84,7 @@ struct Engine {
             ev_edge = nullptr, ev_proj = nullptr;
   std::unique_ptr<DeviceTables> tab;
   DevBuf d_sx, d_snx, d_sw, d_rts, d_rps, d_sxbd, d_rv;
-  DevBuf d_tx, d_nball, d_cnt, d_offs, d_tidx;
+  DevBuf d_tx, d_nball, d_npart, d_cnt, d_offs, d_tidx;
   DevBuf d_label, d_ppanel, d_nrrq, d_lcount, d_lstart, d_ltot, d_lpairs, d_wout, d_val, d_omega, d_ias;
   DevBuf d_abucket, d_apairs, d_acnt;  // adaptive levels: tree cut per pair, pairs sorted by cut, cut counts
   DevBuf d_lgeo, d_balls, d_pq, d_w1, d_oe, d_root, d_eorder, d_vt;

@@ -142,9 +142,11 @@ void launch_direct_split(LevelArgs A, const int* lpairs, const int* ltot, const 
 
 __global__ void nearlist_prep_kernel(int npan, int h, const double* sx, const double* sw, const double* corner,
                                      double diam, double* ball);
-__global__ void nearlist_count_kernel(int npan, int nt, const double* tx, const double* ball, int* count);
-__global__ void nearlist_fill_kernel(int npan, int nt, const double* tx, const double* ball, const int* offs,
-                                     int* idx);
+// the brute-force near list's counts (part: nearlist_parts x npan; count zeroed before)
+// or, with fill, its entries
+int nearlist_parts(int npan, int nt);
+void launch_nearlist(bool fill, int npan, int nt, const double* tx, const double* ball, int* part, int* count,
+                     const int* offs, int* idx, hipStream_t s);
 __global__ void scan_kernel(const int* in, int n, int* out);
 
 __global__ void naive_apply_kernel(int nnz, int h, const int* tidx, const int* ppanel, const double* tx,
