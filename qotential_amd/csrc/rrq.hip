@@ -919,7 +919,6 @@ __global__ void __launch_bounds__(256) rrq_msl_inverse_kernel(RRQTables T, RRQPa
 // rows already pivoted by a register-resident Gauss-Jordan (h <= 128)
 struct RowMask {
   unsigned long long lo = 0ull, hi = 0ull;
-  __device__ __forceinline__ bool has(int r) const { return ((r < 64 ? lo : hi) >> (r & 63)) & 1ull; }
   __device__ __forceinline__ void add(int r) {
     if (r < 64) lo |= 1ull << r;
     else hi |= 1ull << (r & 63);
@@ -927,6 +926,57 @@ struct RowMask {
   // lowest row not yet pivoted
   __device__ __forceinline__ int first_free() const { return ~lo ? __builtin_ctzll(~lo) : 64 + __builtin_ctzll(~hi); }
 };
+
+// largest of 64 lanes' values, in every lane
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+#define QOL_MAX_DPP(CTRL_, ROWS_) \
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL_, ROWS_, 0xf, false))
+  QOL_MAX_DPP(0x111, 0xf);  // row_shr 1, 2, 4, 8: the last lane of each 16 holds theirs
+  QOL_MAX_DPP(0x112, 0xf);
+  QOL_MAX_DPP(0x114, 0xf);
+  QOL_MAX_DPP(0x118, 0xf);
+  QOL_MAX_DPP(0x142, 0xa);  // row_bcast 15, 31
+  QOL_MAX_DPP(0x143, 0xc);
+#undef QOL_MAX_DPP
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The pivot: the unused row with the largest v, ties to the lower row; lane i holds
+// rows i and, with TWO, i + 64 (v1).  Non-negative doubles compare like integers, so
+// the high words' maximum decides, the low words' among the lanes it leaves.  No
+// candidate is left only with NaN entries: then the lowest unused row, so that every
+// row is pivoted once and every index stays in range.  second: the lane's row i + 64
+// is the larger of its two.
+template <bool TWO>
+__device__ __forceinline__ int pivot_row(const RowMask& used, int h, int lane, double v0, double v1, bool& second) {
+  const bool c0 = (lane < h) & !((used.lo >> lane) & 1ull) & (v0 >= 0.0);
+  second = false;
+  if constexpr (TWO) {
+    const bool c1 = (lane + 64 < h) & !((used.hi >> lane) & 1ull) & (v1 >= 0.0);
+    second = c1 & (!c0 | (v1 > v0));
+  }
+  const double v = second ? v1 : v0;
+  const unsigned hi = c0 | second ? (unsigned)__double2hiint(v) + 1u : 0u;
+  const unsigned m = wave_max(hi);
+  if (m == 0u) return used.first_free();
+  unsigned long long tied = __ballot(hi == m);
+  if (tied & (tied - 1ull)) {  // uniform
+    const unsigned lo = (unsigned)__double2loint(v);
+    tied = __ballot((hi == m) & (lo == wave_max(hi == m ? lo : 0u)));
+  }
+  if constexpr (TWO) {
+    const unsigned long long low = tied & __ballot(!second);
+    return low ? __builtin_ctzll(low) : 64 + __builtin_ctzll(tied);
+  }
+  return __builtin_ctzll(tied);
+}
+
+// orders a wave's LDS stores before its later loads
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // X = Fq^{-1} for the h x h pure-quaternion matrix Fq by Gauss-Jordan, the
 // matrix in registers of NW waves (one panel per workgroup).  Lane (ly, lx) of
@@ -937,12 +987,20 @@ struct RowMask {
 // afterwards (the unit column of the row pivoted at step s, zero in every other
 // row until then), so h slots carry the live window (kk, h+kk] at every step.
 // Pivoting is implicit (no row moves): the unused row with the largest |A_r,kk|
-// wins, ties to the lower row.  Column kk lies in one wave: it finds the pivot
-// and publishes the column with a zero in the pivot row (so the rank-1 update,
-// the same in every lane, leaves that row alone; it is scaled by the inverse
-// pivot afterwards).  Each wave already holds its part of the pivot row, so one
-// workgroup barrier per step suffices (LDS double-buffered by step parity).
+// wins, ties to the lower row.  Column kk lies in one wave: it publishes the column,
+// reads it back a row per lane, finds the pivot and its inverse and puts -1 in the
+// pivot row's place.  Each wave holds its part of the pivot row: it publishes that
+// and clears it, so that the rank-1 update, the same in every lane, leaves
+// 0 - (-1) (pivot^-1 row) there.  One workgroup barrier per step suffices (LDS
+// double-buffered by step parity).
 // Afterwards row piv[k] holds row k of X with slot s holding column piv[s].
+//
+// Bound by a step's chain (column, pivot, barrier, row, update) with two or three
+// panels' waves a SIMD to hide it, and at order 8 a quarter by loads and scattered
+// stores.  The pivot from shuffles among the column's own lanes, the inverse in every
+// wave and a separate pass over the pivot row took 1.58 ms for 14,250 panels of order 8
+// (206 VGPRs), this 0.95 (160); 1,600 of order 12: 1.90, now 1.27; the real inverses
+// 0.33 and 0.54, now 0.17 and 0.29.
 template <int RL, int RA, int CL, int CB, int NW>
 __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, RRQPanels P, int npan,
                                                                    const int* __restrict__ nrrq) {
@@ -952,7 +1010,7 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
   if (nrrq && nrrq[k] == 0) return;  // null: every panel
   const int h = T.h;
   constexpr int NRW = RL * RA, NSL = CL * CB;
-  __shared__ double colq[2][4 * NRW], rowq[2][4 * NSL], pivel[2][4];
+  __shared__ double colq[2][4 * NRW], rowq[2][4 * NSL], pinvs[2][4];
   __shared__ int pivs[2], piv[NRW], pos[NRW];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const bool act = lane < RL * CL;
@@ -971,6 +1029,7 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
         e[1] = q[0]; e[2] = q[1]; e[3] = q[2];
       }
     }
+  const int lyr = act ? ly : -NRW - 1;  // lanes past the grid own no row
   RowMask used;
   for (int kk = 0; kk < h; ++kk) {
     const int buf = kk & 1, kt = kk % CL, kbg = kk / CL;
@@ -978,95 +1037,74 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
     double* cq = colq[buf];
     double* rq = rowq[buf];
     if (wv == ow) {  // uniform
-      const bool own = act & (lx == kt);
-      double bv = -1.0;
-      int bi = NRW;
+      // column kk by row, and slot kk turned into right column h+kk: zero, and 1 in
+      // the pivot row, which goes straight into rq below
+      if (act & (lx == kt)) {
 #pragma unroll
-      for (int b = 0; b < CW; ++b) {
-        if (b != kb) continue;  // uniform
+        for (int b = 0; b < CW; ++b) {
+          if (b != kb) continue;  // uniform
 #pragma unroll
-        for (int a = 0; a < RA; ++a) {
-          const int r = ly + RL * a;
-          const double* e = A[a][b];
-          const double v = e[0] * e[0] + e[1] * e[1] + e[2] * e[2] + e[3] * e[3];
-          const bool t = own & (r < h) & !used.has(r) & (v > bv);
-          bv = t ? v : bv;
-          bi = t ? r : bi;
-        }
-      }
-      // best of the RL owner lanes (lane ids kt + CL*t)
-      int p = NRW;
-      {
-        double pv = -1.0;
+          for (int a = 0; a < RA; ++a)
 #pragma unroll
-        for (int t = 0; t < RL; ++t) {
-          const double v = __shfl(bv, kt + CL * t, 64);
-          const int i = __shfl(bi, kt + CL * t, 64);
-          const bool tk = (v > pv) | ((v == pv) & (i < p));
-          pv = tk ? v : pv;
-          p = tk ? i : p;
-        }
-      }
-      p = __builtin_amdgcn_readfirstlane(p);
-      // no candidate only with NaN entries: take the lowest unused row, so every
-      // row is pivoted once and every index stays in range
-      if (p >= h) p = used.first_free();
-      const int pa = p / RL;
-      const bool prow = act & (ly == p % RL);
-      if (lane == 0) pivs[buf] = p;
-      // column kk by row (zero in the pivot row), the pivot itself, and slot kk
-      // turned into right column h+kk: zero, 1 in the pivot row
-#pragma unroll
-      for (int b = 0; b < CW; ++b) {
-        if (b != kb) continue;  // uniform
-#pragma unroll
-        for (int a = 0; a < RA; ++a) {
-          double* e = A[a][b];
-          if (own) {
-            const int r = ly + RL * a;
-            const bool isp = (a == pa) & prow;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cq[4 * r + q] = isp ? 0.0 : e[q];
-            if (isp) {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) pivel[buf][q] = e[q];
+            for (int q = 0; q < 4; ++q) {
+              cq[4 * (ly + RL * a) + q] = A[a][b][q];
+              A[a][b][q] = 0.0;
             }
-            e[0] = isp ? 1.0 : 0.0;
-            e[1] = e[2] = e[3] = 0.0;
-          }
         }
+      }
+      wave_lds_fence();
+      double e[4], f[4], v1 = -1.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) e[q] = cq[4 * (lane < NRW ? lane : NRW - 1) + q];
+      const double v0 = e[0] * e[0] + e[1] * e[1] + e[2] * e[2] + e[3] * e[3];
+      if constexpr (NRW > 64) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) f[q] = cq[4 * (lane + 64 < NRW ? lane + 64 : NRW - 1) + q];
+        v1 = f[0] * f[0] + f[1] * f[1] + f[2] * f[2] + f[3] * f[3];
+      }
+      bool second;
+      const int p = pivot_row<(NRW > 64)>(used, h, lane, v0, v1, second);
+      if constexpr (NRW > 64) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e[q] = second ? f[q] : e[q];
+      }
+      const double in2 = 1.0 / (second ? v1 : v0);
+      if (lane == (p & 63)) {
+        double* c = cq + 4 * p;
+        c[0] = -1.0;
+        c[1] = c[2] = c[3] = 0.0;
+        pinvs[buf][0] = e[0] * in2;
+        pinvs[buf][1] = -e[1] * in2;
+        pinvs[buf][2] = -e[2] * in2;
+        pinvs[buf][3] = -e[3] * in2;
+        pivs[buf] = p;
+        piv[kk] = p;
       }
     }
     __syncthreads();
-    const int p = __builtin_amdgcn_readfirstlane(pivs[buf]);
-    used.add(p);
-    if (threadIdx.x == 0) piv[kk] = p;
-    const int pa = p / RL;
-    const bool prow = act & (ly == p % RL);
+    const int p = pivs[buf];
     // this wave's part of the pivot row, by slot (wave-local exchange)
 #pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      if (a != pa) continue;  // uniform
-      if (prow) {
+    for (int a = 0; a < RA; ++a)
+      if (p - lyr == RL * a) {
 #pragma unroll
         for (int b = 0; b < CW; ++b) {
           const int c = lx + CL * (wv * CW + b);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) rq[4 * c + q] = A[a][b][q];
+          for (int q = 0; q < 4; ++q) {
+            rq[4 * c + q] = A[a][b][q];
+            A[a][b][q] = 0.0;
+          }
         }
       }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if ((wv == ow) & (lane == 0)) rq[4 * kk] = 1.0;
+    wave_lds_fence();
     double pinv[4];
-    {
-      const double* e = pivel[buf];
-      const double in2 = 1.0 / (e[0] * e[0] + e[1] * e[1] + e[2] * e[2] + e[3] * e[3]);
-      pinv[0] = e[0] * in2; pinv[1] = -e[1] * in2; pinv[2] = -e[2] * in2; pinv[3] = -e[3] * in2;
-    }
-    // every other row: A_r -= A_r,kk * (pivot^-1 * pivot row); the normalised
-    // row entries of this wave's slots first, then one column value per row
+#pragma unroll
+    for (int q = 0; q < 4; ++q) pinv[q] = pinvs[buf][q];
+    used.add(__builtin_amdgcn_readfirstlane(p));
+    // every row: A_r -= A_r,kk * (pivot^-1 * pivot row); the normalised row entries of
+    // this wave's slots first, then one column value per row
     double nq[CW][4];
 #pragma unroll
     for (int b = 0; b < CW; ++b) qmul_fma(pinv, rq + 4 * (lx + CL * (wv * CW + b)), nq[b]);
@@ -1076,20 +1114,6 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
       const double cv[4] = {c[0], c[1], c[2], c[3]};
 #pragma unroll
       for (int b = 0; b < CW; ++b) qsub_mul(A[a][b], cv, nq[b]);
-    }
-    // the pivot row: pivot^-1 * row
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      if (a != pa) continue;  // uniform
-      if (prow) {
-#pragma unroll
-        for (int b = 0; b < CW; ++b) {
-          double nq[4];
-          qmul_fma(pinv, A[a][b], nq);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) A[a][b][q] = nq[q];
-        }
-      }
     }
   }
   __syncthreads();
@@ -1110,8 +1134,8 @@ __global__ void __launch_bounds__(64 * NW) rrq_quat_inverse_kernel(RRQTables T, 
 }
 
 // B = (Msl^T)^{-1} by Gauss-Jordan in the registers of one wave per panel, the
-// real counterpart of rrq_quat_inverse_kernel (same lane grid, slot reuse,
-// implicit pivoting with ties to the lower row, zeroed pivot-row column entry).
+// real counterpart of rrq_quat_inverse_kernel (same lane grid, slot reuse, implicit
+// pivoting with ties to the lower row, -1 for the pivot row's column entry).
 // The system matrix is A(r, c) = Msl[r + h*c]; output B transposed, B(kx, j) at
 // Binv[j*h + kx].
 template <int RL, int RA, int CL, int CB>
@@ -1136,81 +1160,54 @@ __global__ void __launch_bounds__(64) rrq_real_inverse_kernel(RRQTables T, RRQPa
       const int r = ly + RL * a, c = lx + CL * b;
       A[a][b] = (act & (r < h) & (c < h)) ? MS[r + (size_t)h * c] : 0.0;
     }
+  const int lyr = act ? ly : -NRW - 1;  // lanes past the grid own no row
   RowMask used;
   for (int kk = 0; kk < h; ++kk) {
     const int buf = kk & 1, kt = kk % CL, kb = kk / CL;
-    const bool own = act & (lx == kt);
-    double bv = -1.0;
-    int bi = NRW;
+    double* cr = colr[buf];
+    double* rr = rowr[buf];
+    if (act & (lx == kt)) {
 #pragma unroll
-    for (int b = 0; b < CB; ++b) {
-      if (b != kb) continue;  // uniform
+      for (int b = 0; b < CB; ++b) {
+        if (b != kb) continue;  // uniform
 #pragma unroll
-      for (int a = 0; a < RA; ++a) {
-        const int r = ly + RL * a;
-        const double v = fabs(A[a][b]);
-        const bool t = own & (r < h) & !used.has(r) & (v > bv);
-        bv = t ? v : bv;
-        bi = t ? r : bi;
-      }
-    }
-    int p = NRW;
-    {
-      double pv = -1.0;
-#pragma unroll
-      for (int t = 0; t < RL; ++t) {
-        const double v = __shfl(bv, kt + CL * t, 64);
-        const int i = __shfl(bi, kt + CL * t, 64);
-        const bool tk = (v > pv) | ((v == pv) & (i < p));
-        pv = tk ? v : pv;
-        p = tk ? i : p;
-      }
-    }
-    p = __builtin_amdgcn_readfirstlane(p);
-    if (p >= h) p = used.first_free();  // NaN entries only
-    used.add(p);
-    if (lane == 0) piv[kk] = p;
-    const int pa = p / RL;
-    const bool prow = act & (ly == p % RL);
-#pragma unroll
-    for (int b = 0; b < CB; ++b) {
-      if (b != kb) continue;  // uniform
-#pragma unroll
-      for (int a = 0; a < RA; ++a) {
-        if (own) {
-          const bool isp = (a == pa) & prow;
-          colr[buf][ly + RL * a] = isp ? 0.0 : A[a][b];
-          if (isp) pivel[buf] = A[a][b];
-          A[a][b] = isp ? 1.0 : 0.0;
+        for (int a = 0; a < RA; ++a) {
+          cr[ly + RL * a] = A[a][b];
+          A[a][b] = 0.0;
         }
       }
     }
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      if (a != pa) continue;  // uniform
-      if (prow) {
-#pragma unroll
-        for (int b = 0; b < CB; ++b) rowr[buf][lx + CL * b] = A[a][b];
-      }
+    wave_lds_fence();
+    const double e0 = cr[lane < NRW ? lane : NRW - 1];
+    const double e1 = NRW > 64 ? cr[lane + 64 < NRW ? lane + 64 : NRW - 1] : 0.0;
+    bool second;
+    const int p = pivot_row<(NRW > 64)>(used, h, lane, fabs(e0), fabs(e1), second);
+    used.add(p);
+    if (lane == (p & 63)) {
+      cr[p] = -1.0;
+      pivel[buf] = 1.0 / (second ? e1 : e0);
+      piv[kk] = p;
     }
-    __syncthreads();  // one wave: orders the LDS stores before the loads
-    const double ip = 1.0 / pivel[buf];
+#pragma unroll
+    for (int a = 0; a < RA; ++a)
+      if (p - lyr == RL * a) {
+#pragma unroll
+        for (int b = 0; b < CB; ++b) {
+          rr[lx + CL * b] = A[a][b];
+          A[a][b] = 0.0;
+        }
+      }
+    if (lane == 0) rr[kk] = 1.0;
+    wave_lds_fence();
+    const double ip = pivel[buf];
     double nr[CB];
 #pragma unroll
-    for (int b = 0; b < CB; ++b) nr[b] = ip * rowr[buf][lx + CL * b];
+    for (int b = 0; b < CB; ++b) nr[b] = ip * rr[lx + CL * b];
 #pragma unroll
     for (int a = 0; a < RA; ++a) {
-      const double c = colr[buf][act ? ly + RL * a : 0];  // lanes past the grid idle
+      const double c = cr[act ? ly + RL * a : 0];  // lanes past the grid idle
 #pragma unroll
       for (int b = 0; b < CB; ++b) A[a][b] = fma(-c, nr[b], A[a][b]);
-    }
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      if (a != pa) continue;  // uniform
-      if (prow) {
-#pragma unroll
-        for (int b = 0; b < CB; ++b) A[a][b] *= ip;
-      }
     }
   }
   __syncthreads();
@@ -1324,8 +1321,11 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
   const char* fu = std::getenv("QOL_SOLVE_FUSED");
   const bool fused = variant == 1 || (variant == 0 && fu && fu[0] == '1');
   if (h <= 78 && !fused) {
-    // lane grid per order (rows RL x RA, slots CL x CB) and waves, about 48 quaternion
-    // entries per lane
+    // lane grid per order (rows RL x RA, slots CL x CB) and waves.  Measured (us): order
+    // 8, 14,250 panels, 2 waves 953 (4: 1078, 9 x 4 rows: 940-998); order 9 of 24 x 60, 3
+    // waves 469 (2: 491, 6: 650); 10: 8 waves 862 (4: 943, 7: 884); 11: 4 waves of three
+    // slot groups, so that two panels share a CU, 1440 (6: 2092); 12: 10 waves of 16 x 5
+    // rows 1279 (8 of 12 x 7: 1318, 7: 1361)
 #define QOL_QINV(RL_, RA_, CL_, CB_, NW_)                                                                \
   hipLaunchKernelGGL((rrq_real_inverse_kernel<RL_, RA_, CL_, CB_>), dim3(npan), dim3(64), 0, s, T, P, npan, nrrq); \
   hipLaunchKernelGGL((rrq_quat_inverse_kernel<RL_, RA_, CL_, CB_, NW_>), dim3(npan), dim3(64 * NW_), 0, s, T, P,   \
@@ -1338,9 +1338,9 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
     else if (h <= 28) { QOL_QINV(4, 7, 16, 2, 2); }
     else if (h <= 36) { QOL_QINV(6, 6, 10, 4, 2); }
     else if (h <= 45) { QOL_QINV(8, 6, 8, 6, 3); }
-    else if (h <= 55) { QOL_QINV(9, 7, 7, 8, 4); }
-    else if (h <= 66) { QOL_QINV(10, 7, 6, 12, 6); }
-    else { QOL_QINV(12, 7, 5, 16, 8); }
+    else if (h <= 55) { QOL_QINV(9, 7, 7, 8, 8); }
+    else if (h <= 66) { QOL_QINV(10, 7, 6, 12, 4); }
+    else { QOL_QINV(16, 5, 4, 20, 10); }
 #undef QOL_QINV
   } else if (rpt <= 3 && cpt <= 5) {
     hipLaunchKernelGGL((rrq_panel_solve_kernel<3, 5>), dim3(npan), dim3(256), 0, s, T, P, npan, nrrq);
