@@ -118,6 +118,20 @@ __global__ void __launch_bounds__(256) naive_apply_list_kernel(const int* __rest
   if (live && part == 0) val[j] = acc;
 }
 
+// The weights by column, out(j, c) at c*nnz + j from rows of 2h per pair: tiles of 32 x
+// 32 through LDS, so that both sides move whole lines and the host, which looped over
+// the rows before, copies two finished blocks
+__global__ void __launch_bounds__(256) weight_columns_kernel(int nnz, int m2, const double* __restrict__ wout,
+                                                             double* __restrict__ cols) {
+  __shared__ double tile[32][33];
+  const int j0 = blockIdx.x * 32, c0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  for (int r = y; r < 32; r += 8)
+    if (j0 + r < nnz && c0 + x < m2) tile[r][x] = wout[(size_t)(j0 + r) * m2 + c0 + x];
+  __syncthreads();
+  for (int c = y; c < 32; c += 8)
+    if (j0 + x < nnz && c0 + c < m2) cols[(size_t)(c0 + c) * nnz + j0 + x] = tile[x][c];
+}
+
 // COO triplets of getnearquad_lap_rrq: out = (tcxi(k)-1)*h + (j-1)*m + i (1-based)
 __global__ void __launch_bounds__(256) triplet_kernel(int nnz, int h, const int* __restrict__ tidx,
                                                       const int* __restrict__ ppanel, const int* __restrict__ trow,

@@ -9,7 +9,7 @@
 //   qol_lap3dsdlpmat_levels_mex_     src/patch_refine_mex.f90:211-223
 //   qol_clear_patch_levels_mex_      src/patch_refine_mex.f90:226-233
 //   qol_clear_patch_levels_all_mex_  src/patch_refine_mex.f90:236-242
-// Each runs on the GPU through a short-lived engine; the batched engine API
+// Each runs on the GPU through an engine kept between calls; the batched engine API
 // (qol_engine_*) keeps geometry, targets and weights resident across calls.
 #include <hip/hip_runtime.h>
 
@@ -93,6 +93,60 @@ Engine& panel_engine(int64_t p, int64_t ichart, const double* sx, const double* 
   level_mode(&ad, &sq);
   cache->e->set_level_mode(ad, sq);
   return *cache->e;
+}
+
+// One whole-surface engine for qol_getnearquad_lap_rrq_mex_, kept between calls of one
+// order, panel count and device: streams, tables and buffers, nothing of a call's data.
+// Making and freeing them took 6 of a 10 ms call for 944 panels of order 4 (150,096
+// pairs; freeing 260 MB alone 4.3).  A call takes the engine out of the slot, so that no
+// two threads hold it, and leaves its own there afterwards if that holds at most 1 GiB;
+// an engine that another replaces, that is larger or whose call failed is freed.  Never
+// destroyed at exit, like the per-panel engines.
+struct SurfaceEngine {
+  std::unique_ptr<Engine> e;
+  int device = -1;
+  int64_t p = -1, npan = -1;
+  long long bytes = 0;
+};
+struct SurfaceSlot {
+  std::mutex mu;
+  SurfaceEngine s;
+};
+SurfaceSlot& surface_slot() {
+  static SurfaceSlot* slot = new SurfaceSlot;
+  return *slot;
+}
+constexpr long long kSurfaceKeep = 1ll << 30;
+
+template <class F>
+void with_surface_engine(int64_t p, int64_t npan, const double* sx, const double* snx, const double* sw,
+                         const double* rts, const double* rps, F&& call) {
+  SurfaceEngine mine;
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  bool ad = false, sq = true;
+  level_mode(&ad, &sq);
+  {
+    std::lock_guard<std::mutex> g(surface_slot().mu);
+    SurfaceEngine& s = surface_slot().s;
+    if (s.e && s.device == dev && s.p == p && s.npan == npan) std::swap(mine, s);
+  }
+  const long long before = thread_device_bytes();
+  if (mine.e) {
+    mine.e->set_surface(sx, snx, sw, rts, rps, nullptr, nullptr, false);
+  } else {
+    mine.e.reset(new Engine(p, npan, sx, snx, sw, rts, rps, 0, nullptr, nullptr, false, nullptr, sq));
+    mine.device = dev;
+    mine.p = p;
+    mine.npan = npan;
+  }
+  mine.e->set_level_mode(ad, sq);
+  call(*mine.e);
+  mine.bytes += thread_device_bytes() - before;
+  if (mine.bytes <= kSurfaceKeep) {
+    std::lock_guard<std::mutex> g(surface_slot().mu);
+    std::swap(mine, surface_slot().s);
+  }
 }
 
 }  // namespace
@@ -509,25 +563,21 @@ void qol_getnearquad_lap_rrq_mex_(const int64_t* npan, const int64_t* nterms, co
     const int64_t np_ = *npan, nt = *ntcx;
     if (tcxi[0] != 1) throw std::runtime_error("tcxi(1) must be 1");
     if ((tcxi[np_] - 1) * h != *nnz) throw std::runtime_error("nnz must equal (tcxi(npan+1)-1)*hdim");
-    bool ad = false, sq = true;
-    level_mode(&ad, &sq);
-    Engine e(p, np_, sx, snx, sw, rts, rps, 0, nullptr, nullptr, false, nullptr, sq);
-    e.set_level_mode(ad, sq);
-    e.set_targets(nt, tcx, false);
     std::vector<int64_t> offs(np_ + 1), idx(tcxi[np_] - 1);
     for (int64_t k = 0; k <= np_; ++k) offs[k] = tcxi[k] - 1;
     for (size_t j = 0; j < idx.size(); ++j) idx[j] = (int64_t)j + 1;
-    e.set_pairs(offs.data(), idx.data());
-    e.eval((*iside % 10) == 0 ? 1 : 0, 1e-10, false);
-    e.triplets(tcxrow, sparsei, sparsej, sparsevs, sparsevd);
-    {
+    with_surface_engine(p, np_, sx, snx, sw, rts, rps, [&](Engine& e) {
+      e.set_targets(nt, tcx, false);
+      e.set_pairs(offs.data(), idx.data());
+      e.eval((*iside % 10) == 0 ? 1 : 0, 1e-10, false);
+      e.triplets(tcxrow, sparsei, sparsej, sparsevs, sparsevd);
       double st = 0.0;
       const int64_t n = e.projection_unconverged(&st);
       set_unconverged(n, st);
-    }
-    double ms[10];
-    e.stage_ms(ms);
-    add_timeinfo(ms, timeinfo);
+      double ms[10];
+      e.stage_ms(ms);
+      add_timeinfo(ms, timeinfo);
+    });
   });
 }
 

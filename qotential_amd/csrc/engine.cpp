@@ -43,12 +43,32 @@ Arena*& thread_arena() {
   return a;
 }
 
-DevBuf::~DevBuf() {
-  if (ptr && owned) (void)hipFree(ptr);
+long long& thread_device_bytes() {
+  static thread_local long long n = 0;
+  return n;
+}
+
+PinnedBuf::~PinnedBuf() {
+  if (ptr) (void)hipHostFree(ptr);
+}
+void PinnedBuf::alloc(size_t b) {
+  if (b <= bytes) return;
+  if (ptr) (void)hipHostFree(ptr);
+  ptr = nullptr;
+  bytes = 0;
+  HIPCHK(hipHostMalloc(&ptr, b, hipHostMallocDefault));
+  bytes = b;
+}
+
+DevBuf::~DevBuf() { release(); }
+void DevBuf::release() {
+  if (!ptr || !owned) return;
+  (void)hipFree(ptr);
+  thread_device_bytes() -= (long long)bytes;
 }
 void DevBuf::alloc(size_t b) {
   if (b <= bytes && ptr) return;
-  if (ptr && owned) (void)hipFree(ptr);
+  release();
   ptr = nullptr;
   bytes = 0;
   owned = false;
@@ -66,6 +86,7 @@ void DevBuf::alloc(size_t b) {
   HIPCHK(hipMalloc(&ptr, b));
   bytes = b;
   owned = true;
+  thread_device_bytes() += (long long)b;
 }
 
 void StreamSet::create_one_stream() {
@@ -788,29 +809,55 @@ void Engine::pair_features(float* feat) {
 
 void Engine::get_weights(double* As, double* Ad, i64* label, double* Omega, double* Ias) {
   if (!evaluated) throw std::runtime_error("weights not evaluated");
-  HIPCHK(hipStreamSynchronize(stream));
+  if (Omega && nnz > 0 && !have_omega) throw std::runtime_error("Omega was not requested at eval");
+  if (Ias && nnz > 0 && !have_omega) throw std::runtime_error("Ias was not requested at eval");
+  struct Part { double* dst; const double* src; size_t n; };
+  std::vector<Part> parts;
+  const size_t n = (size_t)h * (nnz > 0 ? nnz : 0);
   if ((As || Ad) && nnz > 0) {
-    std::vector<double> w(2 * (size_t)h * nnz);
-    HIPCHK(hipMemcpy(w.data(), d_wout.ptr, sizeof(double) * 2 * h * (size_t)nnz, hipMemcpyDeviceToHost));
-    // column-major (nnz, h)
-    for (i64 j = 0; j < nnz; ++j)
-      for (int c = 0; c < h; ++c) {
-        if (As) As[j + (size_t)nnz * c] = w[(size_t)j * 2 * h + c];
-        if (Ad) Ad[j + (size_t)nnz * c] = w[(size_t)j * 2 * h + h + c];
+    // column-major (nnz, h); the moment vectors are used up, and their buffer is the larger
+    d_vt.alloc(sizeof(double) * 2 * n);
+    double* cols = (double*)d_vt.ptr;
+    hipLaunchKernelGGL(weight_columns_kernel, dim3(blocks(nnz, 32), blocks(2 * h, 32)), dim3(256), 0, stream, (int)nnz,
+                       2 * h, (const double*)d_wout.ptr, cols);
+    HIPCHK(hipGetLastError());
+    parts.push_back({As, cols, n});
+    parts.push_back({Ad, cols + n, n});
+  }
+  if (nnz > 0) {
+    parts.push_back({Omega, (const double*)d_omega.ptr, 4 * n});
+    parts.push_back({Ias, (const double*)d_ias.ptr, (size_t)nnz});
+  }
+  size_t total = 0;
+  for (const Part& q : parts) total += q.dst ? sizeof(double) * q.n : 0;
+  // A copy into the caller's pages is pinned and waited for one at a time; memory kept
+  // pinned takes all of them behind one wait (one panel, 124 targets of order 4: 437 to
+  // 386 us a call, 1,501 of order 6: 591 to 564).  Large results are bound by the copy
+  // itself and would pass through memory twice.
+  if (total > 0 && total <= kPinned && !thread_arena()) {
+    pinned.alloc(kPinned);
+    char* at = (char*)pinned.ptr;
+    for (const Part& q : parts)
+      if (q.dst) {
+        HIPCHK(hipMemcpyAsync(at, q.src, sizeof(double) * q.n, hipMemcpyDeviceToHost, stream));
+        at += sizeof(double) * q.n;
       }
+    HIPCHK(hipStreamSynchronize(stream));
+    at = (char*)pinned.ptr;
+    for (const Part& q : parts)
+      if (q.dst) {
+        std::memcpy(q.dst, at, sizeof(double) * q.n);
+        at += sizeof(double) * q.n;
+      }
+  } else {
+    HIPCHK(hipStreamSynchronize(stream));
+    for (const Part& q : parts)
+      if (q.dst) HIPCHK(hipMemcpy(q.dst, q.src, sizeof(double) * q.n, hipMemcpyDeviceToHost));
   }
   if (label && nnz > 0) {
     std::vector<int8_t> l(nnz);
     HIPCHK(hipMemcpy(l.data(), d_label.ptr, nnz, hipMemcpyDeviceToHost));
     for (i64 j = 0; j < nnz; ++j) label[j] = l[j];
-  }
-  if (Omega && nnz > 0) {
-    if (!have_omega) throw std::runtime_error("Omega was not requested at eval");
-    HIPCHK(hipMemcpy(Omega, d_omega.ptr, sizeof(double) * 4 * (size_t)h * nnz, hipMemcpyDeviceToHost));
-  }
-  if (Ias && nnz > 0) {
-    if (!have_omega) throw std::runtime_error("Ias was not requested at eval");
-    HIPCHK(hipMemcpy(Ias, d_ias.ptr, sizeof(double) * (size_t)nnz, hipMemcpyDeviceToHost));
   }
 }
 
@@ -921,7 +968,6 @@ void Engine::triplets(const i64* trow, i64* si, i64* sj, double* vs, double* vd)
   if (!evaluated) throw std::runtime_error("weights not evaluated");
   std::vector<int> tr((size_t)(nt > 0 ? nt : 1), 0);
   for (int t = 0; t < nt; ++t) tr[t] = (int)trow[t];
-  DevBuf d_tr, d_si, d_sj, d_vs, d_vd;
   upload(d_tr, tr.data(), tr.size(), stream);
   const size_t n = (size_t)nnz * h;
   d_si.alloc(sizeof(int64_t) * (n ? n : 1)); d_sj.alloc(sizeof(int64_t) * (n ? n : 1));

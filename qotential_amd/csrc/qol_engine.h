@@ -37,7 +37,23 @@ struct DevBuf {
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf();
   void alloc(size_t b);
+
+ private:
+  void release();
 };
+
+struct PinnedBuf {  // host memory the GPU copies into directly
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  PinnedBuf() = default;
+  PinnedBuf(const PinnedBuf&) = delete;
+  PinnedBuf& operator=(const PinnedBuf&) = delete;
+  ~PinnedBuf();
+  void alloc(size_t b);
+};
+
+// device bytes the calling thread's buffers have taken from and given back to hipMalloc
+long long& thread_device_bytes();
 
 struct DeviceTables {
   int h = 0, ntot = 0, nsubtot = 0;
@@ -92,6 +108,9 @@ struct Engine {
   bool projected = false;      // the last eval ran the projection (it had RRQ pairs to run)
   DevBuf d_frame, d_edge, d_bX, d_cx, d_basis, d_Fq, d_Msl, d_Fn, d_X, d_G, d_Binv;
   DevBuf d_ub, d_ubn, d_u, d_tcount, d_toffs, d_tcur, d_tpairs;
+  DevBuf d_tr, d_si, d_sj, d_vs, d_vd;  // COO triplets: rows of the targets, the four columns
+  static constexpr size_t kPinned = 4 << 20;
+  PinnedBuf pinned;            // results of a call on their way to the caller's memory
   DevBuf d_fsrc, d_fpart;     // far field: packed sources, per-chunk sums
   RRQPanels RP{};
 

@@ -152,6 +152,7 @@ __global__ void scan_kernel(const int* in, int n, int* out);
 __global__ void naive_apply_kernel(int nnz, int h, const int* tidx, const int* ppanel, const double* tx,
                                    const double* sx, const double* snx, const double* sw, const double* ub,
                                    const double* ubn, const double* wout, double* val);
+__global__ void weight_columns_kernel(int nnz, int m2, const double* wout, double* cols);
 __global__ void naive_apply_list_kernel(const int* lpairs, const int* ltot, int first, int last, int h,
                                         const int* tidx, const int* ppanel, const double* tx, const double* sx,
                                         const double* snx, const double* sw, const double* ub, const double* ubn,
