@@ -3,6 +3,8 @@
 // Reference: naive block + apply   stellarator_grf_core_mod.f90:847-870
 //            fixed-order scatter   stellarator_grf_core_mod.f90:895-899
 //            COO triplets          lap3d_close_mod.f90:935-956
+#include <algorithm>
+
 #include "qol_kernels.h"
 
 namespace qol {
@@ -22,31 +24,81 @@ __device__ __forceinline__ void naive_entries(double x0, double x1, double x2, c
   }
 }
 
-// val(pair) = sum_i (S - S_naive)_i ubn_i - (K - K_naive)_i ub_i, i over the
-// panel's h nodes, left to right as in the reference loop.
-// near-correction value of pair j, part p of 4 (nodes p, p+4, ...):
-// sum_i (S - S_naive)_i ubn_i - (K - K_naive)_i ub_i
-__device__ __forceinline__ double pair_correction_part(int j, int part, int h, const int* __restrict__ tidx,
-                                                       const int* __restrict__ ppanel,
-                                                       const double* __restrict__ tx,
-                                                       const double* __restrict__ sx,
-                                                       const double* __restrict__ snx,
-                                                       const double* __restrict__ sw,
-                                                       const double* __restrict__ ub,
-                                                       const double* __restrict__ ubn,
-                                                       const double* __restrict__ wout) {
-  const double pi4inv = 1.0 / (16.0 * atan(1.0));
-  const int t = tidx[j], k = ppanel[j];
-  const double x0 = tx[3 * (size_t)t], x1 = tx[3 * (size_t)t + 1], x2 = tx[3 * (size_t)t + 2];
-  const double* w = wout + (size_t)j * 2 * h;
-  double acc = 0.0;
-  for (int i = part; i < h; i += 4) {
-    const size_t g = (size_t)k * h + i;
-    double an, dn;
-    naive_entries(x0, x1, x2, sx + 3 * g, snx + 3 * g, sw[g], pi4inv, an, dn);
-    acc = acc + (w[i] - an) * ubn[g] - (w[h + i] - dn) * ub[g];
+// val(pair) = sum_i (S - S_naive)_i ubn_i - (K - K_naive)_i ub_i over the panel's h
+// nodes, for pairs pair_of(0 .. cnt-1), which come panel by panel: kAP pairs per
+// workgroup, kAL lanes each (nodes part, part + kAL, ..., the parts summed in a fixed
+// order).
+//
+// Bound by the loads of a node's nine values for every pair rather than by the weights
+// (16 bytes a node): the panels' nodes are therefore gathered in LDS once per
+// workgroup, as many as `slots`, and only pairs of further panels read them from
+// memory.  Eight lanes read a row 64 bytes at a time.  1.62M level pairs of order 8 (0.93
+// GB of weights): 0.45 to 0.33 ms; 30,000 targets of order 12: 158 to 100 us; all pairs
+// of 50,000 targets of order 8: 121 to 81.  With four lanes and every node from memory,
+// eight lanes alone gave 0.44, sixteen 0.51.
+constexpr int kAL = 8, kAP = 32, kRec = 10;  // doubles per node: x, n, w, ubn, ub, and one for the banks
+
+struct ApplyArgs {
+  const int *tidx, *ppanel;
+  const double *tx, *sx, *snx, *sw, *ub, *ubn, *wout;
+  double* val;
+};
+
+template <class F>
+__device__ __forceinline__ void apply_pairs(int cnt, int h, int slots, const ApplyArgs& A, F&& pair_of) {
+  extern __shared__ __align__(16) double rec[];  // [slots][h][kRec]
+  __shared__ int pan[kAP], slot[kAP], npan;
+  const int t0 = blockIdx.x * kAP;
+  if (t0 >= cnt) return;
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x, k = A.ppanel[pair_of(min(t0 + (lane & (kAP - 1)), cnt - 1))];
+    const int before = __shfl_up(k, 1, 64);
+    const bool first = lane < kAP && (lane == 0 || k != before);
+    const uint64_t m = __ballot(first);
+    if (lane < kAP) slot[lane] = __popcll(m & ((2ull << lane) - 1ull)) - 1;
+    if (first) pan[__popcll(m & ((1ull << lane) - 1ull))] = k;
+    if (lane == 0) npan = __popcll(m);
   }
-  return acc;
+  __syncthreads();
+  const int ns = min(npan, slots);
+  for (int e = threadIdx.x; e < ns * h; e += kAL * kAP) {
+    const size_t g = (size_t)pan[e / h] * h + e % h;
+    double* r = rec + (size_t)kRec * e;
+    for (int d = 0; d < 3; ++d) {
+      r[d] = A.sx[3 * g + d];
+      r[3 + d] = A.snx[3 * g + d];
+    }
+    r[6] = A.sw[g];
+    r[7] = A.ubn[g];
+    r[8] = A.ub[g];
+  }
+  __syncthreads();
+  const int q = threadIdx.x / kAL, part = threadIdx.x % kAL;
+  const bool live = t0 + q < cnt;
+  const int j = pair_of(live ? t0 + q : cnt - 1), t = A.tidx[j];
+  const double x0 = A.tx[3 * (size_t)t], x1 = A.tx[3 * (size_t)t + 1], x2 = A.tx[3 * (size_t)t + 2];
+  const double* w = A.wout + (size_t)j * 2 * h;
+  const double pi4inv = 1.0 / (16.0 * atan(1.0));
+  double acc = 0.0, an, dn;
+  if (slot[q] < ns) {
+    const double* r = rec + (size_t)kRec * h * slot[q];
+#pragma unroll 2
+    for (int i = part; i < h; i += kAL) {
+      const double* n = r + kRec * i;
+      naive_entries(x0, x1, x2, n, n + 3, n[6], pi4inv, an, dn);
+      acc = acc + (w[i] - an) * n[7] - (w[h + i] - dn) * n[8];
+    }
+  } else {
+    const size_t k = (size_t)pan[slot[q]] * h;
+    for (int i = part; i < h; i += kAL) {
+      const size_t g = k + i;
+      naive_entries(x0, x1, x2, A.sx + 3 * g, A.snx + 3 * g, A.sw[g], pi4inv, an, dn);
+      acc = acc + (w[i] - an) * A.ubn[g] - (w[h + i] - dn) * A.ub[g];
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < kAL; o <<= 1) acc = acc + __shfl_xor(acc, o, 64);
+  if (live && part == 0) A.val[j] = acc;
 }
 
 // Weights of the pairs labelled 0 (the learned selector found the panel's own
@@ -71,51 +123,42 @@ __global__ void __launch_bounds__(256) naive_fill_kernel(int nnz, int h, const i
   if (val) val[j] = 0.0;
 }
 
-__global__ void __launch_bounds__(256) naive_apply_kernel(int nnz, int h, const int* __restrict__ tidx,
-                                                          const int* __restrict__ ppanel, const double* __restrict__ tx,
-                                                          const double* __restrict__ sx, const double* __restrict__ snx,
-                                                          const double* __restrict__ sw, const double* __restrict__ ub,
-                                                          const double* __restrict__ ubn, const double* __restrict__ wout,
-                                                          double* __restrict__ val) {
-  const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = gt >> 2, part = gt & 3;
-  const bool live = j < nnz;
-  const double acc0 = live ? pair_correction_part(j, part, h, tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout) : 0.0;
-  double acc = acc0 + __shfl_xor(acc0, 1, 64);
-  acc = acc + __shfl_xor(acc, 2, 64);
-  if (live && part == 0) val[j] = acc;
+__global__ void __launch_bounds__(kAL* kAP) naive_apply_kernel(int nnz, int h, int slots, ApplyArgs A) {
+  apply_pairs(nnz, h, slots, A, [](int t) { return t; });
 }
 
-// The same for the pairs of the per-label lists first..last (lists concatenated
-// in label order, lengths ltot), so each part can run as soon as its weights are
-// in.  Four lanes per pair, each taking every fourth node, so a wave reads 16
-// weight rows contiguously; the four partial sums are combined in a fixed order.
-__global__ void __launch_bounds__(256) naive_apply_list_kernel(const int* __restrict__ lpairs,
-                                                               const int* __restrict__ ltot, int first, int last,
-                                                               int h, const int* __restrict__ tidx,
-                                                               const int* __restrict__ ppanel,
-                                                               const double* __restrict__ tx,
-                                                               const double* __restrict__ sx,
-                                                               const double* __restrict__ snx,
-                                                               const double* __restrict__ sw,
-                                                               const double* __restrict__ ub,
-                                                               const double* __restrict__ ubn,
-                                                               const double* __restrict__ wout,
-                                                               double* __restrict__ val) {
+// The same for the pairs of the per-label lists first..last (lists concatenated in label
+// order, lengths ltot), so each part can run as soon as its weights are in
+__global__ void __launch_bounds__(kAL* kAP) naive_apply_list_kernel(const int* __restrict__ lpairs,
+                                                                  const int* __restrict__ ltot, int first, int last,
+                                                                  int h, int slots, ApplyArgs A) {
   int base = 0, cnt = 0;
   for (int q = 0; q <= last; ++q) {
     if (q < first) base += ltot[q];
     else cnt += ltot[q];
   }
-  const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = gt >> 2, part = gt & 3;
-  const bool live = t < cnt;
-  const int j = live ? lpairs[base + t] : 0;
-  double acc = live ? pair_correction_part(j, part, h, tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout) : 0.0;
-  // (p0 + p1) + (p2 + p3) in every lane of the group
-  acc = acc + __shfl_xor(acc, 1, 64);
-  acc = acc + __shfl_xor(acc, 2, 64);
-  if (live && part == 0) val[j] = acc;
+  apply_pairs(cnt, h, slots, A, [&](int t) { return lpairs[base + t]; });
+}
+
+// panels a workgroup gathers: 24 KB, so that six workgroups share a CU
+static int apply_slots(int h) { return std::max(1, std::min(kAP, 24 * 1024 / (kRec * 8 * h))); }
+
+void launch_naive_apply(int64_t nnz, int h, const int* tidx, const int* ppanel, const double* tx, const double* sx,
+                        const double* snx, const double* sw, const double* ub, const double* ubn, const double* wout,
+                        double* val, hipStream_t s) {
+  const int slots = apply_slots(h);
+  hipLaunchKernelGGL(naive_apply_kernel, dim3((unsigned)((nnz + kAP - 1) / kAP)), dim3(kAL * kAP),
+                     sizeof(double) * kRec * h * slots, s, (int)nnz, h, slots,
+                     ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
+}
+
+void launch_naive_apply_list(int64_t nnz, const int* lpairs, const int* ltot, int first, int last, int h, const int* tidx,
+                             const int* ppanel, const double* tx, const double* sx, const double* snx, const double* sw,
+                             const double* ub, const double* ubn, const double* wout, double* val, hipStream_t s) {
+  const int slots = apply_slots(h);
+  hipLaunchKernelGGL(naive_apply_list_kernel, dim3((unsigned)((nnz + kAP - 1) / kAP)), dim3(kAL * kAP),
+                     sizeof(double) * kRec * h * slots, s, lpairs, ltot, first, last, h, slots,
+                     ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
 }
 
 // The weights by column, out(j, c) at c*nnz + j from rows of 2h per pair: tiles of 32 x

@@ -898,11 +898,11 @@ void Engine::build_target_lists() {
 
 // corrections of the pairs in per-label lists first..last (after their weights)
 void Engine::launch_correction(int first, int last, hipStream_t s) {
-  hipLaunchKernelGGL(naive_apply_list_kernel, dim3(blocks(4 * (size_t)nnz, 256)), dim3(256), 0, s,
-                     (const int*)d_lpairs.ptr, (const int*)d_ltot.ptr, first, last, h, (const int*)d_tidx.ptr,
-                     (const int*)d_ppanel.ptr, (const double*)d_tx.ptr, (const double*)d_sx.ptr,
-                     (const double*)d_snx.ptr, (const double*)d_sw.ptr, (const double*)d_ub.ptr,
-                     (const double*)d_ubn.ptr, (const double*)d_wout.ptr, (double*)d_val.ptr);
+  launch_naive_apply_list(nnz, (const int*)d_lpairs.ptr, (const int*)d_ltot.ptr, first, last, h,
+                          (const int*)d_tidx.ptr, (const int*)d_ppanel.ptr, (const double*)d_tx.ptr,
+                          (const double*)d_sx.ptr, (const double*)d_snx.ptr, (const double*)d_sw.ptr,
+                          (const double*)d_ub.ptr, (const double*)d_ubn.ptr, (const double*)d_wout.ptr,
+                          (double*)d_val.ptr, s);
 }
 
 // near-correction values (unless the last eval already made them from the
@@ -910,11 +910,10 @@ void Engine::launch_correction(int first, int last, hipStream_t s) {
 void Engine::apply_device() {
   if (nnz <= 0) return;
   if (!val_current)
-    hipLaunchKernelGGL(naive_apply_kernel, dim3(blocks(4 * (size_t)nnz, 256)), dim3(256), 0, stream, (int)nnz, h,
-                       (const int*)d_tidx.ptr, (const int*)d_ppanel.ptr, (const double*)d_tx.ptr,
+    launch_naive_apply(nnz, h, (const int*)d_tidx.ptr, (const int*)d_ppanel.ptr, (const double*)d_tx.ptr,
                        (const double*)d_sx.ptr, (const double*)d_snx.ptr, (const double*)d_sw.ptr,
                        (const double*)d_ub.ptr, (const double*)d_ubn.ptr, (const double*)d_wout.ptr,
-                       (double*)d_val.ptr);
+                       (double*)d_val.ptr, stream);
   build_target_lists();
   hipLaunchKernelGGL(target_sum_kernel, dim3(blocks(nt, 256)), dim3(256), 0, stream, nt, (const int*)d_toffs.ptr,
                      (int*)d_tpairs.ptr, (const double*)d_val.ptr, (double*)d_u.ptr);
