@@ -84,23 +84,26 @@ def kernel_flops(p, npan, counts, nrrq, nrrq_panels, split_levels):
     info = order_info(p)
     h, nq, ncoef = info["h"], info["nq"], info["ncoef"]
     nb = 3 * nq
-    nc1, nc2 = p * (p + 1) // 2, (p - 1) * p // 2
     ntot = int(sum(info["nl"]))
     lf = level_flops(p, counts)
+    formed = p >= 11
     ns = max(0, min(4, split_levels))
     out = {
         # 9 sequential FMAs per (level node, panel node); matrix cores up to order 12
         "levels": ("level_geom_mfma_kernel", 18.0 * h * ntot * npan, PEAK_FP64_TFLOPS),
-        # real Gauss-Jordan 2h^3; quaternion Gauss-Jordan 32h^3, C = B Fn^T 2h^3, As rows 8h^3
-        "rrq_solve": ("rrq_real_inverse_kernel+rrq_quat_inverse_kernel", 44.0 * h ** 3 * nrrq_panels,
-                      PEAK_FP64_TFLOPS),
-        # raw moments 4 nb (3 nc1 + 9 nc2) (twelve real node weights against the boundary
-        # harmonics of degree < p, resp. < p - 1), their combination into the boundary
-        # moments ~200 ncoef, degree recursion ~200 ncoef
-        "rrq_moments": ("rrq_target_kernel", float(nrrq) * (4 * nb * (3 * nc1 + 9 * nc2) + 400 * ncoef),
-                        PEAK_FP64_TFLOPS),
-        # W = G V: 2 (2h)(5h) per RRQ pair
-        "rrq_weights": ("rrq_weights_kernel", float(nrrq) * 20 * h * h, PEAK_FP64_TFLOPS),
+        # real Gauss-Jordan 2h^3; quaternion Gauss-Jordan 32h^3; orders 11 and 12 also form
+        # C = B Fn^T 2h^3 and C X 8h^3
+        "rrq_solve": ("rrq_real_inverse_kernel+rrq_quat_inverse_kernel" + ("+rrq_operator_kernel" if formed else ""),
+                      (44.0 if formed else 34.0) * h ** 3 * nrrq_panels, PEAK_FP64_TFLOPS),
+        # six real node weights, three each against the p (p+1) real columns of the boundary
+        # harmonics and the (p-1)(p+2) of their tangent combinations; their combination and
+        # the degree recursion ~300 ncoef
+        "rrq_moments": ("rrq_target_kernel",
+                        float(nrrq) * (6 * nb * (p * (p + 1) + (p - 1) * (p + 2)) + 300 * ncoef), PEAK_FP64_TFLOPS),
+        # X^T rhs, Fn^T v and B y per RRQ pair: 2 (4h^2 + h^2 + h^2); with C X formed
+        # 2 (4h^2 + 4h^2 + h^2)
+        "rrq_weights": ("rrq_weights_formed_kernel" if formed else "rrq_weights_kernel",
+                        float(nrrq) * (18 if formed else 12) * h * h, PEAK_FP64_TFLOPS),
     }
     # the direct stage: levels 1..ns on FP32 matrix cores, the rest on FP64
     if ns > 0:
