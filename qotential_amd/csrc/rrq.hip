@@ -1297,7 +1297,7 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
   // variant 2 (or QOL_SOLVE_MFMA=1) selects, for patch orders up to 8, the
   // matrix-core quaternion elimination (A as 4-wave accumulator tiles, B from a
   // separate real inverse), which is slower on the order-8 workload (5.3 vs 4.9
-  // ms for 14,250 panels, against 2.4 ms for the register-resident inverses)
+  // ms for 14,250 panels, against 1.1 ms for the register-resident inverses)
   const char* mf = std::getenv("QOL_SOLVE_MFMA");
   if (variant == 2 || (variant == 0 && mf && mf[0] == '1')) switch (T.p) {
 #define QOL_SOLVE_MFMA(P_, RT_, CT_, RPT_)                                                                  \
