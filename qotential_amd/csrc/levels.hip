@@ -52,66 +52,47 @@ std::vector<int> level_chunks(const LevelArgs& A, const int* suboff_host) {
 }
 
 // balls of a chunk's sub-patches (node range [c0, ...) of level l, sub-patches
-// [sb0, sb1)) from the chunk's x, y, z, w in LDS, summed in node order
+// [sb0, sb1)) from the chunk's x, y, z, w in LDS, summed in node order: eight lanes a
+// ball, lanes 0..3 (and 4..7 again) one of the sums sum w x, w y, w z, w each, then
+// every eighth node of the radius, whose maximum is exact in any order.  Bound by the
+// sums' chain: 0.69 to 0.59 ms of the kernel at order 12 (1,600 panels) and 1.21 to 1.17 at
+// order 8 (14,250) against one thread a ball with all four sums
 __device__ __forceinline__ void chunk_balls(const LevelArgs& A, const double* cn, int k0, int np_, int l, int c0,
                                             int sb0, int sb1, double* __restrict__ balls) {
-  const int nsc = sb1 - sb0;
-  for (int e = threadIdx.x; e < np_ * nsc; e += blockDim.x) {
+  const int nsc = sb1 - sb0, g = threadIdx.x & 7, first = threadIdx.x & 56, q = g & 3;
+  for (int e = threadIdx.x >> 3; e < np_ * nsc; e += blockDim.x >> 3) {
     const int pp = e / nsc, s = sb0 + e % nsc;
     const int s_all = A.sub_base[l] + s;
     const int i0 = A.suboff[A.sub_base[l] + l + s] - c0, i1 = A.suboff[A.sub_base[l] + l + s + 1] - c0;
     const double* L = cn + (size_t)pp * kCP;
-    // four independent sums, each in node order (the oracle's), in one pass; the
-    // LDS loads go in batches of kB nodes ahead of the additions, which keep
-    // their order (one thread serialises a sub-patch, so load latency, not the
-    // adds, bounded the unbatched loop)
+    // the sum in node order (the oracle's); the LDS loads go in batches of kB nodes
+    // ahead of the additions
     constexpr int kB = 8;
-    double swsum = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0;
+    const double *X = L + q * kChunk, *W = L + 3 * kChunk;
+    double a = 0.0;
     int j = i0;
     for (; j + kB <= i1; j += kB) {
-      double bx[kB], by[kB], bz[kB], bw[kB];
+      double bx[kB], bw[kB];
 #pragma unroll
       for (int u = 0; u < kB; ++u) {
-        bx[u] = L[j + u];
-        by[u] = L[kChunk + j + u];
-        bz[u] = L[2 * kChunk + j + u];
-        bw[u] = L[3 * kChunk + j + u];
+        bx[u] = X[j + u];
+        bw[u] = W[j + u];
       }
 #pragma unroll
-      for (int u = 0; u < kB; ++u) {
-        swsum += bw[u];
-        a0 += bx[u] * bw[u];
-        a1 += by[u] * bw[u];
-        a2 += bz[u] * bw[u];
-      }
+      for (int u = 0; u < kB; ++u) a += q == 3 ? bw[u] : bx[u] * bw[u];
     }
-    for (; j < i1; ++j) {
-      const double w = L[3 * kChunk + j];
-      swsum += w;
-      a0 += L[j] * w;
-      a1 += L[kChunk + j] * w;
-      a2 += L[2 * kChunk + j] * w;
-    }
-    const double qp[3] = {a0 / swsum, a1 / swsum, a2 / swsum};
-    // a maximum is exact in any order: kB partial maxima over batches
-    double rm[kB];
-#pragma unroll
-    for (int u = 0; u < kB; ++u) rm[u] = 0.0;
-    j = i0;
-    for (; j + kB <= i1; j += kB) {
-#pragma unroll
-      for (int u = 0; u < kB; ++u) {
-        const double d0 = L[j + u] - qp[0], d1 = L[kChunk + j + u] - qp[1], d2 = L[2 * kChunk + j + u] - qp[2];
-        rm[u] = fmax(rm[u], d0 * d0 + d1 * d1 + d2 * d2);
-      }
-    }
-    for (; j < i1; ++j) {
+    for (; j < i1; ++j) a += q == 3 ? W[j] : X[j] * W[j];
+    const double swsum = __shfl(a, first + 3, 64);
+    const double m = a / swsum;
+    const double qp[3] = {__shfl(m, first, 64), __shfl(m, first + 1, 64), __shfl(m, first + 2, 64)};
+    double rmax2 = 0.0;
+    for (j = i0 + g; j < i1; j += 8) {
       const double d0 = L[j] - qp[0], d1 = L[kChunk + j] - qp[1], d2 = L[2 * kChunk + j] - qp[2];
-      rm[0] = fmax(rm[0], d0 * d0 + d1 * d1 + d2 * d2);
+      rmax2 = fmax(rmax2, d0 * d0 + d1 * d1 + d2 * d2);
     }
-    double rmax2 = rm[0];
 #pragma unroll
-    for (int u = 1; u < kB; ++u) rmax2 = fmax(rmax2, rm[u]);
+    for (int o = 1; o < 8; o <<= 1) rmax2 = fmax(rmax2, __shfl_xor(rmax2, o, 64));
+    if (g > 0) continue;
     const double r2 = A.subtyp[s_all] == 1 ? A.dist2 * fmax(rmax2, 0.5 * swsum) : A.dist2 * fmax(rmax2, swsum);
     double* B = balls + (size_t)(k0 + pp) * 4 * A.nsubtot + 4 * s_all;
     B[0] = qp[0];
