@@ -92,13 +92,14 @@ __device__ __forceinline__ void chunk_balls(const LevelArgs& A, const double* cn
     }
 #pragma unroll
     for (int o = 1; o < 8; o <<= 1) rmax2 = fmax(rmax2, __shfl_xor(rmax2, o, 64));
-    if (g > 0) continue;
-    const double r2 = A.subtyp[s_all] == 1 ? A.dist2 * fmax(rmax2, 0.5 * swsum) : A.dist2 * fmax(rmax2, swsum);
-    double* B = balls + (size_t)(k0 + pp) * 4 * A.nsubtot + 4 * s_all;
-    B[0] = qp[0];
-    B[1] = qp[1];
-    B[2] = qp[2];
-    B[3] = r2;
+    if (g == 0) {
+      const double r2 = A.subtyp[s_all] == 1 ? A.dist2 * fmax(rmax2, 0.5 * swsum) : A.dist2 * fmax(rmax2, swsum);
+      double* B = balls + (size_t)(k0 + pp) * 4 * A.nsubtot + 4 * s_all;
+      B[0] = qp[0];
+      B[1] = qp[1];
+      B[2] = qp[2];
+      B[3] = r2;
+    }
   }
 }
 
