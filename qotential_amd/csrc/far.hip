@@ -15,6 +15,12 @@
 // split into chunks so that few targets still fill the chip; each chunk's sums
 // go to part(chunk, target) and are added in chunk order, so the result does not
 // depend on timing.
+//
+// Where the packed form could leave the FP64 range -- a position or strength beyond
+// kFarHuge or not a number -- the sum is formed again term by term (far_plain): a source
+// like that is packed with a strength that is not a number, which makes every sum one,
+// and sums that are not finite, or whose target lies that far, are formed again.  The
+// direct kernel itself tests nothing.
 #include <algorithm>
 
 #include "qol_kernels.h"
@@ -23,34 +29,50 @@ namespace qol {
 
 namespace {
 
-// coordinates beyond this square past the FP64 range: such sources and targets
-// are taken out of the sum below and get what the plain formula gives
+// below this no square of a coordinate difference and no product with a strength leaves
+// the FP64 range
 constexpr double kFarHuge = 1e150;
+
+struct FarSources {
+  const double *sx, *snx, *sw, *ub, *ubn;
+};
+
+// the sum over sources j0 .. j1 - 1 at x, term by term; a source whose r^2 is not above
+// the coincidence threshold (or not a number) is left out, strength and all
+__device__ double far_plain(const FarSources& S, int j0, int j1, const double* x) {
+  const double pi4inv = 1.0 / (16.0 * atan(1.0));
+  double acc = 0.0;
+#pragma unroll 1
+  for (int j = j0; j < j1; ++j) {
+    const double *y = S.sx + 3 * (size_t)j, *n = S.snx + 3 * (size_t)j;
+    const double dx = x[0] - y[0], dy = x[1] - y[1], dz = x[2] - y[2];
+    const double rr = dx * dx + dy * dy + dz * dz;
+    if (rr > 1.0e-28) {
+      const double ri = 1.0 / sqrt(rr), w = pi4inv * S.sw[j];
+      acc += w * S.ubn[j] * ri - w * S.ub[j] * (dx * n[0] + dy * n[1] + dz * n[2]) * ri * ri * ri;
+    }
+  }
+  return acc;
+}
 
 }  // namespace
 
-// A source whose position is NaN contributes nothing (its r^2 fails the test
-// against the coincidence threshold), nor does one so far that r^2 overflows.
-__global__ void __launch_bounds__(256) far_pack_kernel(int ns, const double* __restrict__ sx,
-                                                       const double* __restrict__ snx, const double* __restrict__ sw,
-                                                       const double* __restrict__ ub, const double* __restrict__ ubn,
-                                                       double2* __restrict__ src) {
+__global__ void __launch_bounds__(256) far_pack_kernel(int ns, FarSources S, double2* __restrict__ src) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= ns) return;
   const double pi4inv = 1.0 / (16.0 * atan(1.0));
-  double x = sx[3 * (size_t)j], y = sx[3 * (size_t)j + 1], z = sx[3 * (size_t)j + 2];
-  const double w = pi4inv * sw[j], d = w * ub[j];
-  double s = w * ubn[j], a = d * snx[3 * (size_t)j], b = d * snx[3 * (size_t)j + 1], c = d * snx[3 * (size_t)j + 2];
-  const double big = fmax(fmax(fabs(x), fabs(y)), fabs(z));
-  if (x != x || y != y || z != z || (big >= kFarHuge && !isinf(big))) {
-    x = y = z = 0.0;
-    s = a = b = c = 0.0;
-  }
+  const double *y = S.sx + 3 * (size_t)j, *n = S.snx + 3 * (size_t)j;
+  const double w = pi4inv * S.sw[j], d = w * S.ub[j];
+  double v[7] = {y[0], y[1], y[2], w * S.ubn[j], d * n[0], d * n[1], d * n[2]};
+  bool out = false;
+#pragma unroll
+  for (int c = 0; c < 7; ++c) out |= !(fabs(v[c]) < kFarHuge);
+  if (out) v[3] = __builtin_nan("");
   double2* o = src + 4 * (size_t)j;
-  o[0] = double2{x, y};
-  o[1] = double2{z, s};
-  o[2] = double2{a, b};
-  o[3] = double2{c, 0.0};
+  o[0] = double2{v[0], v[1]};
+  o[1] = double2{v[2], v[3]};
+  o[2] = double2{v[4], v[5]};
+  o[3] = double2{v[6], 0.0};
 }
 
 // one wave per tile of 64 kFT targets and chunk of sources
@@ -87,9 +109,11 @@ __global__ void __launch_bounds__(64) far_direct_kernel(int nt, const double* __
 }
 
 // u(t) = sum of part(c, t): 64 targets per workgroup, each of the 4 waves adds
-// every fourth chunk in order, then the four sums are added in order
-__global__ void __launch_bounds__(256) far_sum_kernel(int nt, int nchunk, const double* __restrict__ tx,
-                                                      const double* __restrict__ part, double* __restrict__ u) {
+// every fourth chunk in order, then the four sums are added in order; the same four
+// waves form a sum again
+__global__ void __launch_bounds__(256) far_sum_kernel(int nt, int nchunk, int ns, FarSources S,
+                                                      const double* __restrict__ tx, const double* __restrict__ part,
+                                                      double* __restrict__ u) {
   __shared__ double s[4][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int t = blockIdx.x * 64 + lane;
@@ -99,13 +123,17 @@ __global__ void __launch_bounds__(256) far_sum_kernel(int nt, int nchunk, const 
     for (int c = wv; c < nchunk; c += 4) acc += part[(size_t)c * nt + t];
   s[wv][lane] = acc;
   __syncthreads();
-  if (wv != 0 || t >= nt) return;
   double v = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
-  const double x = tx[3 * (size_t)t], y = tx[3 * (size_t)t + 1], z = tx[3 * (size_t)t + 2];
-  const double big = fmax(fmax(fabs(x), fabs(y)), fabs(z));
-  if (x != x || y != y || z != z) v = 0.0;                // every r^2 is NaN: no source contributes
-  else if (big >= kFarHuge) v = isinf(big) ? big - big : 0.0;  // 0 * inf, or every 1/r underflows to 0
-  u[t] = v;
+  const size_t tc = min(t, nt - 1);
+  const double x[3] = {tx[3 * tc], tx[3 * tc + 1], tx[3 * tc + 2]};
+  const bool again = t < nt && !(isfinite(v) && fabs(x[0]) < kFarHuge && fabs(x[1]) < kFarHuge && fabs(x[2]) < kFarHuge);
+  if (__syncthreads_or(again)) {
+    const int per = (ns + 3) / 4;
+    s[wv][lane] = again ? far_plain(S, wv * per, min(ns, (wv + 1) * per), x) : 0.0;
+    __syncthreads();
+    if (again) v = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+  }
+  if (wv == 0 && t < nt) u[t] = v;
 }
 
 // Measured (targets x sources, billions of pairs a second): four targets a thread
@@ -128,14 +156,15 @@ FarPlan far_plan(int nt, int ns) {
 void launch_far(const FarPlan& P, int nt, const double* tx, int ns, const double* sx, const double* snx,
                 const double* sw, const double* ub, const double* ubn, double* src, double* part, double* u,
                 hipStream_t s) {
-  hipLaunchKernelGGL(far_pack_kernel, dim3((ns + 255) / 256), dim3(256), 0, s, ns, sx, snx, sw, ub, ubn, (double2*)src);
+  const FarSources S{sx, snx, sw, ub, ubn};
+  hipLaunchKernelGGL(far_pack_kernel, dim3((ns + 255) / 256), dim3(256), 0, s, ns, S, (double2*)src);
   const dim3 grid((nt + 64 * P.per - 1) / (64 * P.per), P.nchunk);
   switch (P.per) {
     case 1: hipLaunchKernelGGL(far_direct_kernel<1>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
     case 2: hipLaunchKernelGGL(far_direct_kernel<2>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
     default: hipLaunchKernelGGL(far_direct_kernel<4>, grid, dim3(64), 0, s, nt, tx, ns, P.len, src, part); break;
   }
-  hipLaunchKernelGGL(far_sum_kernel, dim3((nt + 63) / 64), dim3(256), 0, s, nt, P.nchunk, tx, part, u);
+  hipLaunchKernelGGL(far_sum_kernel, dim3((nt + 63) / 64), dim3(256), 0, s, nt, P.nchunk, ns, S, tx, part, u);
 }
 
 }  // namespace qol
