@@ -192,7 +192,9 @@ void qol_lap3ddlp_closepanel_mex_(const int64_t* m_tgt, const double* t_x, const
  * (qol_build_patch_levels_mex, qol_lap3dsdlpmat_levels_mex,
  * qol_clear_patch_levels_mex, qol_clear_patch_levels_all_mex).  One slot,
  * generation-tagged handle; ier 0 ok, 1 no free slot, 2 bad handle,
- * 3 npols mismatch, 5 unsupported level set, 6 device failure. */
+ * 3 npols mismatch, 5 unsupported level set, 6 device failure.
+ * qol_clear_patch_levels_all_mex_ also frees the engine (at most 1 GiB of device
+ * memory) that qol_getnearquad_lap_rrq_mex_ keeps between calls. */
 void qol_build_patch_levels_mex_(const int64_t* korder, const int64_t* npols, const double* sx,
                                  const double* rts, const double* rps, const int64_t* order,
                                  const double* dist, const int64_t* nlevel, int64_t* lv,

@@ -99,9 +99,11 @@ Engine& panel_engine(int64_t p, int64_t ichart, const double* sx, const double* 
 // order, panel count and device: streams, tables and buffers, nothing of a call's data.
 // Making and freeing them took 6 of a 10 ms call for 944 panels of order 4 (150,096
 // pairs; freeing 260 MB alone 4.3).  A call takes the engine out of the slot, so that no
-// two threads hold it, and leaves its own there afterwards if that holds at most 1 GiB;
-// an engine that another replaces, that is larger or whose call failed is freed.  Never
-// destroyed at exit, like the per-panel engines.
+// two threads hold it, frees it before its own is made if it is of another shape (so that
+// the two never hold memory together), and leaves its own there afterwards if that holds
+// at most 1 GiB; an engine that is larger or whose call failed is freed.
+// qol_clear_patch_levels_all_mex_ empties the slot.  Never destroyed at exit, like the
+// per-panel engines.
 struct SurfaceEngine {
   std::unique_ptr<Engine> e;
   int device = -1;
@@ -118,19 +120,23 @@ SurfaceSlot& surface_slot() {
 }
 constexpr long long kSurfaceKeep = 1ll << 30;
 
+// empties the slot
+SurfaceEngine take_surface() {
+  SurfaceEngine s;
+  std::lock_guard<std::mutex> g(surface_slot().mu);
+  std::swap(s, surface_slot().s);
+  return s;
+}
+
 template <class F>
 void with_surface_engine(int64_t p, int64_t npan, const double* sx, const double* snx, const double* sw,
                          const double* rts, const double* rps, F&& call) {
-  SurfaceEngine mine;
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   bool ad = false, sq = true;
   level_mode(&ad, &sq);
-  {
-    std::lock_guard<std::mutex> g(surface_slot().mu);
-    SurfaceEngine& s = surface_slot().s;
-    if (s.e && s.device == dev && s.p == p && s.npan == npan) std::swap(mine, s);
-  }
+  SurfaceEngine mine = take_surface();
+  if (mine.device != dev || mine.p != p || mine.npan != npan) mine = SurfaceEngine{};
   const long long before = thread_device_bytes();
   if (mine.e) {
     mine.e->set_surface(sx, snx, sw, rts, rps, nullptr, nullptr, false);
@@ -671,6 +677,7 @@ void qol_clear_patch_levels_all_mex_(int64_t* ier) {
     g_slot.live = false;
     g_slot.generation += 1;
   }
+  take_surface();  // and the whole-surface engine kept between calls, with its device memory
   *ier = 0;
 }
 
