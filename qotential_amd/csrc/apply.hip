@@ -161,18 +161,19 @@ void launch_naive_apply_list(int64_t nnz, const int* lpairs, const int* ltot, in
                      ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
 }
 
-// The weights by column, out(j, c) at c*nnz + j from rows of 2h per pair: tiles of 32 x
-// 32 through LDS, so that both sides move whole lines and the host, which looped over
-// the rows before, copies two finished blocks
-__global__ void __launch_bounds__(256) weight_columns_kernel(int nnz, int m2, const double* __restrict__ wout,
+// The weights by column, out(j, c - c0) at (c - c0)*nnz + j for nc columns c from c0, from
+// rows of m2 = 2h per pair: tiles of 32 x 32 through LDS, so that both sides move whole
+// lines and the host, which looped over the rows before, copies finished blocks
+__global__ void __launch_bounds__(256) weight_columns_kernel(int nnz, int m2, int c0, int nc,
+                                                             const double* __restrict__ wout,
                                                              double* __restrict__ cols) {
   __shared__ double tile[32][33];
-  const int j0 = blockIdx.x * 32, c0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  const int j0 = blockIdx.x * 32, d0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
   for (int r = y; r < 32; r += 8)
-    if (j0 + r < nnz && c0 + x < m2) tile[r][x] = wout[(size_t)(j0 + r) * m2 + c0 + x];
+    if (j0 + r < nnz && d0 + x < nc) tile[r][x] = wout[(size_t)(j0 + r) * m2 + c0 + d0 + x];
   __syncthreads();
   for (int c = y; c < 32; c += 8)
-    if (j0 + x < nnz && c0 + c < m2) cols[(size_t)(c0 + c) * nnz + j0 + x] = tile[x][c];
+    if (j0 + x < nnz && d0 + c < nc) cols[(size_t)(d0 + c) * nnz + j0 + x] = tile[x][c];
 }
 
 // COO triplets of getnearquad_lap_rrq: out = (tcxi(k)-1)*h + (j-1)*m + i (1-based)

@@ -815,14 +815,31 @@ void Engine::get_weights(double* As, double* Ad, i64* label, double* Omega, doub
   std::vector<Part> parts;
   const size_t n = (size_t)h * (nnz > 0 ? nnz : 0);
   if ((As || Ad) && nnz > 0) {
-    // column-major (nnz, h); the moment vectors are used up, and their buffer is the larger
-    d_vt.alloc(sizeof(double) * 2 * n);
+    // column-major (nnz, h).  The moment vectors are used up, and after eval their buffer
+    // holds every column; after eval_levels_only it may hold none, and then grows to
+    // kColumnBytes at most (or one column): so many columns at a time
+    constexpr size_t kColumnBytes = 16 << 20;
+    const size_t column = sizeof(double) * (size_t)nnz;
+    d_vt.alloc(std::max(column, std::min(2 * h * column, kColumnBytes)));
     double* cols = (double*)d_vt.ptr;
-    hipLaunchKernelGGL(weight_columns_kernel, dim3(blocks(nnz, 32), blocks(2 * h, 32)), dim3(256), 0, stream, (int)nnz,
-                       2 * h, (const double*)d_wout.ptr, cols);
-    HIPCHK(hipGetLastError());
-    parts.push_back({As, cols, n});
-    parts.push_back({Ad, cols + n, n});
+    const int m2 = 2 * h, per = (int)std::min<size_t>(m2, d_vt.bytes / column);
+    for (int c0 = 0; c0 < m2; c0 += per) {
+      const int nc = std::min(per, m2 - c0);
+      hipLaunchKernelGGL(weight_columns_kernel, dim3(blocks(nnz, 32), blocks(nc, 32)), dim3(256), 0, stream, (int)nnz,
+                         m2, c0, nc, (const double*)d_wout.ptr, cols);
+      HIPCHK(hipGetLastError());
+      if (nc == m2) {
+        parts.push_back({As, cols, n});
+        parts.push_back({Ad, cols + n, n});
+        break;
+      }
+      HIPCHK(hipStreamSynchronize(stream));
+      const int na = std::max(0, std::min(h, c0 + nc) - c0);  // columns of As, the rest of Ad
+      if (As && na > 0) HIPCHK(hipMemcpy(As + (size_t)nnz * c0, cols, column * na, hipMemcpyDeviceToHost));
+      if (Ad && na < nc)
+        HIPCHK(hipMemcpy(Ad + (size_t)nnz * (c0 + na - h), cols + (size_t)nnz * na, column * (nc - na),
+                         hipMemcpyDeviceToHost));
+    }
   }
   if (nnz > 0) {
     parts.push_back({Omega, (const double*)d_omega.ptr, 4 * n});

@@ -155,7 +155,7 @@ void launch_naive_apply(int64_t nnz, int h, const int* tidx, const int* ppanel, 
 void launch_naive_apply_list(int64_t nnz, const int* lpairs, const int* ltot, int first, int last, int h, const int* tidx,
                              const int* ppanel, const double* tx, const double* sx, const double* snx, const double* sw,
                              const double* ub, const double* ubn, const double* wout, double* val, hipStream_t s);
-__global__ void weight_columns_kernel(int nnz, int m2, const double* wout, double* cols);
+__global__ void weight_columns_kernel(int nnz, int m2, int c0, int nc, const double* wout, double* cols);
 __global__ void target_count_kernel(int nnz, const int* tidx, int* tcount);
 __global__ void target_fill_kernel(int nnz, const int* tidx, const int* toffs, int* tcur, int* tpairs);
 __global__ void target_sum_kernel(int nt, const int* toffs, int* tpairs, const double* val, double* u);
