@@ -289,7 +289,7 @@ int qol_engine_level_data(void* h, double* lgeo, double* balls) {
 }
 
 int qol_engine_triplets(void* h, const int64_t* trow, int64_t* si, int64_t* sj, double* vs, double* vd) {
-  return guarded([&] { E(h)->triplets(trow, si, sj, vs, vd); });
+  return guarded([&] { E(h)->triplets(trow, si, sj, vs, vd, false); });
 }
 
 int qol_engine_set_precision(void* h, int64_t split_levels) {
@@ -576,7 +576,7 @@ void qol_getnearquad_lap_rrq_mex_(const int64_t* npan, const int64_t* nterms, co
       e.set_targets(nt, tcx, false);
       e.set_pairs(offs.data(), idx.data());
       e.eval((*iside % 10) == 0 ? 1 : 0, 1e-10, false);
-      e.triplets(tcxrow, sparsei, sparsej, sparsevs, sparsevd);
+      e.triplets(tcxrow, sparsei, sparsej, sparsevs, sparsevd, true);
       double st = 0.0;
       const int64_t n = e.projection_unconverged(&st);
       set_unconverged(n, st);

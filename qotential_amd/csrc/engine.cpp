@@ -980,10 +980,13 @@ void Engine::level_data(double* lgeo, double* balls) {
   if (balls) HIPCHK(hipMemcpy(balls, d_balls.ptr, sizeof(double) * 4 * (size_t)tab->nsubtot * npan, hipMemcpyDeviceToHost));
 }
 
-void Engine::triplets(const i64* trow, i64* si, i64* sj, double* vs, double* vd) {
+void Engine::triplets(const i64* trow, i64* si, i64* sj, double* vs, double* vd, bool keep) {
   if (!evaluated) throw std::runtime_error("weights not evaluated");
   std::vector<int> tr((size_t)(nt > 0 ? nt : 1), 0);
   for (int t = 0; t < nt; ++t) tr[t] = (int)trow[t];
+  DevBuf own[5];
+  DevBuf &d_tr = keep ? this->d_tr : own[0], &d_si = keep ? this->d_si : own[1], &d_sj = keep ? this->d_sj : own[2],
+         &d_vs = keep ? this->d_vs : own[3], &d_vd = keep ? this->d_vd : own[4];
   upload(d_tr, tr.data(), tr.size(), stream);
   const size_t n = (size_t)nnz * h;
   d_si.alloc(sizeof(int64_t) * (n ? n : 1)); d_sj.alloc(sizeof(int64_t) * (n ? n : 1));

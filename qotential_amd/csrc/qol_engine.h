@@ -154,7 +154,8 @@ struct Engine {
   void far(const double* ub, const double* ubn, double* u);
   void get_values(double* val, double* u);
   void level_data(double* lgeo, double* balls);
-  void triplets(const i64* trow, i64* si, i64* sj, double* vs, double* vd);
+  // the columns' device buffers (32 h bytes a pair) stay with the engine if `keep`
+  void triplets(const i64* trow, i64* si, i64* sj, double* vs, double* vd, bool keep);
 };
 
 // engine stage times (ms: levels, classify, direct, rrq setup, rrq solve,
