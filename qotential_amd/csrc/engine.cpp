@@ -452,7 +452,7 @@ void Engine::direct(hipStream_t s) {
 
 i64 Engine::nearlist() {
   if (nt < 0) throw std::runtime_error("targets not set");
-  d_nball.alloc(sizeof(double) * 4 * npan);
+  d_nball.alloc(sizeof(double) * 4 * 64 * blocks(npan, 64));
   d_cnt.alloc(sizeof(int) * npan);
   d_offs.alloc(sizeof(int) * (npan + 1));
   HIPCHK(hipMemsetAsync(d_cnt.ptr, 0, sizeof(int) * npan, stream));
@@ -482,7 +482,7 @@ i64 Engine::nearlist() {
 // large as the largest panel ball, at most 2^24 cells): bit-identical CSR.
 i64 Engine::nearlist_grid() {
   if (nt < 0) throw std::runtime_error("targets not set");
-  d_nball.alloc(sizeof(double) * 4 * npan);
+  d_nball.alloc(sizeof(double) * 4 * 64 * blocks(npan, 64));
   d_cnt.alloc(sizeof(int) * npan);
   d_offs.alloc(sizeof(int) * (npan + 1));
   hipLaunchKernelGGL(nearlist_prep_kernel, dim3(blocks(npan, 64)), dim3(64), 0, stream, npan, h,

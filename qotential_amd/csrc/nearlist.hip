@@ -14,13 +14,17 @@
 namespace qol {
 
 constexpr int kNearG = 4;  // groups of 16 panels a wave tests
+constexpr int kNearB = 4;  // balls a wave tests between two loads
 
 // ball[k] = (c0, c1, c2, r^2), summed in the reference's order; corner: the 3 x h
 // rows interpolating a panel at its corners (used when diam > 0)
 __global__ void nearlist_prep_kernel(int npan, int h, const double* __restrict__ sx, const double* __restrict__ sw,
                                      const double* __restrict__ corner, double diam, double* __restrict__ ball) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npan) return;
+  if (k >= npan) {  // up to whole sets of 64: nothing lies inside
+    for (int d = 0; d < 4; ++d) ball[4 * k + d] = 0.0;
+    return;
+  }
   double q0 = 0.0, q1 = 0.0, q2 = 0.0, s = 0.0;
   for (int i = 0; i < h; ++i) {
     const size_t g = (size_t)k * h + i;
@@ -68,13 +72,19 @@ __device__ __forceinline__ bool in_ball(const double* b, double x0, double x1, d
 // wave for the 16 panels' own tests: 1/16 of the tests plus those of the candidates, in
 // the targets' order.  A not-a-number ball or target passes the first test and fails the
 // second.  Segments and 64-thread workgroups because the fill's serial walk over all
-// targets left most of the chip idle.  14,250 panels x
-// 50,000 targets: 88 + 88 us; 2,400 x 20,011: 121 + 242 to 29 + 31.
+// targets left most of the chip idle.  Panels in no spatial order leave their groups'
+// balls so large that most targets are candidates: all pairs are tested then, so the
+// tests themselves have to run at the vector rate, four balls at a time from scalar
+// registers with one branch (ball by ball, each waiting for its own load, the kernel was
+// slower on such panels than all pairs by the kernel before it).  14,250 panels x 50,000 targets: 52 +
+// 63 us, panels in random order 292 + 320 (ball by ball 79 + 84 and 694 + 662); 2,400 x
+// 20,011: 121 + 242 to 18 + 24.
 template <bool FILL>
 __global__ void __launch_bounds__(64) nearlist_kernel(int npan, int nt, int seg, const double* __restrict__ tx,
                                                       const double* __restrict__ ball, int* __restrict__ part,
                                                       int* __restrict__ count, const int* __restrict__ offs,
                                                       int* __restrict__ idx) {
+  typedef const __attribute__((address_space(4))) double* const_ptr;  // scalar loads
   __shared__ int cand[kNearG][128];
   const int lane = threadIdx.x, k0 = blockIdx.x * 64, k = min(k0 + lane, npan - 1);
   const int t_lo = blockIdx.y * seg, t_hi = min(nt, t_lo + seg);
@@ -106,22 +116,41 @@ __global__ void __launch_bounds__(64) nearlist_kernel(int npan, int nt, int seg,
 #pragma unroll 4
     for (int y = 0; y < (int)blockIdx.y; ++y) acc += part[(size_t)y * npan + k];
   }
-  // the tests of group g's 16 panels on its first n candidates
-  auto test = [&](int g, int n) {
-    const int t = cand[g][lane];
-    const bool on = lane < n;
-    const double x0 = on ? tx[3 * (size_t)t] : 0.0, x1 = on ? tx[3 * (size_t)t + 1] : 0.0,
-                 x2 = on ? tx[3 * (size_t)t + 2] : 0.0;
-    for (int q = 0; q < 16; ++q) {
-      const int kq = k0 + 16 * g + q;
-      if (kq >= npan) break;
-      const bool in = on && in_ball(ball + 4 * (size_t)kq, x0, x1, x2);
-      const uint64_t b = __ballot(in);
-      if (b == 0) continue;
-      const int base = __builtin_amdgcn_readlane(acc, 16 * g + q);
-      if (FILL && in) idx[base + __popcll(b & ((1ull << lane) - 1ull))] = t;
-      acc += lane == 16 * g + q ? __popcll(b) : 0;
+  // the tests of group g's 16 panels on target t of the lanes in `on`, kNearB balls at a
+  // time, the next ones' scalar loads under way meanwhile
+  auto test_lanes = [&](int g, uint64_t on, int t, double x0, double x1, double x2) {
+    const const_ptr B = (const_ptr)(uintptr_t)(ball + 4 * (size_t)(k0 + 16 * g));
+    double c[4 * kNearB], next[4 * kNearB];
+#pragma unroll
+    for (int i = 0; i < 4 * kNearB; ++i) next[i] = B[i];
+#pragma unroll 1
+    for (int q0 = 0; q0 < 16; q0 += kNearB) {
+#pragma unroll
+      for (int i = 0; i < 4 * kNearB; ++i) {
+        c[i] = next[i];
+        next[i] = B[4 * min(q0 + kNearB, 16 - kNearB) + i];
+      }
+      uint64_t b[kNearB], any = 0;
+#pragma unroll
+      for (int u = 0; u < kNearB; ++u) {
+        const double d0 = x0 - c[4 * u], d1 = x1 - c[4 * u + 1], d2 = x2 - c[4 * u + 2];
+        b[u] = __ballot(d0 * d0 + d1 * d1 + d2 * d2 < c[4 * u + 3]) & on;
+        any |= b[u];
+      }
+      if (any == 0) continue;
+#pragma unroll
+      for (int u = 0; u < kNearB; ++u) {
+        const int to = 16 * g + q0 + u, base = __builtin_amdgcn_readlane(acc, to);
+        if (FILL && (b[u] >> lane & 1ull)) idx[base + __popcll(b[u] & ((1ull << lane) - 1ull))] = t;
+        acc += lane == to ? __popcll(b[u]) : 0;
+      }
     }
+  };
+  // the same on its first n candidates
+  auto test = [&](int g, int n) {
+    const int t = cand[g][min(lane, n - 1)];
+    const double* y = tx + 3 * (size_t)t;
+    test_lanes(g, n < 64 ? (1ull << n) - 1ull : ~0ull, t, y[0], y[1], y[2]);
   };
   double x[3];
   auto load = [&](int t) {
