@@ -36,7 +36,12 @@ __device__ __forceinline__ void naive_entries(double x0, double x1, double x2, c
 // GB of weights): 0.45 to 0.33 ms; 30,000 targets of order 12: 158 to 100 us; all pairs
 // of 50,000 targets of order 8: 121 to 81.  With four lanes and every node from memory,
 // eight lanes alone gave 0.44, sixteen 0.51.
-constexpr int kAL = 8, kAP = 32, kRec = 10;  // doubles per node: x, n, w, ubn, ub, and one for the banks
+//
+// Up to order 5 (15 nodes) eight lanes leave too many idle in their one or two rounds, and four
+// take a pair: 1.97M pairs on 3,570 panels with eight and with four lanes take (with the
+// targets' sums) 134 and 93 us at order 2, 137 and 121 at 3, 228 and 149 at 4, 237 and 189
+// at 5; at order 6 253 and 274.
+constexpr int kAT = 256, kRec = 10;  // doubles per node: x, n, w, ubn, ub, and one for the banks
 
 struct ApplyArgs {
   const int *tidx, *ppanel;
@@ -44,8 +49,10 @@ struct ApplyArgs {
   double* val;
 };
 
-template <class F>
+template <int kAL, class F>
 __device__ __forceinline__ void apply_pairs(int cnt, int h, int slots, const ApplyArgs& A, F&& pair_of) {
+  constexpr int kAP = kAT / kAL;
+  static_assert(kAP <= 64, "one wave finds the workgroup's panels");
   extern __shared__ __align__(16) double rec[];  // [slots][h][kRec]
   __shared__ int pan[kAP], slot[kAP], npan;
   const int t0 = blockIdx.x * kAP;
@@ -61,7 +68,7 @@ __device__ __forceinline__ void apply_pairs(int cnt, int h, int slots, const App
   }
   __syncthreads();
   const int ns = min(npan, slots);
-  for (int e = threadIdx.x; e < ns * h; e += kAL * kAP) {
+  for (int e = threadIdx.x; e < ns * h; e += kAT) {
     const size_t g = (size_t)pan[e / h] * h + e % h;
     double* r = rec + (size_t)kRec * e;
     for (int d = 0; d < 3; ++d) {
@@ -123,41 +130,51 @@ __global__ void __launch_bounds__(256) naive_fill_kernel(int nnz, int h, const i
   if (val) val[j] = 0.0;
 }
 
-__global__ void __launch_bounds__(kAL* kAP) naive_apply_kernel(int nnz, int h, int slots, ApplyArgs A) {
-  apply_pairs(nnz, h, slots, A, [](int t) { return t; });
+template <int kAL>
+__global__ void __launch_bounds__(kAT) naive_apply_kernel(int nnz, int h, int slots, ApplyArgs A) {
+  apply_pairs<kAL>(nnz, h, slots, A, [](int t) { return t; });
 }
 
 // The same for the pairs of the per-label lists first..last (lists concatenated in label
 // order, lengths ltot), so each part can run as soon as its weights are in
-__global__ void __launch_bounds__(kAL* kAP) naive_apply_list_kernel(const int* __restrict__ lpairs,
-                                                                  const int* __restrict__ ltot, int first, int last,
-                                                                  int h, int slots, ApplyArgs A) {
+template <int kAL>
+__global__ void __launch_bounds__(kAT) naive_apply_list_kernel(const int* __restrict__ lpairs,
+                                                               const int* __restrict__ ltot, int first, int last, int h,
+                                                               int slots, ApplyArgs A) {
   int base = 0, cnt = 0;
   for (int q = 0; q <= last; ++q) {
     if (q < first) base += ltot[q];
     else cnt += ltot[q];
   }
-  apply_pairs(cnt, h, slots, A, [&](int t) { return lpairs[base + t]; });
+  apply_pairs<kAL>(cnt, h, slots, A, [&](int t) { return lpairs[base + t]; });
 }
 
-// panels a workgroup gathers: 24 KB, so that six workgroups share a CU
-static int apply_slots(int h) { return std::max(1, std::min(kAP, 24 * 1024 / (kRec * 8 * h))); }
+// lanes per pair, pairs per workgroup, and the panels it gathers: 24 KB, so that six
+// workgroups share a CU
+struct ApplyPlan {
+  int lanes, pairs, slots;
+};
+static ApplyPlan apply_plan(int h) {
+  const int lanes = h <= 15 ? 4 : 8, pairs = kAT / lanes;
+  return {lanes, pairs, std::max(1, std::min(pairs, 24 * 1024 / (kRec * 8 * h)))};
+}
 
 void launch_naive_apply(int64_t nnz, int h, const int* tidx, const int* ppanel, const double* tx, const double* sx,
                         const double* snx, const double* sw, const double* ub, const double* ubn, const double* wout,
                         double* val, hipStream_t s) {
-  const int slots = apply_slots(h);
-  hipLaunchKernelGGL(naive_apply_kernel, dim3((unsigned)((nnz + kAP - 1) / kAP)), dim3(kAL * kAP),
-                     sizeof(double) * kRec * h * slots, s, (int)nnz, h, slots,
-                     ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
+  const ApplyPlan P = apply_plan(h);
+  hipLaunchKernelGGL(P.lanes == 4 ? naive_apply_kernel<4> : naive_apply_kernel<8>,
+                     dim3((unsigned)((nnz + P.pairs - 1) / P.pairs)), dim3(kAT), sizeof(double) * kRec * h * P.slots, s,
+                     (int)nnz, h, P.slots, ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
 }
 
 void launch_naive_apply_list(int64_t nnz, const int* lpairs, const int* ltot, int first, int last, int h, const int* tidx,
                              const int* ppanel, const double* tx, const double* sx, const double* snx, const double* sw,
                              const double* ub, const double* ubn, const double* wout, double* val, hipStream_t s) {
-  const int slots = apply_slots(h);
-  hipLaunchKernelGGL(naive_apply_list_kernel, dim3((unsigned)((nnz + kAP - 1) / kAP)), dim3(kAL * kAP),
-                     sizeof(double) * kRec * h * slots, s, lpairs, ltot, first, last, h, slots,
+  const ApplyPlan P = apply_plan(h);
+  hipLaunchKernelGGL(P.lanes == 4 ? naive_apply_list_kernel<4> : naive_apply_list_kernel<8>,
+                     dim3((unsigned)((nnz + P.pairs - 1) / P.pairs)), dim3(kAT), sizeof(double) * kRec * h * P.slots, s,
+                     lpairs, ltot, first, last, h, P.slots,
                      ApplyArgs{tidx, ppanel, tx, sx, snx, sw, ub, ubn, wout, val});
 }
 
