@@ -1901,17 +1901,29 @@ __global__ void __launch_bounds__(256) rrq_root_kernel(RRQTables T, RRQPanels P,
 // per (pair, edge): the edge's Dirac-string line integral of the solid angle -> oe[r][3].
 // One thread an item when the items fill the chip (their march is up to 50 intervals,
 // and the sort makes a wave's lengths alike); below that 8 or 16 lanes an item, one
-// per node, since then one march's latency is all that counts.  The line: 98,000
-// and 291,000 items at order 6 take 141 and 194 us with one thread and 50 and 147
-// with 8 lanes; 145,000 at order 12 take 146 and 148 with 16 lanes (of which 14
-// work), 240,000 at order 8 (10 work) 152 and 296.  With the parameter test in
-// solid_angle_edge and one thread an item these took 239, 319, 189 and 229 us, the
-// 60 items of one panel 148 (now 31), the 960,000 of the 48 x 120 order-8 workload
-// 480 (now 325, bound by the vector rate).
+// per node, since then one march's latency is all that counts.  The line lies where the
+// two meet, which the lanes that have no node move: one thread and lanes take (us, on a
+// stream of its own)
+//   order 2   132,000 items 527, 394   195,000 549, 560
+//   order 3   132,000       315, 227   195,000 317, 324
+//   order 4   195,000       239, 206   291,000 272, 297
+//   order 5   195,000       197, 182   291,000 225, 254
+//   order 6   393,000       209, 191   480,000 239, 232   720,000 278, 333
+//   order 7    72,000       143, 100   108,000 143, 140   132,000 145, 166
+//   order 8    72,000       138, 101   108,000 142, 142   132,000 147, 166
+//   order 9   132,000       164, 157   195,000 165, 223
+//   order 10  108,000       131, 120   132,000 131, 141
+//   order 11  132,000       155, 144   195,000 161, 201
+//   order 12  132,000       156, 141   195,000 169, 198
+// With the parameter test in solid_angle_edge and one thread an item 98,000 and 291,000
+// items of order 6 took 239 and 319, the 60 items of one panel 148 (now 31), the 960,000
+// of the 48 x 120 order-8 workload 480 (now 325, bound by the vector rate).
 template <int NQ>
 constexpr int solid_lanes() { return NQ <= 8 ? 8 : 16; }
 template <int NQ>
-constexpr int solid_wide() { return NQ <= 8 ? 393216 : 131072; }
+constexpr int solid_wide() {
+  return NQ <= 5 ? 180224 : (NQ <= 7 ? 229376 : (NQ == 8 ? 393216 : (NQ <= 10 ? 106496 : 131072)));
+}
 
 template <int NQ>
 __global__ void __launch_bounds__(256) rrq_solid_kernel(RRQTables T, RRQPanels P, const int* __restrict__ lpairs,
