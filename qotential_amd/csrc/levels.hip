@@ -634,20 +634,17 @@ __global__ void __launch_bounds__(64 * KS) direct_mfma_kernel(LevelArgs A, const
 }
 
 // the template of h columns: whole tiles of 16, then the rest in units of 4, or as
-// one more tile when it takes four units (the same matrix-core time, one load)
+// one more tile when it takes four units (the same matrix-core time, one load): the
+// column counts of orders 2 to 16
 #define QOL_DIRECT_COLUMNS(H, CALL)                                                         \
   switch (((H) % 16 > 12 || (H) % 16 == 0) ? 4 * (((H) + 15) / 16) : 4 * ((H) / 16) + ((H) % 16 + 3) / 4) { \
     case 1: CALL(0, 1); break;                                                              \
     case 2: CALL(0, 2); break;                                                              \
     case 3: CALL(0, 3); break;                                                              \
     case 4: CALL(1, 0); break;                                                              \
-    case 5: CALL(1, 1); break;                                                              \
     case 6: CALL(1, 2); break;                                                              \
     case 7: CALL(1, 3); break;                                                              \
-    case 8: CALL(2, 0); break;                                                              \
     case 9: CALL(2, 1); break;                                                              \
-    case 10: CALL(2, 2); break;                                                             \
-    case 11: CALL(2, 3); break;                                                             \
     case 12: CALL(3, 0); break;                                                             \
     case 14: CALL(3, 2); break;                                                             \
     case 17: CALL(4, 1); break;                                                             \

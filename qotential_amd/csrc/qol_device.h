@@ -184,12 +184,4 @@ __device__ __forceinline__ double rcp_nr(double x) {
 // ---- solid harmonics H'_n^m (m = 0..n), polar axis = frame x, W = y + i z ----
 __device__ __forceinline__ int hidx(int n, int m) { return n * (n + 1) / 2 + m; }
 
-template <class Arr>
-__device__ __forceinline__ cd hget(const Arr& H, int n, int m) {
-  if (n < 0 || m > n || m < -n) return cmk(0.0, 0.0);
-  if (m >= 0) return H[hidx(n, m)];
-  cd v = cconj(H[hidx(n, -m)]);
-  return ((-m) & 1) ? cmk(-v.re, -v.im) : v;
-}
-
 }  // namespace qol

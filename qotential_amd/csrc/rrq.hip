@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256) rrq_panel_frame_kernel(RRQTables T, RRQPa
   const int k = blockIdx.x;
   if (nrrq && nrrq[k] == 0) return;  // null: every panel
   extern __shared__ double sm[];
-  const int h = T.h, nq = T.nq, p = T.p, nb = 3 * nq, ncoef = T.ncoef, H4 = 4 * h;
+  const int h = T.h, nq = T.nq, p = T.p, nb = 3 * nq;
   double* ssx = sm;             // [3][h]
   double* ssn = ssx + 3 * h;    // [3][h]
   double* ssw = ssn + 3 * h;    // [h]
@@ -156,7 +156,6 @@ __global__ void __launch_bounds__(256) rrq_panel_frame_kernel(RRQTables T, RRQPa
   double* ecf = fr + 16;        // [3 edges][3][nq]
   double* bx = ecf + 9 * nq;    // [nb][6]
   double* sg = bx + 6 * nb;     // [h] sigma contributions
-  cd* Hs = (cd*)(sg + h);       // [nb or 64][ncoef]
   const size_t gk = (size_t)k * h;
   for (int i = threadIdx.x; i < h; i += blockDim.x) {
     for (int c = 0; c < 3; ++c) {
@@ -371,7 +370,7 @@ __global__ void __launch_bounds__(SystemPlan<P>::N) rrq_panel_system_kernel(RRQP
         const cd b = cadd(cmul(W, lo), cmul(cconj(W), hi));
         E[m] = cadd(cscale(mid, X[0]), cscale(cmuli(b), 0.5));
         if (node && m > 0) {
-          // the gradient from degree n - 1 (harm_grad)
+          // the gradient, from degree n - 1
           const double F1 = imrot(m, cscale(mid, dn)), F2 = imrot(m, cscale(cmuli(cadd(lo, hi)), 0.5 * dn)),
                        F3 = imrot(m, cscale(csub(hi, lo), 0.5 * dn));
           FN[(size_t)H * kk] = imrot(m, E[m]);
@@ -1360,35 +1359,9 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
 // per-target pieces
 
 // Edge helpers, specialised on the number of edge nodes NQ so that every
-// nq-sized array is a register array and the Legendre recurrence constants
-// (2k+1)/(k+1), k/(k+1) fold at compile time.  cf = 3 x NQ Legendre
-// coefficients of one edge, cf[c*NQ + k].
-
-// X(s), X'(s) of all three coordinates at real s
-template <int NQ>
-__device__ __forceinline__ void leg3_r(const double* cf, double s, double* val, double* der) {
-  double p0 = 1.0, p1 = s, d0 = 0.0, d1 = 1.0;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    val[c] = cf[c * NQ] + cf[c * NQ + 1] * s;
-    der[c] = cf[c * NQ + 1];
-  }
-#pragma unroll
-  for (int k = 1; k + 1 < NQ; ++k) {
-    const double c1 = (2.0 * k + 1.0) / (k + 1.0), c2 = (double)k / (k + 1.0);
-    const double p2 = c1 * s * p1 - c2 * p0;
-    const double d2 = c1 * (p1 + s * d1) - c2 * d0;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      val[c] += cf[c * NQ + k + 1] * p2;
-      der[c] += cf[c * NQ + k + 1] * d2;
-    }
-    p0 = p1; p1 = p2; d0 = d1; d1 = d2;
-  }
-}
-
-// The edges' power-basis coefficients (cf[c * NQ + j] multiplies s^j): value and
-// derivative of the three components by Horner's rule with fused multiply-adds
+// nq-sized array is a register array.  cf = 3 x NQ power-basis coefficients of
+// one edge (cf[c * NQ + j] multiplies s^j): value and derivative of the three
+// components by Horner's rule with fused multiply-adds
 template <int NQ>
 __device__ __forceinline__ void pow3_r(const double* cf, double s, double* val, double* der) {
 #pragma unroll
@@ -1418,29 +1391,6 @@ __device__ __forceinline__ void pow3_c(const double* cf, cd s, cd* val, cd* der)
     }
     val[c] = v;
     der[c] = d;
-  }
-}
-
-// the Legendre series at complex s
-template <int NQ>
-__device__ __forceinline__ void leg3_c(const double* cf, cd s, cd* val, cd* der) {
-  cd p0 = cmk(1.0, 0.0), p1 = s, d0 = cmk(0.0, 0.0), d1 = cmk(1.0, 0.0);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    val[c] = cadd(cmk(cf[c * NQ], 0.0), cscale(s, cf[c * NQ + 1]));
-    der[c] = cmk(cf[c * NQ + 1], 0.0);
-  }
-#pragma unroll
-  for (int k = 1; k + 1 < NQ; ++k) {
-    const double c1 = (2.0 * k + 1.0) / (k + 1.0), c2 = (double)k / (k + 1.0);
-    const cd p2 = csub(cscale(cmul(s, p1), c1), cscale(p0, c2));
-    const cd d2 = csub(cscale(cadd(p1, cmul(s, d1)), c1), cscale(d0, c2));
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      val[c] = cadd(val[c], cscale(p2, cf[c * NQ + k + 1]));
-      der[c] = cadd(der[c], cscale(d2, cf[c * NQ + k + 1]));
-    }
-    p0 = p1; p1 = p2; d0 = d1; d1 = d2;
   }
 }
 
