@@ -364,9 +364,9 @@ __global__ void __launch_bounds__(256) closepanel_sum_kernel(size_t n, int npart
 
 // Parts per target: about 2,048 workgroups, two rounds of what the chip holds, so
 // that uneven targets even out; more parts only repeat the tree.  Measured at order
-// 8 (20, 100, 300, 777, 2,000 targets) with one part 3.50, 3.84, 4.80, 7.00 and
-// 13.7 ms a call, with 12, 8, 6, 3, 2 parts 0.79, 1.60, 3.11, 6.57 and 13.4, with
-// 32, 32, 16, 8, 4 parts 0.92, 2.47, 4.19, 7.66 and 14.7.
+// 8 (20, 100, 300, 777, 2,000 targets) with one part 4.9, 5.0, 5.9, 8.2 and 15.8 ms a
+// call, with the 10, 10, 7, 3 and 2 parts chosen here 1.04, 1.80, 3.4, 6.8 and 13.8, with
+// 16 parts 0.99, 1.83, 4.1, 9.6 and 23.9.
 int cp_parts(int64_t m) { return (int)std::min<int64_t>(10, (2048 + m - 1) / m); }
 
 template <int P>

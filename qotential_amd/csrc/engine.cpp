@@ -315,7 +315,7 @@ Engine::~Engine() {
 }
 
 // The count sets the largest call qol_rrq_noalloc_ accepts, and stays what callers
-// know: the boundary tangents' part of d_basis (at most 104 KB) is not in it, and the
+// know: the boundary tangents' part of d_basis (at most 52 KB) is not in it, and the
 // 10 h^2 (and above 120 KB another 4 h^2) doubles of a former weights operator are,
 // where d_X (and d_G) take 4 h^2.
 size_t Engine::one_panel_bytes(i64 p, i64 m, i64 ichart, bool square) {
@@ -728,7 +728,11 @@ void Engine::eval(int exterior, double side_tol, bool want_omega) {
   // s1: direct levels, after the edge chain (projection, roots, solid angle): that
   // chain heads the path the moments wait for, the direct kernel's 121k waves
   // would crowd it out, and the direct kernel then runs beside the moments.  A list
-  // too short to fill the GPU crowds nothing out: its direct levels start at once
+  // too short to fill the GPU crowds nothing out: its direct levels start at once, which
+  // takes (us an eval, after the chain and at once) 8,700 pairs of order 4 from 358 to
+  // 338, of 6 from 424 to 396, of 8 from 548 to 518, of 12 from 1,350 to 1,292, and is
+  // still ahead at 88,000 (404 and 393, 462 and 443, 661 and 610, 1,727 and 1,672); the
+  // line stays below what was measured, since 1.9M pairs lose by it
   HIPCHK(hipStreamWaitEvent(s1, nnz <= 16384 ? ev_lists : ev_edge, 0));
   rec(2, 0, s1);
   direct(s1);

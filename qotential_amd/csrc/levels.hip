@@ -663,7 +663,10 @@ void launch_direct_mfma(LevelArgs A, const int* lpairs, const int* ltot, const i
   // few tiles: four waves share one, each a quarter of the nodes, since a level-4
   // tile's steps follow one another and its last tiles leave the chip idle: one
   // panel's 124 targets 33 -> 13 us, 2,500 tiles at order 4 88 -> 31, 12,500 at order
-  // 6 305 -> 196, 7,400 at order 12 620 -> 390; 18,400 at order 12 932 -> 986
+  // 6 305 -> 196, 7,400 at order 12 620 -> 390; 18,400 at order 12 932 -> 986.  The
+  // host knows only the number of all the engine's pairs (the lists are the device's), of
+  // which the RRQ pairs and those of other levels are not in this launch: a launch whose own
+  // tiles are few keeps one wave a tile if those others are many
   const int grid = (int)((nnz + 15) / 16) + 4;
   const bool split = grid <= 16384;
 #define QOL_DIRECT(NT_, NU_)                                                                                    \

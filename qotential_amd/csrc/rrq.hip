@@ -1286,8 +1286,10 @@ __global__ void __launch_bounds__(64 * kOpW) rrq_operator_kernel(RRQPanels P, co
 // two differ by how v's rounding passes through B Fn^T, which grows with the condition
 // of X: against the weights by G the potentials of a 12 x 36 surface move by 1e-10
 // (relative 2-norm, largest 7e-9) at order 10, 4e-10 (2e-8) at 11 and 2e-8 (1e-6) at
-// 12, so that the two highest orders keep G.  Up to order 10 the shorter product is the
-// faster one.
+// 12, so that the two highest orders keep G, and with it the weights callers have had.
+// Neither is the nearer one: by Green's identity the potentials at 6,000 targets of a 24 x
+// 60 surface are off by 2.40e-10 (2-norm) with G and 2.42e-10 without at order 12, by
+// 4.44e-10 with either at 11.  Up to order 10 the shorter product is the faster one.
 bool rrq_forms_operator(int p) { return p >= 11; }
 
 void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq, hipStream_t s, int variant) {
@@ -1295,8 +1297,8 @@ void launch_rrq_panel_solve(RRQTables T, RRQPanels P, int npan, const int* nrrq,
   const int rpt = (h + 15) / 16, cpt = (2 * h + 15) / 16;
   // variant 2 (or QOL_SOLVE_MFMA=1) selects, for patch orders up to 8, the
   // matrix-core quaternion elimination (A as 4-wave accumulator tiles, B from a
-  // separate real inverse), which is slower on the order-8 workload (5.3 vs 4.9
-  // ms for 14,250 panels, against 1.1 ms for the register-resident inverses)
+  // separate real inverse), which is slower on the order-8 workload (4.2 ms for 14,250
+  // panels, the fused kernel below 3.8, the register-resident inverses 1.1)
   const char* mf = std::getenv("QOL_SOLVE_MFMA");
   if (variant == 2 || (variant == 0 && mf && mf[0] == '1')) switch (T.p) {
 #define QOL_SOLVE_MFMA(P_, RT_, CT_, RPT_)                                                                  \
