@@ -2110,8 +2110,8 @@ __global__ void __launch_bounds__(64 * kRW, P <= 8 ? 3 : 2)
         to_frame(fr, x, X);
         const double* Y = bx + 6 * ib;
         const double z[3] = {Y[0] - X[0], Y[1] - X[1], Y[2] - X[2]};
-        const double wr =
-            w1g[(size_t)(r0 + tile0 + t) * NB + ib] * rsqrt_h3(z[0] * z[0] + z[1] * z[1] + z[2] * z[2]);
+        const double zz = z[0] * z[0] + z[1] * z[1] + z[2] * z[2];
+        const double wr = w1g[(size_t)(r0 + tile0 + t) * NB + ib] * (zz == HUGE_VAL ? 0.0 : rsqrt_h3(zz));
         wl[t * NB + ib] = wr;
         cross3(z, Y + 3, zx);
         for (int c = 0; c < 3; ++c) {
